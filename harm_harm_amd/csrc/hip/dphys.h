@@ -67,6 +67,45 @@ __device__ __forceinline__ double recip_nr(double x)
   return r;
 }
 
+// IEEE quotients without the scaling steps.  The compiler's n / d scales both
+// operands (div_scale), refines a reciprocal estimate by two Newton steps,
+// forms the quotient with one residual correction and scales back: 11
+// instructions a quotient.  With d and n/d well inside the normal range every
+// scale is 1, and the same refinement and residual correction without them
+// give the same correctly rounded quotient; quotients by one d share its
+// reciprocal (7 instructions for the first quotient, 3 for each further one).
+// Ranges: 2^-1000 < |d| < 2^1000, n zero or 2^-900 < |n| < 2^1000, n/d in the
+// same range as n; callers say why theirs hold or test them.
+struct Recip {
+  double d, r;
+};
+__device__ __forceinline__ Recip recip(double d)
+{
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(fma(-d, r, 1.0), r, r);
+  r = fma(fma(-d, r, 1.0), r, r);
+  return Recip{d, r};
+}
+// n / d; a zero n gives +0 whatever its sign
+__device__ __forceinline__ double quot(double n, const Recip& R)
+{
+  const double q = n * R.r;
+  return fma(fma(-R.d, q, n), R.r, q);
+}
+// 1 / d
+__device__ __forceinline__ double inv1(double d)
+{
+  const Recip R = recip(d);
+  return fma(fma(-R.d, R.r, 1.0), R.r, R.r);
+}
+// n / d for a compile-time d: with the correctly rounded 1/d the one residual
+// correction rounds the quotient correctly (Markstein 1990)
+__device__ __forceinline__ double quot_const(double n, double d, double rd)
+{
+  const double q = n * rd;
+  return fma(fma(-d, q, n), rd, q);
+}
+
 // Load a record stored SoA with field stride `fs` starting at `base`.
 __device__ __forceinline__ void load_geom(const double* __restrict__ tab, long base, long fs, Geom& g)
 {

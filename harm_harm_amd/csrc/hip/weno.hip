@@ -32,8 +32,16 @@
 // last eight values and a four-zone pipeline of weights in registers.  The
 // face-flux kernels read the left and right face values of zones -1 .. N
 // back.  The arithmetic repeats the oracle's operation order (no contraction
-// in this translation unit, IEEE divisions), so the face values agree bit for
-// bit.
+// in this translation unit, correctly rounded quotients), so the face values
+// agree bit for bit.
+//
+// The passes are bound by instruction issue (0.56-0.72 of the vector issue
+// slots, 360 instructions a wave of 52 faces along x1).  Quotients are the
+// largest part of it, so the weights of a zone share one reciprocal per
+// normalisation (hd::recip, hd::quot), 7 + 3 + 3 instructions for three
+// quotients instead of 33, and the SMONO and ratio tests settle clear cases
+// without a quotient.  At 256x128x64 the x1, x2 and x3 passes take 265, 301
+// and 337 us (311, 405 and 450 with the compiler's divisions, same steps).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <float.h>
@@ -74,6 +82,9 @@ constexpr double sym2(double a0, double a1)
   s += a1 * 0;
   return s;
 }
+// the same sum of terms of which one at least is positive and none negative
+// (the additions of 0 only matter for zeros' signs)
+constexpr double sym3p(double a0, double a1, double a2) { return (a0 + a2) + a1; }
 __device__ __forceinline__ double sym5(const double* a)
 {
   double s = 0.0;
@@ -92,6 +103,28 @@ __device__ __forceinline__ double limit_weight(double w)
   if (w < w3) return avg;
   return (w - w3) * (w4 - avg) / (w4 - w3) + avg;
 }
+
+// The same with one quotient by a constant: its numerator and denominator are
+// picked by the branch w falls in (numerators are 0 or at least an ulp of w1,
+// about 1e-17).
+template <int ORDER>
+__device__ __forceinline__ double limit_weight_q(double w)
+{
+  constexpr double avg = 1. / ORDER, w1 = 0.2 * avg, w2 = (1.0 - 0.2) * avg, w3 = (1.0 + 0.2) * avg, w4 = 1.0;
+  constexpr double dlo = w2 - w1, dhi = w4 - w3, rlo = 1.0 / dlo, rhi = 1.0 / dhi;
+  const bool hi = w >= w3;
+  const double num = hi ? (w - w3) * (w4 - avg) : avg * (w - w1);
+  const double q = hd::quot_const(num, hi ? dhi : dlo, hi ? rhi : rlo);
+  double r = hi ? q + avg : w < w2 ? q : avg;
+  return w < w1 ? 0.0 : r;
+}
+
+// Whether the indicator sum n of a zone lies in the range of the unscaled
+// quotients (dphys.h).  Its terms are then at least 1e-28 of it: each holds
+// WENO_EPSILON (1.2e-26) times the window's sum of squares, and n is at most
+// 60 times that sum.  Outside (fields that have decayed to 1e-100, infinities
+// and NaN) the plain divisions are used.
+__device__ __forceinline__ bool plain_range(double n) { return n > 1e-200 && n < 1e200; }
 
 // The weights of the two uniform cases, formed by the same operations as the
 // general code below (constant-folded, round to nearest):
@@ -130,6 +163,24 @@ __device__ __forceinline__ void weights3(const double* u, double* w)
   s1 += err;
   s2 += err;
   double n = sym3(s0, s1, s2) + kMinNum;
+  if (plain_range(n)) {
+    // the quotients below stay between 1e-53 and 1e52 (s/n >= 1e-28, t between
+    // WENO_EPSILON^2 = 1.5e-52 and about 1)
+    const hd::Recip rn = hd::recip(n);
+    double t0 = hd::quot(s0, rn) + kWeps, t1 = hd::quot(s1, rn) + kWeps, t2 = hd::quot(s2, rn) + kWeps;
+    t0 *= t0;
+    t1 *= t1;
+    t2 *= t2;
+    const double w0 = hd::inv1(t0), w1 = hd::inv1(t1), w2 = hd::inv1(t2);
+    const hd::Recip rw = hd::recip(sym3p(w0, w1, w2));
+    const double l0 = limit_weight_q<3>(hd::quot(w0, rw)), l1 = limit_weight_q<3>(hd::quot(w1, rw)),
+                 l2 = limit_weight_q<3>(hd::quot(w2, rw));
+    const hd::Recip rl = hd::recip(sym3p(l0, l1, l2));  // the largest weight is at least 1/3, limited too
+    w[0] = hd::quot(l0, rl);
+    w[1] = hd::quot(l1, rl);
+    w[2] = hd::quot(l2, rl);
+    return;
+  }
   s0 /= n;
   s1 /= n;
   s2 /= n;
@@ -160,6 +211,24 @@ __device__ __forceinline__ void weights2(const double* u, double* L2, double* R2
   s0 += err;
   s1 += err;
   double n = sym2(s0, s1) + kMinNum;
+  if (plain_range(n)) {  // as in weights3
+    const hd::Recip rn = hd::recip(n);
+    double t0 = hd::quot(s0, rn) + kWeps, t1 = hd::quot(s1, rn) + kWeps;
+    t0 *= t0;
+    t1 *= t1;
+    const double w0 = hd::inv1(t0), w1 = hd::inv1(t1);
+    const hd::Recip rw = hd::recip(w0 + w1);
+    const double m0 = limit_weight_q<2>(hd::quot(w0, rw)), m1 = limit_weight_q<2>(hd::quot(w1, rw));
+    const hd::Recip rm = hd::recip(m0 + m1);
+    const double v0 = hd::quot(m0, rm), v1 = hd::quot(m1, rm);
+    const double l0 = v0 * (1. / 4.), l1 = v1 * (3. / 4.), r0 = v0 * (3. / 4.), r1 = v1 * (1. / 4.);
+    const hd::Recip rl = hd::recip((l0 + l1) + kMinNum), rr = hd::recip((r0 + r1) + kMinNum);
+    L2[0] = hd::quot(l0, rl);
+    L2[1] = hd::quot(l1, rl);
+    R2[0] = hd::quot(r0, rr);
+    R2[1] = hd::quot(r1, rr);
+    return;
+  }
   s0 /= n;
   s1 /= n;
   double t0 = s0 + kWeps, t1 = s1 + kWeps;
@@ -191,12 +260,23 @@ __device__ __forceinline__ void weights2(const double* u, double* L2, double* R2
 // numerators already disagree in sign gives 0 without its divisions; m = 0
 // gives the indicator 0 and m >= cut gives 1 (m / cut >= 1 exactly).
 __device__ __forceinline__ bool same_sign(double a, double b) { return (a > 0 && b > 0) || (a < 0 && b < 0); }
+//
+// Rounding is monotone, so the smallest of the quotients by 12 is the quotient
+// of the smallest numerator: one division by 12 decides the indicator.  The
+// minmods' sign products cannot underflow when the smallest estimate is above
+// 1e-150; below that the estimates go through the minmods one by one.
+__device__ __forceinline__ double smono_cut(const double* y, double m)
+{
+  const double norm = fabs(y[0]) + ((fabs(y[-1]) + fabs(y[1])) + (fabs(y[-2]) + fabs(y[2])));
+  const double cut = norm * kSqrtWeps + kMinNum;
+  if (m >= cut) return 1.0;
+  return (m - 0.0) / (cut - 0.0);
+}
 __device__ __forceinline__ double smono(const double* y)
 {
   const double L3 = (((-3 * y[-2] - y[2]) + (10 * y[-1] + 6 * y[1])) - 12 * y[0]) / 2.;
   const double R3 = (((y[-2] + 3 * y[2]) - (6 * y[-1] + 10 * y[1])) + 12 * y[0]) / 2.;
-  const double m3 = fabs(wminmod(L3, R3));
-  if (m3 == 0.0) return 0.0;
+  if (!same_sign(L3, R3)) return 0.0;
   const double L2n = (((11 * y[-2] - y[2]) + (-20 * y[-1] + 4 * y[1])) + 6 * y[0]);
   const double R2n = (((-y[-2] + 11 * y[2]) + (4 * y[-1] - 20 * y[1])) + 6 * y[0]);
   if (!same_sign(L2n, R2n)) return 0.0;
@@ -204,18 +284,24 @@ __device__ __forceinline__ double smono(const double* y)
   const double R1n = (((-y[-2] + 3 * y[2]) + (6 * y[-1] + 10 * y[1])) - 18 * y[0]);
   const double dl = y[-1] - y[-2], dr = y[2] - y[1];
   if (!same_sign(L1n, dl) || !same_sign(R1n, dr)) return 0.0;
+  const double d3 = fmin(fabs(L3), fabs(R3)), d1 = fmin(fabs(dl), fabs(dr));
+  const double n12 = fmin(fmin(fabs(L2n), fabs(R2n)), fmin(fabs(L1n), fabs(R1n)));
+  const double m = fmin(fmin(hd::quot_const(n12, 12., 1. / 12.), d1), d3);
+  if (m > 1e-150 && m < kBIG) {
+    if (!same_sign(dl, dr)) return 0.0;
+    return smono_cut(y, m);
+  }
+  const double m3 = fabs(wminmod(L3, R3));
+  if (m3 == 0.0) return 0.0;
   const double L1 = wminmod(L1n / 12., dl);
   const double R1 = wminmod(R1n / 12., dr);
   const double m2 = fabs(wminmod(L2n / 12., R2n / 12.));
-  double m = kBIG;
-  m = wmin(m, fabs(wminmod(L1, R1)));
-  m = wmin(m, m2);
-  m = wmin(m, m3);
-  if (m == 0.0) return 0.0;
-  const double norm = fabs(y[0]) + ((fabs(y[-1]) + fabs(y[1])) + (fabs(y[-2]) + fabs(y[2])));
-  const double cut = norm * kSqrtWeps + kMinNum;
-  if (m >= cut) return 1.0;
-  return (m - 0.0) / (cut - 0.0);
+  double mm = kBIG;
+  mm = wmin(mm, fabs(wminmod(L1, R1)));
+  mm = wmin(mm, m2);
+  mm = wmin(mm, m3);
+  if (mm == 0.0) return 0.0;
+  return smono_cut(y, mm);
 }
 
 // five-point interpolant at the left (RIGHT = false) or right face
@@ -298,18 +384,29 @@ __device__ __forceinline__ void zone_weights(const double* y, ZoneW& z)
 }
 
 // one side of the AND ratio test: the zone's outer sub-stencil weight against
-// the neighbour's weight of the same three zones (equal weights: exactly 1)
+// the neighbour's weight of the same three zones (equal weights: exactly 1).
+// Both lie in [WENO_EPSILON, 1 + WENO_EPSILON].
 __device__ __forceinline__ double side_ratio(double uc, double un)
 {
   if (uc == un) return 1.0;
-  return (uc + kWeps) / (un + kWeps);
+  return hd::quot(uc + kWeps, hd::recip(un + kWeps));
 }
 
-// lower-order fraction from the ratio test (BIG for a side that does not exist)
-__device__ __forceinline__ double ratio_lof(double wl, double wr)
+// Lower-order fraction of a zone from its outer sub-stencil weights uc against
+// the neighbours' un (a side that does not exist counts as BIG): the smaller
+// ratio's place in the band 1.3 .. 1.6, clamped.  A ratio that is clearly at
+// or below 1.3 on one side gives 0 without its quotient, two that are clearly
+// at or above 1.6 give 1.
+__device__ __forceinline__ double ratio_lof(double ucl, double unl, bool hasl, double ucr, double unr, bool hasr)
 {
-  const double wrat = wmin(wl, wr);
   const double min_rat = 1.3, max_rat = 1.6;
+  if (!hasl && !hasr) return 1.0;
+  const double al = ucl + kWeps, bl = unl + kWeps, ar = ucr + kWeps, br = unr + kWeps;
+  if (hasr && ar <= 1.2999 * br) return 0.0;
+  if (hasl && al <= 1.2999 * bl && !__builtin_isunordered(ar, br)) return 0.0;  // (a NaN on the right wins below)
+  if ((!hasl || al >= 1.6001 * bl) && (!hasr || ar >= 1.6001 * br)) return 1.0;
+  const double wl = hasl ? side_ratio(ucl, unl) : kBIG, wr = hasr ? side_ratio(ucr, unr) : kBIG;
+  const double wrat = wmin(wl, wr);
   // the clamps below give exactly these at and beyond the band's ends
   if (wrat <= min_rat) return 0.0;
   if (wrat >= max_rat) return 1.0;
@@ -344,14 +441,14 @@ __device__ __forceinline__ void zone_faces(const double* y, const ZoneW& z, doub
       R[0] = z.u[0] * (5. / 16.);
       R[1] = z.u[1] * (5. / 8.);
       R[2] = z.u[2] * (1. / 16.);
-      double n = sym3(L[0], L[1], L[2]) + kMinNum;
-      L[0] /= n;
-      L[1] /= n;
-      L[2] /= n;
-      n = sym3(R[0], R[1], R[2]) + kMinNum;
-      R[0] /= n;
-      R[1] /= n;
-      R[2] /= n;
+      // the unoptimized weights are 0 or at least 1e-17 and sum to 1
+      const hd::Recip rl = hd::recip(sym3p(L[0], L[1], L[2]) + kMinNum);
+      const hd::Recip rr = hd::recip(sym3p(R[0], R[1], R[2]) + kMinNum);
+#pragma unroll
+      for (int s = 0; s < 3; s++) {
+        L[s] = hd::quot(L[s], rl);
+        R[s] = hd::quot(R[s], rr);
+      }
     }
     double vl = 0.0, vr = 0.0;
     if (0.0 < lof) {
@@ -474,7 +571,7 @@ __global__ __launch_bounds__(kBlock) void k_weno_dp(Dims d, Box z, const double*
 // transverse plane with i fastest (no lanes padded per row); blockIdx.y is
 // (primitive, segment).
 template <int DIR>
-__global__ __launch_bounds__(kBlock) void k_weno_recon(Dims d, Box b, int seg, const double* __restrict__ pb,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_weno_recon(Dims d, Box b, int seg, const double* __restrict__ pb,
                                                          const double* __restrict__ dpd, double* __restrict__ L,
                                                          double* __restrict__ R)
 {
@@ -529,9 +626,7 @@ __global__ __launch_bounds__(kBlock) void k_weno_recon(Dims d, Box b, int seg, c
     fd[1] = fd[2];
     fd[2] = 0.0;
     if (r >= 2 && r >= f0 - 1) {
-      const double wl = r >= 4 ? side_ratio(zw[2].u[2], z6u0) : kBIG;
-      const double wr = r <= n - 5 ? side_ratio(zw[2].u[0], zw[0].u[2]) : kBIG;
-      fd[2] = ratio_lof(wl, wr);
+      fd[2] = ratio_lof(zw[2].u[2], z6u0, r >= 4, zw[2].u[0], zw[0].u[2], r <= n - 5);
     }
     // faces of zone f = s-5 (zw[3], values y[0..4] centred on y[2])
     const int f = s - 5;
@@ -565,9 +660,7 @@ __device__ __forceinline__ bool lane_faces(const double* y, int c, int n, int g,
   const double ul = __shfl_up(z.u[0], 2, GL), ur = __shfl_down(z.u[2], 2, GL);
   double fd = 0.0;
   if (act && c >= 2 && c <= n - 3 && g >= 2 && g <= GL - 3) {
-    const double wl = c >= 4 ? side_ratio(z.u[2], ul) : kBIG;
-    const double wr = c <= n - 5 ? side_ratio(z.u[0], ur) : kBIG;
-    fd = ratio_lof(wl, wr);
+    fd = ratio_lof(z.u[2], ul, c >= 4, z.u[0], ur, c <= n - 5);
   }
   const double fdm = __shfl_up(fd, 1, GL), fdp = __shfl_down(fd, 1, GL);
   if (act && c >= 3 && c <= n - 4 && g >= 3 && g <= GL - 4) {
@@ -590,7 +683,7 @@ __device__ __forceinline__ bool lane_faces(const double* y, int c, int n, int g,
 // scalar registers.  (Along x2 and x3 the same scheme, with strided loads or
 // staged through LDS, measured slower than the sweep.)
 constexpr int kX1Lanes = 32;
-__global__ __launch_bounds__(kBlock) void k_weno_recon_x1(Dims d, Box b, int nw, const double* __restrict__ pb,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_weno_recon_x1(Dims d, Box b, int nw, const double* __restrict__ pb,
                                                             const double* __restrict__ dpd, double* __restrict__ L,
                                                             double* __restrict__ R)
 {
