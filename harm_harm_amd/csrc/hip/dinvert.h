@@ -36,26 +36,36 @@ __device__ __forceinline__ void fix_delta_to(const Params& P, const Geom& G, con
 // fixup1zone on the final substep (fixup.c:561-830): the density and
 // internal-energy floors (mass and energy added in the ZAMO frame, then the
 // floors' own Utoprimgen from the primitives so far) and the Lorentz-factor
-// limit, on pz with flag fl (replaced by the floors' inversion flag when the
-// floors changed the zone).  G: the zone's centre geometry.  Returns the
-// flag; the floors' Newton strokes are added to ns.  *changed reports
-// whether pz changed.  DIAG: as invert_zone.
+// limit, on the zone's primitives pf[pl * ncell + o], left in pz, with flag fl
+// (replaced by the floors' inversion flag when the floors changed the zone).
+// Returns the flag; the floors' Newton strokes are added to ns.  *changed
+// reports whether pz differs from pf, which is not written.  The geometry and
+// the primitives are read again after the solve (an L1/L2 hit) instead of
+// holding 86 registers through the Newton iterations.  DIAG: as invert_zone.
 template <bool DIAG = false>
-__device__ __forceinline__ int floors_zone(const Dims& d, const Params& P, const Geom& G,
-                                           const double* __restrict__ floors, double* pz, int fl, long o, long pp,
-                                           int& ns, bool* changed, double* __restrict__ fx_p0,
-                                           double* __restrict__ fx_pfl, uint8_t* __restrict__ fx_flag)
+__device__ __forceinline__ int floors_zone(const Dims& d, const Params& P, const double* __restrict__ gcent,
+                                           const double* __restrict__ floors, const double* pf,
+                                           double* pz, int fl, long o, long pp, int& ns, bool* changed,
+                                           double* __restrict__ fx_p0, double* __restrict__ fx_pfl,
+                                           uint8_t* __restrict__ fx_flag)
 {
   const long nc = d.ncell;
-  double prfloor[2] = {floors[pp], floors[d.nplane + pp]};
-  for (int pl = 0; pl < 2; pl++)
-    if (prfloor[pl] < D_SMALL) prfloor[pl] = D_SMALL;
-  double prnew[HARM_NPR];
+  Geom G;
+  hd::load_geom(gcent, pp, d.nplane, G);
+#pragma unroll
+  for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = pf[pl * nc + o];
+  auto floor_of = [&](const double* __restrict__ fls, int pl) {
+    const double v = fls[pl * d.nplane + pp];
+    return v < D_SMALL ? D_SMALL : v;
+  };
   bool didchange = false;
+  double dpr[HARM_NPR];
 #pragma unroll
   for (int pl = 0; pl < HARM_NPR; pl++) {
-    if (pl <= HARM_UU && prfloor[pl] > pz[pl]) { didchange = true; prnew[pl] = prfloor[pl]; }
-    else prnew[pl] = pz[pl];
+    const double fv = pl <= HARM_UU ? floor_of(floors, pl) : 0.0;
+    const bool below = pl <= HARM_UU && fv > pz[pl];
+    didchange = didchange || below;
+    dpr[pl] = below ? fv - pz[pl] : 0.0;
   }
   if (didchange) {
     if (DIAG) {
@@ -65,27 +75,39 @@ __device__ __forceinline__ int floors_zone(const Dims& d, const Params& P, const
     Geom G1 = G;
     G1.gdet = 1.0;
     State q, dq;
-    double Ua[HARM_NPR], dpr[HARM_NPR], dUa[HARM_NPR];
+    double Ua[HARM_NPR], dUa[HARM_NPR];
     hd::get_state(pz, G, P.gam, q);
     hd::primtoflux(pz, q, 0, G1, Ua);
-#pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) dpr[pl] = 0.0;
-    for (int pl = HARM_RHO; pl <= HARM_UU; pl++) dpr[pl] = prnew[pl] - pz[pl];
     hd::get_state(dpr, G, P.gam, dq);
     hd::primtoflux(dpr, dq, 0, G1, dUa);
 #pragma unroll
     for (int pl = 0; pl < HARM_NPR; pl++) Ua[pl] += dUa[pl];
     // the floors' own Utoprimgen (UNOTHING), from the primitives so far;
-    // any flag > 0, the cold retry's mark included, restores prnew
-    double p0[HARM_NPR];
+    // any flag > 0, the cold retry's mark included, restores the floored
+    // primitives
+    bool solved;
+    fl = hd::jon(Ua, G, P.gam, P.gammafail, pz, ns, __builtin_nan(""), 200, &solved);
+    const double* pfr = hd::fresh(pf);
+    if (!solved) {
 #pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) p0[pl] = pz[pl];
-    fl = hd::jon(Ua, G, P.gam, P.gammafail, pz, ns, __builtin_nan(""));
-    if (hd::needs_after_hot(fl, P.hot2cold, P.checkinv))
+      for (int pl = 0; pl <= HARM_U3; pl++) pz[pl] = pfr[pl * nc + o];
+    }
+    hd::load_geom(hd::fresh(gcent), pp, d.nplane, G);
+    if (hd::needs_after_hot(fl, P.hot2cold, P.checkinv)) {
+      double p0[HARM_NPR];
+#pragma unroll
+      for (int pl = 0; pl < HARM_NPR; pl++) p0[pl] = pfr[pl * nc + o];
       fl = hd::after_hot(fl, Ua, G, P.gam, P.gammafail, p0, pz, ns, P.hot2cold, P.checkinv);
+    }
     if (fl > 0) {
 #pragma unroll
-      for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = prnew[pl];
+      for (int pl = 0; pl < HARM_NPR; pl++) {
+        pz[pl] = pfr[pl * nc + o];
+        if (pl <= HARM_UU) {
+          const double fv = floor_of(hd::fresh(floors), pl);
+          if (fv > pz[pl]) pz[pl] = fv;
+        }
+      }
     }
   }
   double pb4[HARM_NPR];  // DIAG: the primitives ahead of the gamma limit
@@ -130,7 +152,7 @@ __device__ __forceinline__ int floors_zone(const Dims& d, const Params& P, const
 // Uz in registers through the Newton iterations.
 template <bool SEEDED = false, bool DIAG = false, bool FLOORS = true>
 __device__ __forceinline__ int invert_zone(const Dims& d, const Params& P, double* Uz, const double* __restrict__ Ug,
-                                           const double* __restrict__ pg, double* __restrict__ pf,
+                                           const double* __restrict__ pg, double* pf,
                                            int32_t* __restrict__ pflag, const double* __restrict__ gcent,
                                            const double* __restrict__ floors, int finalstep, long o, long pp, int& ns,
                                            double wp_seed = 0.0, int* fellback = nullptr,
@@ -143,7 +165,13 @@ __device__ __forceinline__ int invert_zone(const Dims& d, const Params& P, doubl
   double pz[HARM_NPR];
 #pragma unroll
   for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = pg[pl * nc + o];  // guess: the substep's starting primitives
-  int fl = hd::utoprimgen(Uz, G, P.gam, P.gammafail, pz, ns, SEEDED ? wp_seed : __builtin_nan(""));
+  bool solved;
+  int fl = hd::utoprimgen(Uz, G, P.gam, P.gammafail, pz, ns, SEEDED ? wp_seed : __builtin_nan(""), 200, &solved);
+  if (!solved) {  // the guess stands (read again rather than kept through the iterations)
+    const double* pgr = hd::fresh(pg);
+#pragma unroll
+    for (int pl = 0; pl <= HARM_U3; pl++) pz[pl] = pgr[pl * nc + o];
+  }
   if (SEEDED && fl != 0) {
     *fellback = 1;
 #pragma unroll
@@ -166,7 +194,9 @@ __device__ __forceinline__ int invert_zone(const Dims& d, const Params& P, doubl
   }
   if (FLOORS && finalstep) {
     bool changed;
-    fl = floors_zone<DIAG>(d, P, G, floors, pz, fl, o, pp, ns, &changed, fx_p0, fx_pfl, fx_flag);
+#pragma unroll
+    for (int pl = 0; pl < HARM_NPR; pl++) pf[pl * nc + o] = pz[pl];
+    fl = floors_zone<DIAG>(d, P, gcent, floors, pf, pz, fl, o, pp, ns, &changed, fx_p0, fx_pfl, fx_flag);
   } else if (FLOORS && DIAG) {
     fx_flag[o] = 0;
   }

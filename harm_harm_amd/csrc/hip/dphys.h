@@ -92,6 +92,11 @@ __device__ __forceinline__ double quot(double n, const Recip& R)
   const double q = n * R.r;
   return fma(fma(-R.d, q, n), R.r, q);
 }
+// n / d with IEEE's zeros, infinities and NaN for either operand
+__device__ __forceinline__ double quot_any(double n, const Recip& R)
+{
+  return __builtin_amdgcn_div_fixup(quot(n, R), R.d, n);
+}
 // 1 / d
 __device__ __forceinline__ double inv1(double d)
 {
@@ -453,6 +458,50 @@ __device__ __forceinline__ void func_eprime(double Wp, const Inv& s, double& dx,
   df = -2. * f;
 }
 
+// Whether a solve's invariants lie where func_eprime_q's unscaled quotients
+// hold (dphys.h's ranges): with these bounds and 1e-40 < W < 1e40 no
+// denominator or quotient below leaves 1e-271 .. 1e271.
+__device__ __forceinline__ bool moderate(const Inv& s)
+{
+  return s.D > 1e-40 && s.D < 1e40 && s.Bsq >= 0.0 && s.Bsq < 1e40 && fabs(s.Qtsq) < 1e40 && s.QdotBsq < 1e40 &&
+         fabs(s.Qdotnp) < 1e40;
+}
+
+// func_eprime with the quotients unscaled (the same bits) and without a
+// branch, for moderate invariants.  Returns false where W or the Lorentz
+// factor leaves the range that holds in or the residual is unusable; the
+// outputs then mean nothing and func_eprime decides.
+__device__ __forceinline__ bool func_eprime_q(double Wp, const Inv& s, double& dx, double& resid)
+{
+  const double D = s.D, Bsq = s.Bsq;
+  const double W = Wp + D;
+  const double SoW = quot(s.QdotB, recip(W));
+  const double top = s.Qtsq + (Bsq + 2.0 * W) * SoW * SoW;
+  const double bot = (Bsq * Bsq - s.Qtsq) + 2.0 * Bsq * W + W * W - SoW * SoW * (Bsq + 2.0 * W);
+  const double utsq = quot(top, recip(bot));
+  const double gammasq = 1.0 + utsq;
+  const double X = Bsq + W + D_SMALL;
+  const double X2 = X * X, X3 = X2 * X;
+  const double gamma = sqrt(gammasq);
+  const Recip rg = recip(gammasq);
+  const double wmrho0 = quot(Wp - quot(D * utsq, recip(1.0 + gamma)), rg);
+  const double igr = (s.gam - 1.0) / s.gam;
+  const double pofchi = igr * wmrho0, dpdchi = igr;
+  const double BQ = Bsq * s.Qtsq - s.QdotBsq;
+  const double Ep = s.Qdotnp + Wp - pofchi + 0.5 * Bsq + quot(0.5 * BQ, recip(X2));
+  const double Xd = Bsq + W, Wsq = W * W, W3 = Wsq * W, Xd3 = Xd * Xd * Xd;
+  const double dvsq = quot(-2.0, recip(Xd3)) * (s.Qtsq + quot(s.QdotBsq * (3.0 * W * Xd + Bsq * Bsq), recip(W3)));
+  const double dpdW = quot(1.0, rg) * dpdchi;
+  const double dpdvsq = (D * (gamma * 0.5 - 1.0) - Wp) * dpdchi;
+  const double dpdWp = dpdW + dpdvsq * dvsq;
+  const double dE = (1.0 - dpdWp) - quot(BQ, recip(X3));
+  resid = Ep;
+  dx = quot(-Ep, recip(dE));
+  // (a NaN anywhere makes Ep or dE one)
+  return (W > 1e-40) & (W < 1e40) & (gammasq > 1e-40) & (gammasq < 1e250) & (utsq >= -0.9 * s.utsq_too_big) &
+         (fabs(Ep) < 1e100) & (fabs(dE) > 1e-40) & (fabs(dE) < 1e250);
+}
+
 // Cold GRMHD residual W^2 P^2 of the momentum equation and its W' derivative
 // (func_Psq, utoprim_jon.c:3103, with Psq_Wp :1923 and dPsqdWp_Wp :1944).
 __device__ __forceinline__ void func_psq(double Wp, const Inv& s, double& dx, double& resid, double& jac, double& f,
@@ -482,10 +531,11 @@ __device__ __forceinline__ void residual(double Wp, const Inv& s, double& dx, do
 }
 
 __device__ __forceinline__ bool ultrarel(double x0, const Inv& s) { return (fabs(s.w1) > s.w2) || (fabs(x0) > s.w2); }
-__device__ __forceinline__ bool errcheck(double errx, double x0, const Inv& s)
+__device__ __forceinline__ double errlimit(double x0, const Inv& s)
 {
-  return ultrarel(x0, s) ? (fabs(errx) <= D_NUMEPSILON) : (fabs(errx) <= 1E3 * D_NUMEPSILON);
+  return ultrarel(x0, s) ? D_NUMEPSILON : 1E3 * D_NUMEPSILON;
 }
+__device__ __forceinline__ bool errcheck(double errx, double x0, const Inv& s) { return fabs(errx) <= errlimit(x0, s); }
 __device__ __forceinline__ int extracheck(double x0, const Inv& s) { return ultrarel(x0, s) ? 4 : 2; }
 
 __device__ __forceinline__ void validate_wp(double Wpold, double& Wpnew, const Inv& s)
@@ -495,54 +545,122 @@ __device__ __forceinline__ void validate_wp(double Wpold, double& Wpnew, const I
     coldgrhd(s.Qtsq, s.D, Wp);
     Wpnew = Wp * 10.0;
   }
-  Wpnew = (fabs(Wpnew / s.w1) > s.gsq_too_big) ? 0.5 * (Wpold + Wpnew) : Wpnew;
+  // the quotient is formed only near the limit (and for NaN)
+  if (!(fabs(Wpnew) < 0.999 * (s.gsq_too_big * s.w1)))
+    Wpnew = (fabs(Wpnew / s.w1) > s.gsq_too_big) ? 0.5 * (Wpold + Wpnew) : Wpnew;
 }
 
 // general_newton_raphson for n=1 without line search (COLD: on the cold
-// residual).  Returns retval.
-template <bool COLD = false>
-__device__ __forceinline__ int newton(int& pflag, double& xio, const Inv& s, int& nstroke)
+// residual).  Returns retval, or kUnfinished after `limit` iterations when
+// limit is below the reference's 200.
+//
+// A wave on its own issues one vector instruction in 8 cycles and loses many
+// times that at a taken branch, so an ordinary iteration (moderate invariants,
+// a usable residual, W' clear of its bounds and the error clear of its limit)
+// runs straight through with its quotients unscaled; any other one leaves the
+// state alone there and goes through the general form below it.  On 4096 zones
+// (one wave a SIMD) an iteration took 1.9 us with the reference's branches and
+// scaled divisions; on 2^24 zones see k_invert_batch.
+//
+// CYCLE: an iteration is a function of (x, x_old, dx_old, damp) once its
+// count is past the damping's tenth, so a state that comes back has entered a
+// cycle that no later iteration leaves: the whole cycles left until the cap
+// are counted without being run (2 % of the zones of a log-uniform sample in
+// Lorentz factor and magnetisation circle between neighbouring W' within 14
+// iterations and would run all 200).  The states compared with are kept at
+// iterations 12, 16, 24, 40, 72 and 136.  (Off in the grid kernels, whose
+// solves take 5 to 7 iterations and whose registers are full.)
+constexpr int kUnfinished = -1, kUnfinishedFlag = -1000;  // (no pflag value)
+template <bool COLD = false, bool CYCLE = false>
+__device__ __forceinline__ int newton(int& pflag, double& xio, const Inv& s, int& nstroke, int limit = 200)
 {
-  double x = xio, x_old = x, x_older = x, dx = 0.0, dx_old = D_VERYBIG, resid, jac, f = 1., df = 1.;
-  double errx = 1., damp = 1.0;
-  int n_iter = 0, i_extra = 0, lntries = 0;
-  bool doing_extra = false, keep = true, diddamp = false;
-  while (keep) {
-    nstroke++;
-    lntries++;
-    if (lntries > 10 && !diddamp) damp = 0.5;
-    residual<COLD>(x, s, dx, resid, jac, f, df);
-    x_older = x_old;
-    x_old = x;
-    diddamp = false;
-    if (n_iter == 0) {
-      x_older = x;
+  double x = xio, x_old = x, dx_old = 0.0, resid = 0.0;
+  double errn = 1.0, errd = 1.0;  // the error is |errn| / errd
+  double damp = 1.0;
+  int i_extra = 0, it = 0, skipped = 0;  // it + skipped: iterations done; it is the same in every lane
+  bool doing_extra = false, diddamp = false, keep = true;
+  double cx = 0.0, cxo = 0.0, cdx = 0.0;  // the state kept at the start of iteration ck
+  int ck = 0, cknext = 12;
+  const bool mod = !COLD && moderate(s) && s.w0 > 0.0;
+  const double wlim = 0.999 * (s.gsq_too_big * s.w1);
+#pragma clang loop unroll(disable)
+  do {
+    if (it >= 10 && !diddamp) damp = 0.5;
+    double dxn, rn;
+    bool ok = false;
+    if (!COLD) {
+      ok = func_eprime_q(x, s, dxn, rn);
+      const double xn = x + damp * dxn;
+      const double en = fabs(it == 0 ? dxn : dx_old), ed = fmax(fabs(s.w0), fabs(xn));
+      const bool ur = (fabs(s.w1) > s.w2) | (fabs(xn) > s.w2);
+      const double el = (ur ? D_NUMEPSILON : 1E3 * D_NUMEPSILON) * ed;
+      const bool ec = en < 0.999 * el;
+      ok = mod & ok & (ec | (en >= 1.001 * el)) & (xn >= -s.D) & (fabs(xn) < wlim);
+      if (ok) {
+        x_old = x;
+        x = xn;
+        dx_old = dxn;
+        errn = en;
+        errd = ed;
+        resid = rn;
+        diddamp = false;
+        doing_extra = doing_extra || ec;
+        i_extra += doing_extra ? 1 : 0;
+        keep = i_extra <= (ur ? 4 : 2);
+      }
+    }
+    if (!ok) {  // the reference's iteration as it stands
+      double dx, jac, f, df, x_older;
+      residual<COLD>(x, s, dx, resid, jac, f, df);
+      x_older = x_old;
       x_old = x;
-      dx_old = dx;
-    } else {
-      if (resid <= -D_VERYBIG || jac == 0.0) {
+      diddamp = false;
+      if (it == 0) {
+        dx_old = dx;
+      } else if (resid <= -D_VERYBIG || jac == 0.0) {
         damp = 0.5 * damp;
         x = x_older;
-        dx = dx_old;
         diddamp = true;
         residual<COLD>(x, s, dx, resid, jac, f, df);
-        if (resid <= -D_VERYBIG || jac == 0.0) { xio = x; return 1; }
-        x_older = x;
+        if (resid <= -D_VERYBIG || jac == 0.0) {
+          nstroke += it + 1 + skipped;
+          xio = x;
+          return 1;
+        }
         x_old = x;
         dx_old = dx;
       }
+      x += damp * dx;
+      errn = fabs(dx_old);
+      errd = (s.w0 == 0.) ? 1.0 : fmax(fabs(s.w0), fabs(x));
+      validate_wp(x_old, x, s);
+      dx_old = dx;
+      const bool ec = errcheck(errn / errd, x, s);
+      const int xc = extracheck(x, s);
+      doing_extra = doing_extra || ec;  // (extracheck is 2 or 4)
+      i_extra += doing_extra ? 1 : 0;
+      keep = i_extra <= xc;
     }
-    x += damp * dx;
-    errx = (s.w0 == 0.) ? fabs(dx_old) : fabs(dx_old / fmax(fabs(s.w0), fabs(x)));
-    validate_wp(x_old, x, s);
-    dx_old = dx;
-    const bool ec = errcheck(errx, x, s);
-    const int xc = extracheck(x, s);
-    if (ec && !doing_extra && xc > 0) doing_extra = true;
-    if (doing_extra) i_extra++;
-    if ((ec && !doing_extra) || (i_extra > xc) || (n_iter >= 199)) keep = false;
-    n_iter++;
-  }
+    it++;
+    if (it + skipped >= 200) keep = false;
+    if (CYCLE && it >= 12 && keep && !doing_extra && !diddamp && damp == 0.5) {
+      if (ck != 0 && x == cx && x_old == cxo && dx_old == cdx) {
+        const int period = it - ck;
+        skipped = (199 - it) / period * period;
+        ck = 0;
+        cknext = 0;
+      } else if (it == cknext) {
+        cx = x;
+        cxo = x_old;
+        cdx = dx_old;
+        ck = it;
+        cknext = 2 * it - 8;
+      }
+    }
+  } while (keep && it < limit);
+  nstroke += it + skipped;
+  if (keep) return kUnfinished;
+  const double f = COLD ? 0.5 * resid * resid : 0.5 * (resid * resid), df = -2. * f, errx = errn / errd;
   if (!isfinite(x) || !isfinite(f) || !isfinite(df)) {
     pflag = 8;
     xio = x;
@@ -610,9 +728,9 @@ __device__ __forceinline__ void inv_setup(const double* Ut, const Geom& g, doubl
 
 // COLD: the cold GRMHD solve (eomtype EOMCOLDGRMHD): the cold EOS (pressure 0,
 // pickeos_eomtype eos.c:259, coldeos.c) in the guess and the result, u = 0.
-template <bool COLD = false>
+template <bool COLD = false, bool CYCLE = false>
 __device__ __forceinline__ int new_body(int& pflag, const double* Ut, const Geom& g, double gam, double gammafail,
-                                        double* prim, int& nstroke, double wp_seed)
+                                        double* prim, int& nstroke, double wp_seed, int limit = 200)
 {
   Inv s;
   pflag = 0;
@@ -684,7 +802,7 @@ __device__ __forceinline__ int new_body(int& pflag, const double* Ut, const Geom
   }
 
   double Wp = Wp_last;
-  const int rv = newton<COLD>(pflag, Wp, s, nstroke);
+  const int rv = newton<COLD, CYCLE>(pflag, Wp, s, nstroke, limit);
   if (rv != 0) return rv;
 
   if (Wp == 1.e100) pflag = 51;
@@ -729,9 +847,12 @@ __device__ __forceinline__ int new_body(int& pflag, const double* Ut, const Geom
 }
 
 // Utoprim_jon_nonrelcompat_inputnorestmass on geometry-free Ugf.
-template <bool COLD = false>
+// *solved (if given): whether pr holds a solution; where it does not, pr is
+// left as it came in apart from the field, and a caller that reads it again
+// there need not keep it in registers.
+template <bool COLD = false, bool CYCLE = false>
 __device__ __forceinline__ int jon(const double* Ugf, const Geom& g, double gam, double gammafail, double* pr,
-                                   int& nstroke, double wp_seed)
+                                   int& nstroke, double wp_seed, int limit = 200, bool* solved = nullptr)
 {
   double Ut[HARM_NPR], pt[HARM_NPR];
   pr[HARM_B1] = Ugf[HARM_B1];
@@ -746,7 +867,9 @@ __device__ __forceinline__ int jon(const double* Ugf, const Geom& g, double gam,
   pt[HARM_B2] = alpha * pr[HARM_B2];
   pt[HARM_B3] = alpha * pr[HARM_B3];
   int pflag = 0;
-  const int ret = new_body<COLD>(pflag, Ut, g, gam, gammafail, pt, nstroke, wp_seed);
+  const int ret = new_body<COLD, CYCLE>(pflag, Ut, g, gam, gammafail, pt, nstroke, wp_seed, limit);
+  if (solved) *solved = ret == 0;
+  if (ret == kUnfinished) return kUnfinishedFlag;
   if (ret == 0) {
 #pragma unroll
     for (int i = 0; i <= HARM_U3; i++) pr[i] = pt[i];
@@ -765,12 +888,13 @@ __device__ __forceinline__ void geometry_free(const double* U, const Geom& g, do
 }
 
 // The hot solve of Utoprimgen(UEVOLVE): strip gdet then invert.
+template <bool CYCLE = false>
 __device__ __forceinline__ int utoprimgen(const double* U, const Geom& g, double gam, double gammafail, double* pr,
-                                          int& nstroke, double wp_seed)
+                                          int& nstroke, double wp_seed, int limit = 200, bool* solved = nullptr)
 {
   double Ugf[HARM_NPR];
   geometry_free(U, g, Ugf);
-  return jon(Ugf, g, gam, gammafail, pr, nstroke, wp_seed);
+  return jon<false, CYCLE>(Ugf, g, gam, gammafail, pr, nstroke, wp_seed, limit, solved);
 }
 
 // check_on_inversion with FAILIFBADCHECK (utoprimgen.c:697-850, :18) after the

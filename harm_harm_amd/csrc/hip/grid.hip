@@ -318,7 +318,7 @@ __device__ __forceinline__ void invert_body(Dims d, Params P, const double* __re
 // DIAG: also keeps the states the fixes started from (floors_zone; fx = {p0,
 // after-floor, flags}).
 template <bool DIAG = false>
-__device__ __forceinline__ void floors_body(Dims d, Params P, double* __restrict__ pf, int32_t* __restrict__ pflag,
+__device__ __forceinline__ void floors_body(Dims d, Params P, double* pf, int32_t* __restrict__ pflag,
                                             const double* __restrict__ gcent, const double* __restrict__ floors,
                                             unsigned long long* __restrict__ di, const int blk,
                                             double* __restrict__ fx_p0 = nullptr,
@@ -334,14 +334,11 @@ __device__ __forceinline__ void floors_body(Dims d, Params P, double* __restrict
     const long o = hd::cidx(d, i, j, k);
     const long pp = hd::pidx(d, i, j);
     const long nc = d.ncell;
-    Geom G;
-    hd::load_geom(gcent, pp, d.nplane, G);
     double pz[HARM_NPR];
-#pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = pf[pl * nc + o];
     const int fl0 = pflag[o];
     bool changed;
-    const int fl = floors_zone<DIAG>(d, P, G, floors, pz, fl0, o, pp, ns, &changed, fx_p0, fx_pfl, fx_flag);
+    const int fl =
+        floors_zone<DIAG>(d, P, gcent, floors, pf, pz, fl0, o, pp, ns, &changed, fx_p0, fx_pfl, fx_flag);
     if (changed) {
 #pragma unroll
       for (int pl = 0; pl < HARM_NPR; pl++) pf[pl * nc + o] = pz[pl];
@@ -352,9 +349,12 @@ __device__ __forceinline__ void floors_body(Dims d, Params P, double* __restrict
   newton_counts_to(ns, nf, di);
 }
 
-// Four waves per SIMD (128 VGPRs): measured faster than three on the torus
-// step.
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_invert(
+// Bound by issue: about 1000 instructions a wave around the Newton iterations
+// and 176 in each of them.  Three waves per SIMD: at four the solve spills 100 B
+// a lane (188 us a launch at 256x128x64 against 171; 177 with the scaled
+// divisions).  The floors likewise: 206 us at three waves, 226 at two, 251 at
+// four; 230 with the geometry and the primitives kept through the solve.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_invert(
     Dims d, Params P, const double* __restrict__ U, const double* __restrict__ pg, double* __restrict__ pf,
     int32_t* __restrict__ pflag, const double* __restrict__ gcent, int finalstep, unsigned long long* __restrict__ di)
 {
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 }
 
 template <bool DIAG>
-__global__ __launch_bounds__(kBlock) void k_floors(Dims d, Params P, double* __restrict__ pf,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_floors(Dims d, Params P, double* pf,
                                                    int32_t* __restrict__ pflag, const double* __restrict__ gcent,
                                                    const double* __restrict__ floors,
                                                    unsigned long long* __restrict__ di, double* __restrict__ fx_p0,
@@ -1643,7 +1643,7 @@ __global__ __launch_bounds__(kBlock) void kb_update(const GridRef* __restrict__ 
                         gmem(g.conn), cuf0, cuf1, cuf2, cun0, cun1, cun2, timeorder, gmem(g.ds), lb);
 }
 
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void kb_invert(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void kb_invert(
     const GridRef* __restrict__ G, const int* __restrict__ pre, int ng, int which_pb, int which_pf, int finalstep)
 {
   BATCH_DECODE(true)
@@ -1651,7 +1651,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
               gmem(g.arr[which_pf]), gmem(g.pflag), gmem(g.geom[HARM_LOC_CENT]), finalstep, gmem(g.di), lb);
 }
 
-__global__ __launch_bounds__(kBlock) void kb_floors(const GridRef* __restrict__ G, const int* __restrict__ pre, int ng,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void kb_floors(const GridRef* __restrict__ G, const int* __restrict__ pre, int ng,
                                                     int which_pf)
 {
   BATCH_DECODE(true)

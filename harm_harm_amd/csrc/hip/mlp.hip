@@ -519,7 +519,7 @@ __global__ __launch_bounds__(kBlock) void k_invert_grid_mlp(const uint16_t* __re
                                                             const float* __restrict__ w32,
                                                             const float* __restrict__ norm, hd::Dims d, hk::Params P,
                                                             const double* __restrict__ U,
-                                                            const double* __restrict__ pg, double* __restrict__ pf,
+                                                            const double* __restrict__ pg, double* pf,
                                                             int32_t* __restrict__ pflag,
                                                             const double* __restrict__ gcent,
                                                             const double* __restrict__ floors, int finalstep,
