@@ -218,7 +218,10 @@ __device__ __forceinline__ void newton_counts_to(int ns, int nf, unsigned long l
   __syncthreads();
   if (threadIdx.x == 0) {
     if (red[0]) atomicAdd(&di[DI_NSTROKE], red[0]);
-    if (red[1]) atomicAdd(&di[DI_NFAIL], red[1]);
+    if (red[1]) {
+      atomicAdd(&di[DI_NFAIL], red[1]);
+      atomicAdd(&di[DI_FIX], red[1]);
+    }
   }
 }
 

@@ -458,6 +458,13 @@ __device__ __forceinline__ void func_eprime(double Wp, const Inv& s, double& dx,
   df = -2. * f;
 }
 
+// the conjunction without short circuits (no branches)
+template <class... B>
+__device__ __forceinline__ bool all_of(B... b)
+{
+  return (int(b) & ...) != 0;
+}
+
 // Whether a solve's invariants lie where func_eprime_q's unscaled quotients
 // hold (dphys.h's ranges): with these bounds and 1e-40 < W < 1e40 no
 // denominator or quotient below leaves 1e-271 .. 1e271.
@@ -498,8 +505,8 @@ __device__ __forceinline__ bool func_eprime_q(double Wp, const Inv& s, double& d
   resid = Ep;
   dx = quot(-Ep, recip(dE));
   // (a NaN anywhere makes Ep or dE one)
-  return (W > 1e-40) & (W < 1e40) & (gammasq > 1e-40) & (gammasq < 1e250) & (utsq >= -0.9 * s.utsq_too_big) &
-         (fabs(Ep) < 1e100) & (fabs(dE) > 1e-40) & (fabs(dE) < 1e250);
+  return all_of(W > 1e-40, W < 1e40, gammasq > 1e-40, gammasq < 1e250, utsq >= -0.9 * s.utsq_too_big,
+                fabs(Ep) < 1e100, fabs(dE) > 1e-40, fabs(dE) < 1e250);
 }
 
 // Cold GRMHD residual W^2 P^2 of the momentum equation and its W' derivative
@@ -592,10 +599,10 @@ __device__ __forceinline__ int newton(int& pflag, double& xio, const Inv& s, int
       ok = func_eprime_q(x, s, dxn, rn);
       const double xn = x + damp * dxn;
       const double en = fabs(it == 0 ? dxn : dx_old), ed = fmax(fabs(s.w0), fabs(xn));
-      const bool ur = (fabs(s.w1) > s.w2) | (fabs(xn) > s.w2);
+      const bool ur = !all_of(!(fabs(s.w1) > s.w2), !(fabs(xn) > s.w2));
       const double el = (ur ? D_NUMEPSILON : 1E3 * D_NUMEPSILON) * ed;
       const bool ec = en < 0.999 * el;
-      ok = mod & ok & (ec | (en >= 1.001 * el)) & (xn >= -s.D) & (fabs(xn) < wlim);
+      ok = all_of(mod, ok, !all_of(!ec, !(en >= 1.001 * el)), xn >= -s.D, fabs(xn) < wlim);
       if (ok) {
         x_old = x;
         x = xn;

@@ -21,8 +21,11 @@ enum { DS_DT = 0, DS_T = 1, DS_NDT1 = 2, DS_NDT2 = 3, DS_NDT3 = 4, DS_ACCDT = 5,
 // Newton counters: the current step's, and their sums over the steps since
 // the time was last set
 // and the zones whose learned-guess solve fell back to the plain guess
+// DI_FIX: zones of the current substep that its inversion left with pflag > 0
+// (what failure averaging will change); DI_TICKET: blocks of the 2-D boundary
+// launch that are done, 0 between launches
 enum { DI_NSTROKE = 0, DI_NFAIL = 1, DI_NSTROKE_SUM = 2, DI_NFAIL_SUM = 3, DI_NFALLBACK = 4, DI_NFALLBACK_SUM = 5,
-       DI_N = 8 };
+       DI_FIX = 6, DI_TICKET = 7, DI_N = 8 };
 // Energy-file accumulators (dump_ener.c:391-407), per grid: boundary flux
 // sums of the last substep (pdot) and their time integral (pcum), six
 // boundaries X1UP, X1DN, X2UP, X2DN, X3UP, X3DN by eight variables; the

@@ -565,8 +565,10 @@ template <bool DIAG>
 __global__ __launch_bounds__(kBlock) void k_post_fixup(Dims d, Params P, const double* __restrict__ pf,
                                                        const int32_t* __restrict__ pflag, double* __restrict__ pout,
                                                        const double* __restrict__ gcent, int finalstep,
-                                                       double* __restrict__ fl_part)
+                                                       double* __restrict__ fl_part,
+                                                       const unsigned long long* __restrict__ di)
 {
+  if (!DIAG && di && di[DI_FIX] == 0) return;  // di: inside a step, where the inversion counted the failed zones
   double dfl[HARM_NPR] = {0, 0, 0, 0, 0, 0, 0, 0};
   int cat = 0;
   const bool ch = post_fixup_body<DIAG>(d, P, pf, pflag, pout, gcent, finalstep, blockIdx.x, dfl, &cat);
@@ -606,8 +608,10 @@ __device__ __forceinline__ void fixup_apply_body(const Dims& d, double* __restri
 }
 
 __global__ __launch_bounds__(kBlock) void k_fixup_apply(Dims d, double* __restrict__ pf, int32_t* __restrict__ pflag,
-                                                        const double* __restrict__ pin, int finalstep)
+                                                        const double* __restrict__ pin, int finalstep,
+                                                        const unsigned long long* __restrict__ di)
 {
+  if (di && di[DI_FIX] == 0) return;
   fixup_apply_body(d, pf, pflag, pin, finalstep, blockIdx.x);
 }
 
@@ -619,7 +623,7 @@ __global__ __launch_bounds__(kBlock) void k_fixup_apply(Dims d, double* __restri
 // three boundary zones, which no ghost write touches, so the ghost zones of a
 // line can be filled by separate threads.
 __device__ void extrap_line(const Dims& d, const Params& P, double* p, const double* gcent, int up, int j, int k,
-                            int gsel)
+                            int gsel, long img = 0)
 {
   const long nc = d.ncell;
   const int ri = up ? d.n1 - 1 : 0;
@@ -714,7 +718,10 @@ __device__ void extrap_line(const Dims& d, const Params& P, double* p, const dou
     }
     const long oi = hd::cidx(d, i, j, k);
 #pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) p[pl * nc + oi] = pi[pl];
+    for (int pl = 0; pl < HARM_NPR; pl++) {
+      p[pl * nc + oi] = pi[pl];
+      if (img) p[pl * nc + oi + img] = pi[pl];
+    }
   }
 }
 
@@ -776,8 +783,10 @@ __global__ __launch_bounds__(kBlock) void k_bound_x1(Dims d, Params P, double* _
 }
 
 // one ghost zone of the polar reflection: ghost row j = -ng2 + g (side 0) or
-// n2 + g (side 1) of column col = (i + ng1) + ns1 * k
-__device__ __forceinline__ void x2_reflect_zone(const Dims& d, double* __restrict__ p, int side, int g, long col)
+// n2 + g (side 1) of column col = (i + ng1) + ns1 * k; img (not 0): the offset
+// of a second place that gets the same values, the plane's periodic image
+__device__ __forceinline__ void x2_reflect_zone(const Dims& d, double* __restrict__ p, int side, int g, long col,
+                                                long img = 0)
 {
   const int i = (int)(col % d.ns1) - d.ng1, k = (int)(col / d.ns1);
   const int n2 = d.n2, n3 = d.n3;
@@ -791,6 +800,7 @@ __device__ __forceinline__ void x2_reflect_zone(const Dims& d, double* __restric
     double v = p[pl * nc + so];
     if (pl == HARM_U2 || pl == HARM_B2) v *= -1.;
     p[pl * nc + doff] = v;
+    if (img) p[pl * nc + doff + img] = v;
   }
 }
 
@@ -814,7 +824,7 @@ __global__ __launch_bounds__(kBlock) void k_x2_reflect(Dims d, double* __restric
 // directly (the reflection of that ghost row has not run).
 __device__ __forceinline__ void x2_poledeath_col(const Dims& d, const Params& P, double* __restrict__ p,
                                                  const double* __restrict__ gcent, const double* __restrict__ rcent,
-                                                 int side, long col, bool mirror_ghost = false)
+                                                 int side, long col, bool mirror_ghost = false, long img = 0)
 {
   const int i = (int)(col % d.ns1) - d.ng1, k = (int)(col / d.ns1);
   const int n2 = d.n2, n3 = d.n3;
@@ -866,7 +876,10 @@ __device__ __forceinline__ void x2_poledeath_col(const Dims& d, const Params& P,
       hd::limit_gamma(P.gammamax, pj, Gj);
     }
 #pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) p[pl * nc + o] = pj[pl];
+    for (int pl = 0; pl < HARM_NPR; pl++) {
+      p[pl * nc + o] = pj[pl];
+      if (img) p[pl * nc + o + img] = pj[pl];
+    }
   }
 }
 
@@ -944,10 +957,201 @@ __global__ __launch_bounds__(kBlock) void k_bound_x3(Dims d, double* __restrict_
 }
 
 // ---------------------------------------------------------------------------
+// The whole boundary pass in one launch
+// ---------------------------------------------------------------------------
+// A substep applies the boundary conditions twice, around failure averaging,
+// and each of their three directions reads what the one before wrote, so they
+// were six launches, with the flag bounds and the averaging ten; a dependent
+// launch costs about 4.5 us whatever it does, which was most of a step on the
+// 2-D grids.  Here each block owns a closed set of zones:
+//  A: a chunk of rows at one radial end, in one phi plane and the plane half a
+//     turn away (polar reflection reads across).  Its radial ghost zones first;
+//     then, if the chunk holds a pole's rows, after a barrier the polar rows of
+//     the ghost columns and of the three active columns the extrapolation
+//     reads (pole death rewrites the first active row, which the extrapolation
+//     must see as it was).
+//  B: the polar rows of the other active columns, which no radial ghost enters.
+//  C: phi ghost planes: the active rows that no pole rewrites, copied from
+//     their source planes.  Everything A and B write in a plane that has a
+//     periodic image goes to the image too.
+//  D: the flags' ghost layer (bound_pflag), both phases: the flags phase 0
+//     copies along phi before phase 1 rewrites them are copied by the thread
+//     that then rewrites them.
+// Needs n2 > ng2 (as x2_poles) and n1 >= 8 (the two radial ends' columns are
+// disjoint); other grids take the direction-by-direction launches.
+// On such grids the pass applied twice gives the same values as once: the rows
+// it reads are rows it does not write, except the first active row's fields in
+// 2-D and its other variables, which both come from the second active row
+// alone.  So the second pass of a substep runs only where failure averaging
+// changed zones (DI_FIX).
+struct BoundPlan {
+  int nchunk, nA, nB, nC, nD;
+  __host__ __device__ int total() const { return nA + nB + nC + nD; }
+};
+__host__ __device__ __forceinline__ bool bounds_merge(const Dims& d) { return d.n1 >= 8 && d.n2 > d.ng2; }
+__host__ __device__ __forceinline__ long pflag_items(const Dims& d)
+{
+  return (long)d.n2 * d.n3 + (long)(d.n1 + 2) * d.n3 + (d.n3 > 1 ? (long)(d.n1 + 1) * d.n2 : 0);
+}
+__host__ __device__ __forceinline__ BoundPlan bound_plan(const Dims& d, bool flags)
+{
+  BoundPlan b;
+  const int rows = kBlock / (d.ng1 * (d.n3 > 1 ? 2 : 1));  // one radial ghost zone a thread
+  b.nchunk = (d.n2 + rows - 1) / rows;
+  while (b.nchunk > 1 && d.n2 / b.nchunk < d.ng2) b.nchunk--;  // a pole's rows in one chunk
+  b.nA = 2 * b.nchunk * (d.n3 > 1 ? d.n3 / 2 : 1);
+  b.nB = (int)((2L * (d.n1 - 6) * d.n3 * d.ng2 + kBlock - 1) / kBlock);
+  b.nC = d.n3 > 1 ? (int)(((long)d.n1 * (d.n2 - 2) * 2 * d.ng3 + kBlock - 1) / kBlock) : 0;
+  b.nD = flags ? (int)((pflag_items(d) + kBlock - 1) / kBlock) : 0;
+  return b;
+}
+
+// offset of plane k's periodic image, 0 if it has none
+__device__ __forceinline__ long phi_image(const Dims& d, int k)
+{
+  if (d.n3 == 1) return 0;
+  return k < d.ng3 ? d.n3 * d.nplane : k >= d.n3 - d.ng3 ? -d.n3 * d.nplane : 0;
+}
+
+// polar item g of column (i, k) at one pole: 0 the rows next to the pole
+// (pole death; Bondi: the first ghost row), 1 .. ng2-1 the ghost rows beyond
+__device__ __forceinline__ void polar_item(const Dims& d, const Params& P, double* p, const double* gcent,
+                                           const double* rcent, int side, int g, int i, int k)
+{
+  const long col = (i + d.ng1) + (long)d.ns1 * k, img = phi_image(d, k);
+  if (g > 0) x2_reflect_zone(d, p, side, g - 1 + side, col, img);
+  else if (P.bc == HARM_PROBLEM_BONDI) x2_reflect_zone(d, p, side, side == 0 ? d.ng2 - 1 : 0, col, img);
+  else x2_poledeath_col(d, P, p, gcent, rcent, side, col, true, img);
+}
+
+__device__ __forceinline__ void bounds_prims(const Dims& d, const Params& P, const BoundPlan& b, double* p,
+                                             const double* gcent, const double* rcent, int blk)
+{
+  const int tid = threadIdx.x;
+  const bool A = blk < b.nA;
+  int up = 0, pr = 0, lo = 1, hi = 1;
+  if (A) {
+    const int c = (blk >> 1) % b.nchunk, np = d.n3 > 1 ? 2 : 1;
+    up = blk & 1;
+    pr = (blk >> 1) / b.nchunk;
+    const int j0 = (int)((long)d.n2 * c / b.nchunk), nr = (int)((long)d.n2 * (c + 1) / b.nchunk) - j0;
+    for (int t = tid; t < nr * d.ng1 * np; t += kBlock) {
+      const int gsel = t % d.ng1, r = t / d.ng1, j = j0 + r % nr, k = pr + (r / nr) * (d.n3 / 2);
+      if (P.bc == HARM_PROBLEM_BONDI) bondi_line(d, P, p, gcent, up, j, k, gsel);
+      else extrap_line(d, P, p, gcent, up, j, k, gsel, phi_image(d, k));
+    }
+    lo = c == 0;
+    hi = c == b.nchunk - 1;
+    if (!lo && !hi) return;
+    __syncthreads();
+  }
+  if (blk < b.nA + b.nB) {
+    // polar items: of a block's edge columns (A), or one a thread of the others (B)
+    const int m = A ? d.ng1 + 3 : d.n1 - 6, np = A ? (d.n3 > 1 ? 2 : 1) : d.n3, i0 = A ? (up ? d.n1 - 3 : -d.ng1) : 3;
+    const long n = (long)m * np * d.ng2 * (lo + hi);
+    const long t0 = A ? 0 : (long)(blk - b.nA) * kBlock, t1 = A ? n : min(n, t0 + kBlock);
+    for (long t = t0 + tid; t < t1; t += kBlock) {
+      const int i = i0 + (int)(t % m);
+      const long r = t / m;
+      const int kk = (int)(r % np), u = (int)(r / np);
+      polar_item(d, P, p, gcent, rcent, lo && hi ? u / d.ng2 : hi, u % d.ng2, i, A ? pr + kk * (d.n3 / 2) : kk);
+    }
+    return;
+  }
+  const long t = (long)(blk - b.nA - b.nB) * kBlock + tid;
+  if (t >= (long)d.n1 * (d.n2 - 2) * 2 * d.ng3) return;
+  const int i = (int)(t % d.n1);
+  const long r = t / d.n1;
+  const int j = 1 + (int)(r % (d.n2 - 2)), g = (int)(r / (d.n2 - 2));
+  const int k = g < d.ng3 ? -d.ng3 + g : d.n3 + (g - d.ng3);
+  const long o = hd::cidx(d, i, j, k), so = hd::cidx(d, i, j, k < 0 ? k + d.n3 : k - d.n3);
+#pragma unroll
+  for (int pl = 0; pl < HARM_NPR; pl++) p[pl * d.ncell + o] = p[pl * d.ncell + so];
+}
+
+__device__ __forceinline__ void bounds_flags(const Dims& d, int bc, int32_t* __restrict__ pflag, long t)
+{
+  const int n1 = d.n1, n2 = d.n2, n3 = d.n3;
+  auto at = [&](int i, int j, int k) -> int32_t& { return pflag[hd::cidx(d, i, j, k)]; };
+  auto rewrite = [&](int i, int j, int k, int32_t v) {  // phase 0's copy of the old flag, then phase 1's flag
+    const int32_t old = at(i, j, k);
+    if (n3 > 1 && k == 0) at(i, j, n3) = old;
+    if (n3 > 1 && k == n3 - 1) at(i, j, -1) = old;
+    at(i, j, k) = v;
+  };
+  const long nr = (long)n2 * n3, np = (long)(n1 + 2) * n3;
+  if (t < nr) {  // radial copy (torus, outer end)
+    const int j = (int)(t % n2), k = (int)(t / n2);
+    if (bc == HARM_PROBLEM_TORUS) rewrite(n1, j, k, at(n1 - 1, j, k));
+    return;
+  }
+  t -= nr;
+  if (t < np) {  // polar mirrors
+    const int i = (int)(t % (n1 + 2)) - 1, k = (int)(t / (n1 + 2));
+    const int ii = (i == n1 && bc == HARM_PROBLEM_TORUS) ? n1 - 1 : i;
+    rewrite(i, -1, k, at(ii, 0, k));
+    rewrite(i, n2, k, at(ii, n2 - 1, k));
+    return;
+  }
+  t -= np;
+  if (n3 == 1 || t >= (long)(n1 + 1) * n2) return;
+  const int i = (int)(t % (n1 + 1)) - 1, j = (int)(t / (n1 + 1));
+  at(i, j, -1) = at(i, j, n3 - 1);
+  at(i, j, n3) = at(i, j, 0);
+}
+
+// cond: the second pass, only where failure averaging changed zones and
+// without the flags (a batch counts their blocks for both passes).  FIX2D (2-D grids, flags
+// bounded in the same launch): the block that ends last goes on with failure
+// averaging and the second pass when there are failed zones; they are few, so
+// one block is enough.  Its zones come from every block, hence the fences.
+template <bool FIX2D>
+__device__ __forceinline__ void bounds_body(const Dims& d, const Params& P, double* p, const double* gcent,
+                                            const double* rcent, int32_t* pflag, double* pfix,
+                                            unsigned long long* di, int finalstep, bool flags, bool cond, int blk)
+{
+  const bool fix = (FIX2D || cond) && di[DI_FIX] != 0;
+  if (cond && !fix) return;
+  const BoundPlan b = bound_plan(d, flags);
+  const int nprim = b.nA + b.nB + b.nC;
+  if (blk >= nprim && !cond) bounds_flags(d, P.bc, pflag, (long)(blk - nprim) * kBlock + threadIdx.x);
+  int v0 = blk, v1 = blk < nprim ? blk + 1 : blk;
+  for (bool again = false;; again = true) {
+    for (int v = v0; v < v1; v++) bounds_prims(d, P, b, p, gcent, rcent, v);
+    if (!FIX2D || !fix) return;
+    if (again) break;
+    __shared__ bool last;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(&di[DI_TICKET], 1ull) == (unsigned long long)(b.total() - 1);
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    const int nz = (d.n1 * d.n2 * d.n3 + kBlock - 1) / kBlock;
+    for (int z = 0; z < nz; z++) post_fixup_body(d, P, p, pflag, pfix, gcent, finalstep, z);
+    __syncthreads();
+    for (int z = 0; z < nz; z++) fixup_apply_body(d, p, pflag, pfix, finalstep, z);
+    __syncthreads();
+    v0 = 0;
+    v1 = nprim;
+  }
+  if (threadIdx.x == 0) di[DI_TICKET] = 0;
+}
+
+template <bool FIX2D>
+__global__ __launch_bounds__(kBlock) void k_bounds(Dims d, Params P, double* p, const double* gcent,
+                                                   const double* rcent, int32_t* pflag, double* pfix,
+                                                   unsigned long long* di, int finalstep, int flags, int cond)
+{
+  bounds_body<FIX2D>(d, P, p, gcent, rcent, pflag, pfix, di, finalstep, flags, cond, blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------
 // scalars: reset, per-substep dt, end of step
 // ---------------------------------------------------------------------------
-__global__ void k_scal_begin_flux(double* ds)
+__global__ void k_scal_begin_flux(double* ds, unsigned long long* di)
 {
+  di[DI_FIX] = 0;
   ds[DS_NDT1] = kBIG;
   ds[DS_NDT2] = kBIG;
   ds[DS_NDT3] = kBIG;
@@ -1307,7 +1511,7 @@ harm_status enq_fluxcalc(harm_handle* h, int which_p, int do_ct)
   const Dims& d = h->d;
   hipStream_t s = h->stream;
   const double* pb = h->arr[which_p];
-  hipLaunchKernelGGL(k_scal_begin_flux, dim3(1), dim3(1), 0, s, h->ds);
+  hipLaunchKernelGGL(k_scal_begin_flux, dim3(1), dim3(1), 0, s, h->ds, h->di);
   const int recon = h->cfg.recon, ft = h->cfg.flux;
   const bool weno = recon == HARM_RECON_WENO5;
   if (weno) {
@@ -1432,12 +1636,20 @@ harm_status enq_invert(harm_handle* h, int which_pb, int which_pf, int finalstep
   return hh::check_launch("k_invert");
 }
 
-harm_status enq_bound(harm_handle* h, int which)
+// flags: bound the flags in the same launch; cond: only where the substep's
+// inversion left failed zones (bounds_merge grids)
+harm_status enq_bound(harm_handle* h, int which, bool flags = false, bool cond = false)
 {
   const Dims& d = h->d;
   hipStream_t s = h->stream;
   double* p = h->arr[which];
   prof_begin(h);
+  if (bounds_merge(d)) {
+    hipLaunchKernelGGL(k_bounds<false>, dim3((unsigned)bound_plan(d, flags).total()), dim3(kBlock), 0, s, d, h->P, p,
+                       h->geom[HARM_LOC_CENT], h->rcent, h->pflag, nullptr, h->di, 0, flags, cond);
+    prof_end(h, HARM_K_BOUND);
+    return hh::check_launch("k_bounds");
+  }
   if (d.n1 > 1)
     hipLaunchKernelGGL(k_bound_x1, dim3(nblocks(2L * d.ng1 * d.n2 * d.n3)), dim3(kBlock), 0, s, d, h->P, p,
                        h->geom[HARM_LOC_CENT]);
@@ -1460,25 +1672,27 @@ harm_status enq_bound(harm_handle* h, int which)
 // scratch pfix (reading pf and the flags unchanged: failed neighbours are read
 // too), then write them back and mark the accounted zones.
 // ener: the averaged zones' changes go to their fladdterms (final substep only)
-harm_status enq_post_fixup(harm_handle* h, int which, int finalstep, bool ener = false)
+// bounded: the flags are bounded and the failed zones counted (inside a step)
+harm_status enq_post_fixup(harm_handle* h, int which, int finalstep, bool ener = false, bool bounded = false)
 {
   const Dims& d = h->d;
   const unsigned nb = nblocks((long)d.n1 * d.n2 * d.n3);
   prof_begin(h);
-  for (int ph = 0; ph < 2; ph++) {
+  for (int ph = 0; ph < 2 && !bounded; ph++) {
     const long n = bound_pflag_items(d, ph);
     if (n > 0)
       hipLaunchKernelGGL(k_bound_pflag, dim3(nblocks(n)), dim3(kBlock), 0, h->stream, d, h->cfg.problem, h->pflag,
                          ph);
   }
+  const unsigned long long* di = bounded ? h->di : nullptr;
   if (ener)
     hipLaunchKernelGGL(k_post_fixup<true>, dim3(nb), dim3(kBlock), 0, h->stream, d, h->P, h->arr[which], h->pflag,
-                       h->pfix, h->geom[HARM_LOC_CENT], finalstep, h->enpart);
+                       h->pfix, h->geom[HARM_LOC_CENT], finalstep, h->enpart, di);
   else
     hipLaunchKernelGGL(k_post_fixup<false>, dim3(nb), dim3(kBlock), 0, h->stream, d, h->P, h->arr[which], h->pflag,
-                       h->pfix, h->geom[HARM_LOC_CENT], finalstep, nullptr);
+                       h->pfix, h->geom[HARM_LOC_CENT], finalstep, nullptr, di);
   hipLaunchKernelGGL(k_fixup_apply, dim3(nb), dim3(kBlock), 0, h->stream, d, h->arr[which], h->pflag, h->pfix,
-                     finalstep);
+                     finalstep, di);
   prof_end(h, HARM_K_FIXUP);
   if (ener) {
     int dst[4];
@@ -1486,6 +1700,27 @@ harm_status enq_post_fixup(harm_handle* h, int which, int finalstep, bool ener =
     launch_ener_reduce(h->enpart, nb, h->en, dst, 4, h->stream);
   }
   return hh::check_launch("k_post_fixup");
+}
+
+// The end of a substep (post_advance): bounds, failure averaging, bounds.  On
+// 2-D grids one launch, on 3-D ones four of which the last three have nothing
+// to do unless a zone failed; grids that bounds_merge leaves out take every
+// pass in full.
+harm_status enq_finish(harm_handle* h, int which, int finalstep, bool ener)
+{
+  const Dims& d = h->d;
+  const bool merge = bounds_merge(d);
+  if (merge && d.n3 == 1 && !ener) {
+    prof_begin(h);
+    hipLaunchKernelGGL(k_bounds<true>, dim3((unsigned)bound_plan(d, true).total()), dim3(kBlock), 0, h->stream, d,
+                       h->P, h->arr[which], h->geom[HARM_LOC_CENT], h->rcent, h->pflag, h->pfix, h->di, finalstep, 1,
+                       0);
+    prof_end(h, HARM_K_BOUND);
+    return hh::check_launch("k_bounds");
+  }
+  HH_TRY(enq_bound(h, which, merge));
+  HH_TRY(enq_post_fixup(h, which, finalstep, ener, merge));
+  return enq_bound(h, which, false, merge);
 }
 
 int rk_tables(int timeorder, double CUf[4][4], double Cunew[4][4])
@@ -1545,9 +1780,7 @@ harm_status enq_substep(harm_handle* h, int to, int nto, const double CUf[4][4],
   HH_TRY(enq_update(h, pii[to], pbb[to], CUf[to], Cunew[to], to, mode));
   HH_TRY(enq_invert(h, pbb[to], pff[to], finalstep, false, ener));
   hipLaunchKernelGGL(k_scal_substep_dt, dim3(1), dim3(1), 0, h->stream, h->ds);
-  HH_TRY(enq_bound(h, pff[to]));
-  HH_TRY(enq_post_fixup(h, pff[to], finalstep, ener && finalstep));
-  HH_TRY(enq_bound(h, pff[to]));
+  HH_TRY(enq_finish(h, pff[to], finalstep, ener && finalstep));
   return hh::check_launch("substep");
 }
 
@@ -1577,7 +1810,7 @@ void rk_flux_weights(int timeorder, double* w)
 // replayed.
 // ---------------------------------------------------------------------------
 enum { BS_FLUX1 = 0, BS_FLUX2, BS_FLUX3, BS_EMF, BS_CT, BS_FACC, BS_ZONE, BS_BX1, BS_X2R, BS_X2P,
-       BS_X2M, BS_BX3, BS_ONE, BS_PFB, BS_N };
+       BS_X2M, BS_BX3, BS_ONE, BS_PFB, BS_BND, BS_N };
 
 __device__ __forceinline__ void batch_decode(const int* __restrict__ pre, int ng, int b, int& gi, int& lb)
 {
@@ -1667,19 +1900,32 @@ __global__ __launch_bounds__(kBlock) void kb_bound_pflag(const GridRef* __restri
   if (t < bound_pflag_items(g.d, phase)) bound_pflag_body(g.d, g.P.bc, gmem(g.pflag), phase, t);
 }
 
+// cond: the grids' inversions counted the failed zones (bounds_merge grids)
 __global__ __launch_bounds__(kBlock) void kb_post_fixup(const GridRef* __restrict__ G, const int* __restrict__ pre,
-                                                        int ng, int which, int finalstep)
+                                                        int ng, int which, int finalstep, int cond)
 {
   BATCH_DECODE(false)
+  if (cond && gmem(g.di)[DI_FIX] == 0) return;
   post_fixup_body(g.d, g.P, gmem(g.arr[which]), gmem(g.pflag), gmem(g.pfix), gmem(g.geom[HARM_LOC_CENT]), finalstep,
                   lb);
 }
 
 __global__ __launch_bounds__(kBlock) void kb_fixup_apply(const GridRef* __restrict__ G, const int* __restrict__ pre,
-                                                         int ng, int which, int finalstep)
+                                                         int ng, int which, int finalstep, int cond)
 {
   BATCH_DECODE(false)
+  if (cond && gmem(g.di)[DI_FIX] == 0) return;
   fixup_apply_body(g.d, gmem(g.arr[which]), gmem(g.pflag), gmem(g.pfix), finalstep, lb);
+}
+
+// every grid's boundary pass (bounds_body); pre: block counts with the flags'
+template <bool FIX2D>
+__global__ __launch_bounds__(kBlock) void kb_bounds(const GridRef* __restrict__ G, const int* __restrict__ pre, int ng,
+                                                    int which, int finalstep, int cond)
+{
+  BATCH_DECODE(false)
+  bounds_body<FIX2D>(g.d, g.P, gmem(g.arr[which]), gmem(g.geom[HARM_LOC_CENT]), gmem(g.rcent), gmem(g.pflag),
+                     gmem(g.pfix), gmem(g.di), finalstep, true, cond, lb);
 }
 
 __global__ __launch_bounds__(kBlock) void kb_bound_x1(const GridRef* __restrict__ G, const int* __restrict__ pre,
@@ -1725,6 +1971,7 @@ __global__ void kb_scal(const GridRef* __restrict__ G, int ng, int what)
   double* ds = G[gi].ds;
   if (what == 0) {  // begin flux
     ds[DS_NDT1] = kBIG; ds[DS_NDT2] = kBIG; ds[DS_NDT3] = kBIG; ds[DS_ACCDT] = kBIG;
+    G[gi].di[DI_FIX] = 0;
   } else if (what == 1) {  // begin step
     ds[DS_LASTNDT] = kBIG;
     G[gi].di[DI_NSTROKE] = 0;
@@ -1787,6 +2034,7 @@ struct harm_batch {
   int ntot[BS_N] = {0};
   int recon = 0, timeorder = 0, dm = 0;
   bool x2_merged = true;  // every grid has n2 > ng2 (or no polar boundary): both poles in one launch
+  bool bnd_merged = true; // every grid takes the boundary pass in one launch (bounds_merge)
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
 };
@@ -1819,6 +2067,8 @@ harm_status batch_build(harm_batch* b)
     cnt[BS_BX3] = e2 ? nblocks(d.nplane * 2L * d.ng3) : 0;
     cnt[BS_ONE] = 1;
     cnt[BS_PFB] = nblocks(std::max(bound_pflag_items(d, 0), bound_pflag_items(d, 1)));
+    if (bounds_merge(d)) cnt[BS_BND] = bound_plan(d, true).total();
+    else b->bnd_merged = false;
     for (int st = 0; st < BS_N; st++) {
       const long nx = (long)pre[(size_t)st * (ng + 1) + gi] + cnt[st];
       if (nx > 0x7fffffffL) return hh::set_error(HARM_EINVAL, "harm_batch: too many blocks in one stage");
@@ -1899,12 +2149,24 @@ harm_status enq_batch_substep(harm_batch* b, int to, int nto, const double CUf[4
   if (finalstep) hipLaunchKernelGGL(kb_floors, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to]);
   hipLaunchKernelGGL(kb_scal, dim3(g1), dim3(64), 0, s, G, ng, 2);
   // bounds, failure averaging, bounds
+  if (b->bnd_merged) {
+    const dim3 gb((unsigned)b->ntot[BS_BND]);
+    if (b->dm == 3) {
+      hipLaunchKernelGGL(kb_bounds<true>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 0);
+    } else {
+      hipLaunchKernelGGL(kb_bounds<false>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 0);
+      hipLaunchKernelGGL(kb_post_fixup, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to], finalstep, 1);
+      hipLaunchKernelGGL(kb_fixup_apply, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to], finalstep, 1);
+      hipLaunchKernelGGL(kb_bounds<false>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 1);
+    }
+    return hh::check_launch("batch substep");
+  }
   for (int pass = 0; pass < 2; pass++) {
     if (pass == 1) {
       for (int ph = 0; ph < 2; ph++)
         hipLaunchKernelGGL(kb_bound_pflag, dim3((unsigned)b->ntot[BS_PFB]), blk, 0, s, G, P(BS_PFB), ng, ph);
-      hipLaunchKernelGGL(kb_post_fixup, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to], finalstep);
-      hipLaunchKernelGGL(kb_fixup_apply, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to], finalstep);
+      hipLaunchKernelGGL(kb_post_fixup, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to], finalstep, 0);
+      hipLaunchKernelGGL(kb_fixup_apply, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to], finalstep, 0);
     }
     if (b->ntot[BS_BX1]) hipLaunchKernelGGL(kb_bound_x1, dim3((unsigned)b->ntot[BS_BX1]), blk, 0, s, G, P(BS_BX1), ng,
                                             pff[to]);
