@@ -73,15 +73,17 @@ def algorithmic_bytes(g, kernel):
         return faces * ((128 if g.cfg.recon == H.RECON["weno5"] else 64) + 64) + ni * nj * geom
     zones = n1 * n2 * n3
     if kernel == "update":
-        # inside a step every substep moves 448 B per zone: pb 64 + 3 face
-        # fluxes 192 + (pi read, ui write | ui read, uf read) 128 + one of
-        # uf write / ucum write 64; plus geometry and connection per column
+        # inside a step every substep moves 448 B per zone: pb 64 + the mass,
+        # energy and momentum fluxes of 3 faces 120 + EMFs 24 + field fluxes
+        # written 48 + (pi read, ui write | ui read, uf read) 128 + one of uf
+        # write / ucum write 64; plus geometry and connection per column
         return zones * 448 + n1 * n2 * (geom + 40 * 8)
     if kernel == "invert":
         # U read, guess read, solution write, flag write
         return zones * (64 + 64 + 64 + 4) + n1 * n2 * geom
     if kernel == "emf_ct":
-        return zones * (6 * 8 + 3 * 8 + 3 * 8 + 6 * 8)
+        # six field fluxes read, three EMFs written (the update applies the CT)
+        return zones * (6 * 8 + 3 * 8)
     if kernel == "bound":
         # every ghost zone written once from a zone read once (8 doubles each)
         ghosts = (n1 + 2 * 4 * e0) * (n2 + 2 * 4 * e1) * (n3 + 2 * 4 * e2) - zones

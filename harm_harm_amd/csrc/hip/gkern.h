@@ -275,12 +275,16 @@ void launch_ener_totals(const hd::Dims& d, const Params& P, const double* p, con
                         double* out, hipStream_t s);
 
 // Launchers of the face-flux kernels (flux.hip): one direction of one grid,
-// or one direction of every grid of a batch.  With WENO5BND the face values
-// come from wl, wr (launch_weno_recon) instead of an in-tile reconstruction.
+// every direction of one grid (not WENO5BND; T, F, gface: directions 1 to 3),
+// or every direction of every grid of a batch (n, pre: blocks and prefix sums
+// of the three directions).  With WENO5BND the face values come from wl, wr
+// (launch_weno_recon) instead of an in-tile reconstruction.
 void launch_flux(int dir, int recon, const FaceTile& T, hipStream_t s, const Dims& d, const double* pb, double* F,
                  const double* gface, const Params& P, int fluxtype, int do_ct, double* ds,
                  const double* wl = nullptr, const double* wr = nullptr);
-void launch_flux_batch(int dir, int recon, unsigned nblk, hipStream_t s, const GridRef* G, const int* pre, int ng,
+void launch_flux_all(int recon, const FaceTile* T, hipStream_t s, const Dims& d, const double* pb, double* const* F,
+                     const double* const* gface, const Params& P, int fluxtype, int do_ct, double* ds);
+void launch_flux_batch(int recon, const int* n, const int* const* pre, hipStream_t s, const GridRef* G, int ng,
                        int which, int do_ct);
 // WENO5BND (weno.hip): the dP measure of every active direction, then the
 // face values of one direction's lines

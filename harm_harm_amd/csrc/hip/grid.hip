@@ -38,6 +38,88 @@ using namespace hk;
 
 namespace {
 
+// ---------------------------------------------------------------------------
+// scalars: reset, per-substep dt, end of step.  Inside a step they ride in
+// launches whose other blocks neither read nor write the same slots (a launch
+// of their own costs 4.5 us).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void scal_begin_flux(double* ds)
+{
+  ds[DS_NDT1] = kBIG;
+  ds[DS_NDT2] = kBIG;
+  ds[DS_NDT3] = kBIG;
+  ds[DS_ACCDT] = kBIG;
+}
+__device__ __forceinline__ void scal_begin_step(double* ds, unsigned long long* di)
+{
+  ds[DS_LASTNDT] = kBIG;
+  di[DI_NSTROKE] = 0;
+  di[DI_NFAIL] = 0;
+  di[DI_NFALLBACK] = 0;
+}
+// the substep's dt limit, then the slots ready for the next flux calculation
+__device__ __forceinline__ void scal_substep_dt(double* ds)
+{
+  const double wavedt = 1. / (1. / ds[DS_NDT1] + 1. / ds[DS_NDT2] + 1. / ds[DS_NDT3]);
+  const double nd = 1.0 * fmin(wavedt, ds[DS_ACCDT]);
+  if (nd < ds[DS_LASTNDT]) ds[DS_LASTNDT] = nd;
+  scal_begin_flux(ds);
+}
+__device__ __forceinline__ void scal_end_step(double* ds, unsigned long long* di, double safe)
+{
+  double fullndt = ds[DS_LASTNDT];
+  const double dt = ds[DS_DT];
+  if (fullndt > safe * dt) fullndt = safe * dt;
+  ds[DS_DTSTEP] = dt;
+  ds[DS_T] = ds[DS_T] + dt;
+  ds[DS_DT] = fullndt;
+  ds[DS_NSTEP] = ds[DS_NSTEP] + 1.0;
+  di[DI_NSTROKE_SUM] += di[DI_NSTROKE];
+  di[DI_NFAIL_SUM] += di[DI_NFAIL];
+  di[DI_NFALLBACK_SUM] += di[DI_NFALLBACK];
+}
+
+// Boundary flux sums through the inner and outer radial faces
+// (diag_flux_pureflux), deterministic: kFaccBlocks blocks each reduce a fixed
+// slice of the (j, k) faces in a fixed tree order into `part`, then one block
+// adds the partial sums in block order.
+constexpr int kFaccBlocks = 64;
+
+__device__ __forceinline__ void fluxacc_part_body(Dims d, const double* __restrict__ F1,
+                                                         double* __restrict__ part, const int blk)
+{
+  __shared__ double red[4][kBlock];
+  double s[4] = {0, 0, 0, 0};
+  const int nf = d.n2 * d.n3, chunk = (nf + kFaccBlocks - 1) / kFaccBlocks;
+  const int t0 = blk * chunk, t1 = min(nf, t0 + chunk);
+  const long nc = d.ncell;
+  for (int t = t0 + threadIdx.x; t < t1; t += kBlock) {
+    const int k = t / d.n2, j = t - k * d.n2;
+    const long oi = hd::cidx(d, 0, j, k), oo = hd::cidx(d, d.n1, j, k);
+    s[0] += F1[HARM_RHO * nc + oi];
+    s[1] += F1[HARM_UU * nc + oi];
+    s[2] += F1[HARM_RHO * nc + oo];
+    s[3] += F1[HARM_UU * nc + oo];
+  }
+  for (int c = 0; c < 4; c++) red[c][threadIdx.x] = s[c];
+  __syncthreads();
+  for (int w = kBlock / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w)
+      for (int c = 0; c < 4; c++) red[c][threadIdx.x] += red[c][threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x < 4) part[blk * 4 + threadIdx.x] = red[threadIdx.x][0];
+}
+
+__device__ __forceinline__ void fluxacc_final_body(const Params& P, const double* __restrict__ part,
+                                                   double* __restrict__ ds, double weight)
+{
+  const int c = threadIdx.x;
+  if (c >= 4) return;
+  double v = 0.0;
+  for (int b = 0; b < kFaccBlocks; b++) v += part[b * 4 + c];
+  ds[DS_FLUXACC + c] += v * P.dx[2] * P.dx[3] * ds[DS_DT] * weight;
+}
 
 // Toth EMFs at corners, each multiplied by the corner gdet (CORNGDETVERSION)
 __device__ __forceinline__ void emf_body(Dims d, int ni, int nj, int nk, const double* __restrict__ F1,
@@ -76,12 +158,22 @@ __device__ __forceinline__ void emf_body(Dims d, int ni, int nj, int nk, const d
   emf[2 * n + t] = e * gc3[pp];
 }
 
+// facc: the boundary flux sums' partials in kFaccBlocks more blocks (they read
+// F1's mass and energy only); di: clears the failed zones' count ahead of the
+// substep's inversion (either null: not)
 __global__ __launch_bounds__(kBlock) void k_emf(Dims d, int ni, int nj, int nk, const double* __restrict__ F1,
                                                 const double* __restrict__ F2, const double* __restrict__ F3,
                                                 const double* __restrict__ gf1, const double* __restrict__ gf2,
-                                                const double* __restrict__ gc3, double* __restrict__ emf)
+                                                const double* __restrict__ gc3, double* __restrict__ emf, int nemf,
+                                                double* __restrict__ facc, unsigned long long* __restrict__ di)
 {
-  emf_body(d, ni, nj, nk, F1, F2, F3, gf1, gf2, gc3, emf, xcd_tile(blockIdx.x, gridDim.x));
+  const int b = blockIdx.x;
+  if (b >= nemf) {
+    fluxacc_part_body(d, F1, facc, b - nemf);
+    return;
+  }
+  if (di && b == 0 && threadIdx.x == 0) di[DI_FIX] = 0;
+  emf_body(d, ni, nj, nk, F1, F2, F3, gf1, gf2, gc3, emf, xcd_tile(b, nemf));
 }
 
 // The three directions' B fluxes from the corner EMFs (fluxct.c:1106-1161)
@@ -147,10 +239,16 @@ __global__ __launch_bounds__(kBlock) void k_ct_all(Dims d, int ni, int nj, int n
 //              it).
 enum { kUpdAll = 0, kUpdFirst = 1, kUpdMiddle = 2, kUpdLast = 3 };
 
+// The modes inside a step take the field's fluxes from the corner EMFs (emf)
+// and write them to F1..F3 as ct_all_body does (the same expressions; the face
+// kernel's exact +0 stands for the own component), so that the CT needs no
+// launch and no trip of six fluxes through memory: 72 B a zone less; at
+// 256x128x64 the 22 us of the CT launch go and the update stays at 270-285 us.
 template <int DM, int MODE>
 __device__ __forceinline__ void update_body(Dims d, Params P, const double* __restrict__ pi,
-                                                   const double* __restrict__ pb, const double* __restrict__ F1,
-                                                   const double* __restrict__ F2, const double* __restrict__ F3,
+                                                   const double* __restrict__ pb, double* __restrict__ F1,
+                                                   double* __restrict__ F2, double* __restrict__ F3,
+                                                   const double* __restrict__ emf, int ni, int nj, int nk,
                                                    double* __restrict__ ui, double* __restrict__ uf,
                                                    double* __restrict__ ucum, const double* __restrict__ gcent,
                                                    const double* __restrict__ conn, double cuf0, double cuf1,
@@ -176,11 +274,61 @@ __device__ __forceinline__ void update_body(Dims d, Params P, const double* __re
     const double idx1 = 1.0 / P.dx[1], idx2 = 1.0 / P.dx[2], idx3 = 1.0 / P.dx[3];
     const long s2 = d.ps1, s3 = (long)d.ps1 * d.ns2;
     double dUt[HARM_NPR];
+    constexpr bool CT = MODE != kUpdAll;
+    const bool e1 = DM < 0 ? d.n1 > 1 : (DM & 1), e2 = DM < 0 ? d.n2 > 1 : (DM & 2) != 0,
+               e3 = DM < 0 ? d.n3 > 1 : (DM & 4) != 0;
+    if constexpr (CT) {
+      const int n = ni * nj * nk;
+      auto E = [&](int c, int a1, int a2, int a3) {
+        return emf[c * n + ((k + a3) * nj + j + a2) * ni + i + a1];
+      };
+      const int x = e1, y = e2, z = e3;  // the steps to the next corner
+      double g1[3] = {0.0, 0.0, 0.0}, g2[3] = {0.0, 0.0, 0.0}, g3[3] = {0.0, 0.0, 0.0};  // -(upper - lower) / dx
+      if (e1) {
+        const double l2 = 0.5 * (E(2, 0, 0, 0) + E(2, 0, y, 0)), l3 = -0.5 * (E(1, 0, 0, 0) + E(1, 0, 0, z));
+        const double u2 = 0.5 * (E(2, x, 0, 0) + E(2, x, y, 0)), u3 = -0.5 * (E(1, x, 0, 0) + E(1, x, 0, z));
+        F1[HARM_B2 * nc + o] = l2;
+        F1[HARM_B3 * nc + o] = l3;
+        if (i == d.n1 - 1) {
+          F1[HARM_B2 * nc + o + 1] = u2;
+          F1[HARM_B3 * nc + o + 1] = u3;
+        }
+        g1[0] = -0.0;
+        g1[1] = (-(u2 - l2) * idx1);
+        g1[2] = (-(u3 - l3) * idx1);
+      }
+      if (e2) {
+        const double l1 = -0.5 * (E(2, 0, 0, 0) + E(2, x, 0, 0)), l3 = 0.5 * (E(0, 0, 0, 0) + E(0, 0, 0, z));
+        const double u1 = -0.5 * (E(2, 0, y, 0) + E(2, x, y, 0)), u3 = 0.5 * (E(0, 0, y, 0) + E(0, 0, y, z));
+        F2[HARM_B1 * nc + o] = l1;
+        F2[HARM_B3 * nc + o] = l3;
+        if (j == d.n2 - 1) {
+          F2[HARM_B1 * nc + o + s2] = u1;
+          F2[HARM_B3 * nc + o + s2] = u3;
+        }
+        g2[0] = (-(u1 - l1) * idx2);
+        g2[1] = -0.0;
+        g2[2] = (-(u3 - l3) * idx2);
+      }
+      if (e3) {
+        const double l1 = 0.5 * (E(1, 0, 0, 0) + E(1, x, 0, 0)), l2 = -0.5 * (E(0, 0, 0, 0) + E(0, 0, y, 0));
+        const double u1 = 0.5 * (E(1, 0, 0, z) + E(1, x, 0, z)), u2 = -0.5 * (E(0, 0, 0, z) + E(0, 0, y, z));
+        F3[HARM_B1 * nc + o] = l1;
+        F3[HARM_B2 * nc + o] = l2;
+        if (k == d.n3 - 1) {
+          F3[HARM_B1 * nc + o + s3] = u1;
+          F3[HARM_B2 * nc + o + s3] = u2;
+        }
+        g3[0] = (-(u1 - l1) * idx3);
+        g3[1] = (-(u2 - l2) * idx3);
+        g3[2] = -0.0;
+      }
 #pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) {
+      for (int b = 0; b < 3; b++) dUt[HARM_B1 + b] = g1[b] + g2[b] + g3[b];
+    }
+#pragma unroll
+    for (int pl = 0; pl < (CT ? HARM_B1 : HARM_NPR); pl++) {
       double dU1 = 0, dU2 = 0, dU3 = 0;
-      const bool e1 = DM < 0 ? d.n1 > 1 : (DM & 1), e2 = DM < 0 ? d.n2 > 1 : (DM & 2) != 0,
-                 e3 = DM < 0 ? d.n3 > 1 : (DM & 4) != 0;
       if (e1) dU1 = (-(F1[pl * nc + o + 1] - F1[pl * nc + o]) * idx1);
       if (e2) dU2 = (-(F2[pl * nc + o + s2] - F2[pl * nc + o]) * idx2);
       if (e3) dU3 = (-(F3[pl * nc + o + s3] - F3[pl * nc + o]) * idx3);
@@ -234,8 +382,6 @@ __device__ __forceinline__ void update_body(Dims d, Params P, const double* __re
         dtsource[jj] = P.cour * (mydx[jj] / ag);
       }
       if (dtsource[0] < dts) dts = dtsource[0];
-      const bool e1 = DM < 0 ? d.n1 > 1 : (DM & 1), e2 = DM < 0 ? d.n2 > 1 : (DM & 2) != 0,
-                 e3 = DM < 0 ? d.n3 > 1 : (DM & 4) != 0;
       if (e1 && dtsource[1] < dts) dts = dtsource[1];
       if (e2 && dtsource[2] < dts) dts = dtsource[2];
       if (e3 && dtsource[3] < dts) dts = dtsource[3];
@@ -272,17 +418,25 @@ __device__ __forceinline__ void update_body(Dims d, Params P, const double* __re
   block_min_to(dts, ds + DS_ACCDT);
 }
 
+// facc (or null): one more block adds the boundary flux sums' partials
 template <int DM, int MODE>
 __global__ __launch_bounds__(kBlock) void k_update(Dims d, Params P, const double* __restrict__ pi,
-                                                   const double* __restrict__ pb, const double* __restrict__ F1,
-                                                   const double* __restrict__ F2, const double* __restrict__ F3,
+                                                   const double* __restrict__ pb, double* __restrict__ F1,
+                                                   double* __restrict__ F2, double* __restrict__ F3,
+                                                   const double* __restrict__ emf, int ni, int nj, int nk,
                                                    double* __restrict__ ui, double* __restrict__ uf,
                                                    double* __restrict__ ucum, const double* __restrict__ gcent,
                                                    const double* __restrict__ conn, double cuf0, double cuf1,
                                                    double cuf2, double cun0, double cun1, double cun2, int timeorder,
-                                                   double* __restrict__ ds)
+                                                   double* __restrict__ ds, const double* __restrict__ facc,
+                                                   double weight)
 {
-  update_body<DM, MODE>(d, P, pi, pb, F1, F2, F3, ui, uf, ucum, gcent, conn, cuf0, cuf1, cuf2, cun0, cun1, cun2, timeorder, ds, xcd_tile(blockIdx.x, gridDim.x));
+  const int nb = (int)gridDim.x - (facc ? 1 : 0);
+  if ((int)blockIdx.x >= nb) {
+    fluxacc_final_body(P, facc, ds, weight);
+    return;
+  }
+  update_body<DM, MODE>(d, P, pi, pb, F1, F2, F3, emf, ni, nj, nk, ui, uf, ucum, gcent, conn, cuf0, cuf1, cuf2, cun0, cun1, cun2, timeorder, ds, xcd_tile(blockIdx.x, nb));
 }
 
 // The grid inversion is two passes.  The solve pass (every substep) is
@@ -356,9 +510,15 @@ __device__ __forceinline__ void floors_body(Dims d, Params P, double* pf, int32_
 // four; 230 with the geometry and the primitives kept through the solve.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_invert(
     Dims d, Params P, const double* __restrict__ U, const double* __restrict__ pg, double* __restrict__ pf,
-    int32_t* __restrict__ pflag, const double* __restrict__ gcent, int finalstep, unsigned long long* __restrict__ di)
+    int32_t* __restrict__ pflag, const double* __restrict__ gcent, int finalstep, unsigned long long* __restrict__ di,
+    double* __restrict__ ds)
 {
-  invert_body(d, P, U, pg, pf, pflag, gcent, finalstep, di, xcd_tile(blockIdx.x, gridDim.x));
+  const int nb = (int)gridDim.x - (ds ? 1 : 0);  // ds (or null): one more block forms the substep's dt
+  if ((int)blockIdx.x >= nb) {
+    if (threadIdx.x == 0) scal_substep_dt(ds);
+    return;
+  }
+  invert_body(d, P, U, pg, pf, pflag, gcent, finalstep, di, xcd_tile(blockIdx.x, nb));
 }
 
 template <bool DIAG>
@@ -1101,15 +1261,18 @@ __device__ __forceinline__ void bounds_flags(const Dims& d, int bc, int32_t* __r
 }
 
 // cond: the second pass, only where failure averaging changed zones and
-// without the flags (a batch counts their blocks for both passes).  FIX2D (2-D grids, flags
+// without the flags (a batch counts their blocks for both passes).  ds_end
+// (or null): the step's last launch, which also ends the step.  FIX2D (2-D grids, flags
 // bounded in the same launch): the block that ends last goes on with failure
 // averaging and the second pass when there are failed zones; they are few, so
 // one block is enough.  Its zones come from every block, hence the fences.
 template <bool FIX2D>
 __device__ __forceinline__ void bounds_body(const Dims& d, const Params& P, double* p, const double* gcent,
                                             const double* rcent, int32_t* pflag, double* pfix,
-                                            unsigned long long* di, int finalstep, bool flags, bool cond, int blk)
+                                            unsigned long long* di, int finalstep, bool flags, bool cond, int blk,
+                                            double* ds_end)
 {
+  if (ds_end && blk == 0 && threadIdx.x == 0) scal_end_step(ds_end, di, P.safe);
   const bool fix = (FIX2D || cond) && di[DI_FIX] != 0;
   if (cond && !fix) return;
   const BoundPlan b = bound_plan(d, flags);
@@ -1141,95 +1304,27 @@ __device__ __forceinline__ void bounds_body(const Dims& d, const Params& P, doub
 template <bool FIX2D>
 __global__ __launch_bounds__(kBlock) void k_bounds(Dims d, Params P, double* p, const double* gcent,
                                                    const double* rcent, int32_t* pflag, double* pfix,
-                                                   unsigned long long* di, int finalstep, int flags, int cond)
+                                                   unsigned long long* di, int finalstep, int flags, int cond,
+                                                   double* ds_end)
 {
-  bounds_body<FIX2D>(d, P, p, gcent, rcent, pflag, pfix, di, finalstep, flags, cond, blockIdx.x);
+  bounds_body<FIX2D>(d, P, p, gcent, rcent, pflag, pfix, di, finalstep, flags, cond, blockIdx.x, ds_end);
 }
 
 // ---------------------------------------------------------------------------
-// scalars: reset, per-substep dt, end of step
+// scalars on their own: outside a step and for grids without the merged passes
 // ---------------------------------------------------------------------------
 __global__ void k_scal_begin_flux(double* ds, unsigned long long* di)
 {
   di[DI_FIX] = 0;
-  ds[DS_NDT1] = kBIG;
-  ds[DS_NDT2] = kBIG;
-  ds[DS_NDT3] = kBIG;
-  ds[DS_ACCDT] = kBIG;
+  scal_begin_flux(ds);
 }
 __global__ void k_scal_begin_step(double* ds, unsigned long long* di)
 {
-  ds[DS_LASTNDT] = kBIG;
-  di[DI_NSTROKE] = 0;
-  di[DI_NFAIL] = 0;
-  di[DI_NFALLBACK] = 0;
+  scal_begin_step(ds, di);
+  scal_begin_flux(ds);
 }
-__global__ void k_scal_substep_dt(double* ds)
-{
-  const double wavedt = 1. / (1. / ds[DS_NDT1] + 1. / ds[DS_NDT2] + 1. / ds[DS_NDT3]);
-  const double nd = 1.0 * fmin(wavedt, ds[DS_ACCDT]);
-  if (nd < ds[DS_LASTNDT]) ds[DS_LASTNDT] = nd;
-}
-__global__ void k_scal_end_step(double* ds, unsigned long long* di, double safe)
-{
-  double fullndt = ds[DS_LASTNDT];
-  const double dt = ds[DS_DT];
-  if (fullndt > safe * dt) fullndt = safe * dt;
-  ds[DS_DTSTEP] = dt;
-  ds[DS_T] = ds[DS_T] + dt;
-  ds[DS_DT] = fullndt;
-  ds[DS_NSTEP] = ds[DS_NSTEP] + 1.0;
-  di[DI_NSTROKE_SUM] += di[DI_NSTROKE];
-  di[DI_NFAIL_SUM] += di[DI_NFAIL];
-  di[DI_NFALLBACK_SUM] += di[DI_NFALLBACK];
-}
-
-// Boundary flux sums through the inner and outer radial faces
-// (diag_flux_pureflux), deterministic: kFaccBlocks blocks each reduce a fixed
-// slice of the (j, k) faces in a fixed tree order into `part`, then one block
-// adds the partial sums in block order.
-constexpr int kFaccBlocks = 64;
-
-__device__ __forceinline__ void fluxacc_part_body(Dims d, const double* __restrict__ F1,
-                                                         double* __restrict__ part, const int blk)
-{
-  __shared__ double red[4][kBlock];
-  double s[4] = {0, 0, 0, 0};
-  const int nf = d.n2 * d.n3, chunk = (nf + kFaccBlocks - 1) / kFaccBlocks;
-  const int t0 = blk * chunk, t1 = min(nf, t0 + chunk);
-  const long nc = d.ncell;
-  for (int t = t0 + threadIdx.x; t < t1; t += kBlock) {
-    const int k = t / d.n2, j = t - k * d.n2;
-    const long oi = hd::cidx(d, 0, j, k), oo = hd::cidx(d, d.n1, j, k);
-    s[0] += F1[HARM_RHO * nc + oi];
-    s[1] += F1[HARM_UU * nc + oi];
-    s[2] += F1[HARM_RHO * nc + oo];
-    s[3] += F1[HARM_UU * nc + oo];
-  }
-  for (int c = 0; c < 4; c++) red[c][threadIdx.x] = s[c];
-  __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w)
-      for (int c = 0; c < 4; c++) red[c][threadIdx.x] += red[c][threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x < 4) part[blk * 4 + threadIdx.x] = red[threadIdx.x][0];
-}
-
-__global__ __launch_bounds__(kBlock) void k_fluxacc_part(Dims d, const double* __restrict__ F1,
-                                                         double* __restrict__ part)
-{
-  fluxacc_part_body(d, F1, part, blockIdx.x);
-}
-
-__global__ void k_fluxacc_final(Params P, const double* __restrict__ part, double* __restrict__ ds, double weight)
-{
-  const int c = threadIdx.x;
-  if (c >= 4) return;
-  double v = 0.0;
-  for (int b = 0; b < kFaccBlocks; b++) v += part[b * 4 + c];
-  ds[DS_FLUXACC + c] += v * P.dx[2] * P.dx[3] * ds[DS_DT] * weight;
-}
+__global__ void k_scal_substep_dt(double* ds) { scal_substep_dt(ds); }
+__global__ void k_scal_end_step(double* ds, unsigned long long* di, double safe) { scal_end_step(ds, di, safe); }
 
 inline unsigned nblocks(long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
@@ -1506,12 +1601,16 @@ FaceTile plan_face_tile(const Dims& d, int dir, int td_force = 0)
 double* wl_dir(harm_handle* h, int dir) { return h->wl + (size_t)(dir - 1) * HARM_NPR * h->d.ncell; }
 double* wr_dir(harm_handle* h, int dir) { return h->wr + (size_t)(dir - 1) * HARM_NPR * h->d.ncell; }
 
-harm_status enq_fluxcalc(harm_handle* h, int which_p, int do_ct)
+// in_step: the dt slots are ready, the EMFs' launch also forms the boundary flux
+// partials (facc) and clears the failed zones' count, and the update applies the
+// CT; ct: write the field fluxes here all the same (for readers ahead of it)
+harm_status enq_fluxcalc(harm_handle* h, int which_p, int do_ct, bool in_step = false, bool facc = false,
+                         bool ct = true)
 {
   const Dims& d = h->d;
   hipStream_t s = h->stream;
   const double* pb = h->arr[which_p];
-  hipLaunchKernelGGL(k_scal_begin_flux, dim3(1), dim3(1), 0, s, h->ds, h->di);
+  if (!in_step) hipLaunchKernelGGL(k_scal_begin_flux, dim3(1), dim3(1), 0, s, h->ds, h->di);
   const int recon = h->cfg.recon, ft = h->cfg.flux;
   const bool weno = recon == HARM_RECON_WENO5;
   if (weno) {
@@ -1548,9 +1647,14 @@ harm_status enq_fluxcalc(harm_handle* h, int which_p, int do_ct)
     prof_end(h, HARM_K_FLUX1 + DIR - 1);                                                                    \
     if (fork && DIR > 1) HH_HIP(hipEventRecord(h->evjoin[DIR - 2], sd));                                    \
   } while (0)
-  if (d.n1 > 1) LAUNCH_FLUX(1, h->arr[HARM_ARR_F1], h->geom[HARM_LOC_FACE1]);
-  if (d.n2 > 1) LAUNCH_FLUX(2, h->arr[HARM_ARR_F2], h->geom[HARM_LOC_FACE2]);
-  if (d.n3 > 1) LAUNCH_FLUX(3, h->arr[HARM_ARR_F3], h->geom[HARM_LOC_FACE3]);
+  if (!weno && !h->prof && d.n1 * (long)d.n2 * d.n3 > 1) {
+    launch_flux_all(recon, &h->ft[1], s, d, pb, &h->arr[HARM_ARR_F1], &h->geom[HARM_LOC_FACE1], h->P, ft, do_ct,
+                    h->ds);
+  } else {  // timed one by one when profiling
+    if (d.n1 > 1) LAUNCH_FLUX(1, h->arr[HARM_ARR_F1], h->geom[HARM_LOC_FACE1]);
+    if (d.n2 > 1) LAUNCH_FLUX(2, h->arr[HARM_ARR_F2], h->geom[HARM_LOC_FACE2]);
+    if (d.n3 > 1) LAUNCH_FLUX(3, h->arr[HARM_ARR_F3], h->geom[HARM_LOC_FACE3]);
+  }
 #undef LAUNCH_FLUX
   if (fork) {
     if (d.n2 > 1) HH_HIP(hipStreamWaitEvent(s, h->evjoin[0], 0));
@@ -1560,12 +1664,15 @@ harm_status enq_fluxcalc(harm_handle* h, int which_p, int do_ct)
   if (do_ct) {
     prof_begin(h);
     const int ni = h->emf_ni, nj = h->emf_nj, nk = h->emf_nk;
-    hipLaunchKernelGGL(k_emf, dim3(nblocks((long)ni * nj * nk)), dim3(kBlock), 0, s, d, ni, nj, nk,
+    const unsigned nemf = nblocks((long)ni * nj * nk);
+    hipLaunchKernelGGL(k_emf, dim3(nemf + (facc ? kFaccBlocks : 0)), dim3(kBlock), 0, s, d, ni, nj, nk,
                        h->arr[HARM_ARR_F1], h->arr[HARM_ARR_F2], h->arr[HARM_ARR_F3], h->geom[HARM_LOC_FACE1],
-                       h->geom[HARM_LOC_FACE2], h->gcorn3, h->emf);
+                       h->geom[HARM_LOC_FACE2], h->gcorn3, h->emf, (int)nemf, facc ? h->facc : nullptr,
+                       in_step ? h->di : nullptr);
     const long nct = (long)(d.n1 + (d.n1 > 1)) * (d.n2 + (d.n2 > 1)) * (d.n3 + (d.n3 > 1));
-    hipLaunchKernelGGL(k_ct_all, dim3(nblocks(nct)), dim3(kBlock), 0, s, d, ni, nj, nk, h->emf,
-                       h->arr[HARM_ARR_F1], h->arr[HARM_ARR_F2], h->arr[HARM_ARR_F3]);
+    if (ct)
+      hipLaunchKernelGGL(k_ct_all, dim3(nblocks(nct)), dim3(kBlock), 0, s, d, ni, nj, nk, h->emf,
+                         h->arr[HARM_ARR_F1], h->arr[HARM_ARR_F2], h->arr[HARM_ARR_F3]);
     prof_end(h, HARM_K_EMFCT);
     HH_TRY(hh::check_launch("k_emf/k_ct_all"));
   }
@@ -1573,17 +1680,18 @@ harm_status enq_fluxcalc(harm_handle* h, int which_p, int do_ct)
 }
 
 harm_status enq_update(harm_handle* h, int which_pi, int which_pb, const double* CUf, const double* Cunew,
-                       int timeorder, int mode)
+                       int timeorder, int mode, bool facc = false, double weight = 0.0)
 {
   const Dims& d = h->d;
   prof_begin(h);
   const int dm = (d.n1 > 1) | ((d.n2 > 1) << 1) | ((d.n3 > 1) << 2);
 #define LAUNCH_UPDATE(DM, MODE)                                                                                     \
-  hipLaunchKernelGGL((k_update<DM, MODE>), dim3(nblocks((long)d.n1 * d.n2 * d.n3)), dim3(kBlock), 0, h->stream, d, \
-                     h->P, h->arr[which_pi], h->arr[which_pb], h->arr[HARM_ARR_F1], h->arr[HARM_ARR_F2],           \
-                     h->arr[HARM_ARR_F3], h->arr[HARM_ARR_UI], h->arr[HARM_ARR_UF], h->arr[HARM_ARR_UCUM],          \
-                     h->geom[HARM_LOC_CENT], h->conn, CUf[0], CUf[1], CUf[2], Cunew[0], Cunew[1], Cunew[2],         \
-                     timeorder, h->ds)
+  hipLaunchKernelGGL((k_update<DM, MODE>), dim3(nblocks((long)d.n1 * d.n2 * d.n3) + (facc ? 1 : 0)), dim3(kBlock), \
+                     0, h->stream, d, h->P, h->arr[which_pi], h->arr[which_pb], h->arr[HARM_ARR_F1],                \
+                     h->arr[HARM_ARR_F2], h->arr[HARM_ARR_F3], h->emf, h->emf_ni, h->emf_nj, h->emf_nk,             \
+                     h->arr[HARM_ARR_UI], h->arr[HARM_ARR_UF], h->arr[HARM_ARR_UCUM], h->geom[HARM_LOC_CENT],       \
+                     h->conn, CUf[0], CUf[1], CUf[2], Cunew[0], Cunew[1], Cunew[2], timeorder, h->ds,               \
+                     facc ? h->facc : nullptr, weight)
 #define LAUNCH_UPDATE_MODES(DM)                         \
   switch (mode) {                                       \
     case kUpdFirst: LAUNCH_UPDATE(DM, kUpdFirst); break;   \
@@ -1605,7 +1713,9 @@ harm_status enq_update(harm_handle* h, int which_pi, int which_pb, const double*
 // guess from pb and writes every active zone of pf, and the boundary pass that
 // follows rewrites every ghost zone of pf before anything reads it.
 // ener: the final substep's floor and gamma-limit changes go to their fladdterms
-harm_status enq_invert(harm_handle* h, int which_pb, int which_pf, int finalstep, bool copy_all, bool ener = false)
+// substep_dt: form the substep's dt limit beside it
+harm_status enq_invert(harm_handle* h, int which_pb, int which_pf, int finalstep, bool copy_all, bool ener = false,
+                       bool substep_dt = false)
 {
   const Dims& d = h->d;
   const size_t bytes = sizeof(double) * HARM_NPR * d.ncell;
@@ -1619,9 +1729,11 @@ harm_status enq_invert(harm_handle* h, int which_pb, int which_pf, int finalstep
     HH_TRY(launch_invert_grid_mlp(h->guess, d, h->P, U, h->arr[which_pb], h->arr[which_pf], h->pflag,
                                   h->geom[HARM_LOC_CENT], h->floors, finalstep, h->di, h->stream,
                                   diag ? h->fx_p0 : nullptr, h->fx_pfl, h->fx_flag));
+    if (substep_dt) hipLaunchKernelGGL(k_scal_substep_dt, dim3(1), dim3(1), 0, h->stream, h->ds);
   } else {
-    hipLaunchKernelGGL(k_invert, dim3(nb), dim3(kBlock), 0, h->stream, d, h->P, U, h->arr[which_pb],
-                       h->arr[which_pf], h->pflag, h->geom[HARM_LOC_CENT], finalstep, h->di);
+    hipLaunchKernelGGL(k_invert, dim3(nb + (substep_dt ? 1 : 0)), dim3(kBlock), 0, h->stream, d, h->P, U,
+                       h->arr[which_pb], h->arr[which_pf], h->pflag, h->geom[HARM_LOC_CENT], finalstep, h->di,
+                       substep_dt ? h->ds : nullptr);
     if (finalstep && diag)
       hipLaunchKernelGGL(k_floors<true>, dim3(nb), dim3(kBlock), 0, h->stream, d, h->P, h->arr[which_pf], h->pflag,
                          h->geom[HARM_LOC_CENT], h->floors, h->di, h->fx_p0, h->fx_pfl, h->fx_flag);
@@ -1637,8 +1749,8 @@ harm_status enq_invert(harm_handle* h, int which_pb, int which_pf, int finalstep
 }
 
 // flags: bound the flags in the same launch; cond: only where the substep's
-// inversion left failed zones (bounds_merge grids)
-harm_status enq_bound(harm_handle* h, int which, bool flags = false, bool cond = false)
+// inversion left failed zones; end: the step's last launch (bounds_merge grids)
+harm_status enq_bound(harm_handle* h, int which, bool flags = false, bool cond = false, bool end = false)
 {
   const Dims& d = h->d;
   hipStream_t s = h->stream;
@@ -1646,7 +1758,8 @@ harm_status enq_bound(harm_handle* h, int which, bool flags = false, bool cond =
   prof_begin(h);
   if (bounds_merge(d)) {
     hipLaunchKernelGGL(k_bounds<false>, dim3((unsigned)bound_plan(d, flags).total()), dim3(kBlock), 0, s, d, h->P, p,
-                       h->geom[HARM_LOC_CENT], h->rcent, h->pflag, nullptr, h->di, 0, flags, cond);
+                       h->geom[HARM_LOC_CENT], h->rcent, h->pflag, nullptr, h->di, 0, flags, cond,
+                       end ? h->ds : nullptr);
     prof_end(h, HARM_K_BOUND);
     return hh::check_launch("k_bounds");
   }
@@ -1706,7 +1819,8 @@ harm_status enq_post_fixup(harm_handle* h, int which, int finalstep, bool ener =
 // 2-D grids one launch, on 3-D ones four of which the last three have nothing
 // to do unless a zone failed; grids that bounds_merge leaves out take every
 // pass in full.
-harm_status enq_finish(harm_handle* h, int which, int finalstep, bool ener)
+// end: the substep ends a whole step.
+harm_status enq_finish(harm_handle* h, int which, int finalstep, bool ener, bool end)
 {
   const Dims& d = h->d;
   const bool merge = bounds_merge(d);
@@ -1714,13 +1828,15 @@ harm_status enq_finish(harm_handle* h, int which, int finalstep, bool ener)
     prof_begin(h);
     hipLaunchKernelGGL(k_bounds<true>, dim3((unsigned)bound_plan(d, true).total()), dim3(kBlock), 0, h->stream, d,
                        h->P, h->arr[which], h->geom[HARM_LOC_CENT], h->rcent, h->pflag, h->pfix, h->di, finalstep, 1,
-                       0);
+                       0, end ? h->ds : nullptr);
     prof_end(h, HARM_K_BOUND);
     return hh::check_launch("k_bounds");
   }
   HH_TRY(enq_bound(h, which, merge));
   HH_TRY(enq_post_fixup(h, which, finalstep, ener, merge));
-  return enq_bound(h, which, false, merge);
+  HH_TRY(enq_bound(h, which, false, merge, end));
+  if (end && !merge) hipLaunchKernelGGL(k_scal_end_step, dim3(1), dim3(1), 0, h->stream, h->ds, h->di, h->P.safe);
+  return HARM_OK;
 }
 
 int rk_tables(int timeorder, double CUf[4][4], double Cunew[4][4])
@@ -1761,15 +1877,7 @@ harm_status enq_substep(harm_handle* h, int to, int nto, const double CUf[4][4],
       launch_ener_source(h->d, h->P, h->arr[pbb[to]], h->geom[HARM_LOC_CENT], h->conn, h->enpart, h->en,
                          h->stream);
   }
-  HH_TRY(enq_fluxcalc(h, pbb[to], 1));
-  if (ener)
-    launch_ener_pdot(h->d, h->P, h->arr[HARM_ARR_F1], h->arr[HARM_ARR_F2], h->arr[HARM_ARR_F3], h->enpart, h->en,
-                     h->ds, wflux[to], h->stream);
-  if (diag && h->d.n1 > 1) {
-    hipLaunchKernelGGL(k_fluxacc_part, dim3(kFaccBlocks), dim3(kBlock), 0, h->stream, h->d, h->arr[HARM_ARR_F1],
-                       h->facc);
-    hipLaunchKernelGGL(k_fluxacc_final, dim3(1), dim3(64), 0, h->stream, h->P, h->facc, h->ds, wflux[to]);
-  }
+  const bool facc = diag && h->d.n1 > 1;
   // The reduced-traffic modes rely on the tables keeping ucum at zero until
   // the last substep (true of the RK2 and RK3 tables); otherwise run the
   // reference loop as is.
@@ -1777,10 +1885,14 @@ harm_status enq_substep(harm_handle* h, int to, int nto, const double CUf[4][4],
   for (int s = 0; s + 1 < nto; s++)
     zero_ucum = zero_ucum && Cunew[s][0] == 0.0 && Cunew[s][1] == 0.0 && Cunew[s][2] == 0.0;
   const int mode = !zero_ucum ? kUpdAll : to == 0 ? kUpdFirst : finalstep ? kUpdLast : kUpdMiddle;
-  HH_TRY(enq_update(h, pii[to], pbb[to], CUf[to], Cunew[to], to, mode));
-  HH_TRY(enq_invert(h, pbb[to], pff[to], finalstep, false, ener));
-  hipLaunchKernelGGL(k_scal_substep_dt, dim3(1), dim3(1), 0, h->stream, h->ds);
-  HH_TRY(enq_finish(h, pff[to], finalstep, ener && finalstep));
+  // the update of a step forms the field fluxes itself; the energy sums read them ahead of it
+  HH_TRY(enq_fluxcalc(h, pbb[to], 1, in_step, facc, mode == kUpdAll || ener));
+  if (ener)
+    launch_ener_pdot(h->d, h->P, h->arr[HARM_ARR_F1], h->arr[HARM_ARR_F2], h->arr[HARM_ARR_F3], h->enpart, h->en,
+                     h->ds, wflux[to], h->stream);
+  HH_TRY(enq_update(h, pii[to], pbb[to], CUf[to], Cunew[to], to, mode, facc, wflux[to]));
+  HH_TRY(enq_invert(h, pbb[to], pff[to], finalstep, false, ener, true));
+  HH_TRY(enq_finish(h, pff[to], finalstep, ener && finalstep, in_step && finalstep));
   return hh::check_launch("substep");
 }
 
@@ -1831,9 +1943,19 @@ __device__ __forceinline__ void batch_decode(const int* __restrict__ pre, int ng
   batch_decode(pre, ng, (REMAP) ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x, gi, lb); \
   const GridRef& g = G[gi];
 
-__global__ __launch_bounds__(kBlock) void kb_emf(const GridRef* __restrict__ G, const int* __restrict__ pre, int ng)
+// EMFs of every grid (n blocks), then their boundary flux partials (pref)
+__global__ __launch_bounds__(kBlock) void kb_emf(const GridRef* __restrict__ G, const int* __restrict__ pre,
+                                                 const int* __restrict__ pref, int n, int ng)
 {
-  BATCH_DECODE(true)
+  int gi, lb;
+  if ((int)blockIdx.x >= n) {
+    batch_decode(pref, ng, blockIdx.x - n, gi, lb);
+    fluxacc_part_body(G[gi].d, gmem(G[gi].arr[HARM_ARR_F1]), gmem(G[gi].facc), lb);
+    return;
+  }
+  batch_decode(pre, ng, xcd_tile(blockIdx.x, n), gi, lb);
+  const GridRef& g = G[gi];
+  if (lb == 0 && threadIdx.x == 0) gmem(g.di)[DI_FIX] = 0;
   emf_body(g.d, g.emf_ni, g.emf_nj, g.emf_nk, gmem(g.arr[HARM_ARR_F1]), gmem(g.arr[HARM_ARR_F2]), gmem(g.arr[HARM_ARR_F3]),
            gmem(g.geom[HARM_LOC_FACE1]), gmem(g.geom[HARM_LOC_FACE2]), gmem(g.gcorn3), gmem(g.emf), lb);
 }
@@ -1846,40 +1968,41 @@ __global__ __launch_bounds__(kBlock) void kb_ct_all(const GridRef* __restrict__ 
               gmem(g.arr[HARM_ARR_F3]), lb);
 }
 
-__global__ __launch_bounds__(kBlock) void kb_fluxacc_part(const GridRef* __restrict__ G, const int* __restrict__ pre,
-                                                          int ng)
-{
-  BATCH_DECODE(false)
-  fluxacc_part_body(g.d, gmem(g.arr[HARM_ARR_F1]), gmem(g.facc), lb);
-}
-
-__global__ void kb_fluxacc_final(const GridRef* __restrict__ G, double weight)
-{
-  const GridRef& g = G[blockIdx.x];
-  const int c = threadIdx.x;
-  if (c >= 4 || g.d.n1 < 2) return;
-  double v = 0.0;
-  for (int b = 0; b < kFaccBlocks; b++) v += gmem(g.facc)[b * 4 + c];
-  gmem(g.ds)[DS_FLUXACC + c] += v * g.P.dx[2] * g.P.dx[3] * gmem(g.ds)[DS_DT] * weight;
-}
-
-
+// update of every grid (n blocks), then one block a grid for its boundary flux sums
 template <int DM, int MODE>
 __global__ __launch_bounds__(kBlock) void kb_update(const GridRef* __restrict__ G, const int* __restrict__ pre, int ng,
-                                                    int which_pi, int which_pb, double cuf0, double cuf1, double cuf2,
-                                                    double cun0, double cun1, double cun2, int timeorder)
+                                                    int n, int which_pi, int which_pb, double cuf0, double cuf1,
+                                                    double cuf2, double cun0, double cun1, double cun2, int timeorder,
+                                                    double weight)
 {
-  BATCH_DECODE(true)
+  if ((int)blockIdx.x >= n) {
+    const GridRef& g = G[blockIdx.x - n];
+    if (g.d.n1 > 1) fluxacc_final_body(g.P, gmem(g.facc), gmem(g.ds), weight);
+    return;
+  }
+  int gi, lb;
+  batch_decode(pre, ng, xcd_tile(blockIdx.x, n), gi, lb);
+  const GridRef& g = G[gi];
   update_body<DM, MODE>(g.d, g.P, gmem(g.arr[which_pi]), gmem(g.arr[which_pb]), gmem(g.arr[HARM_ARR_F1]),
-                        gmem(g.arr[HARM_ARR_F2]), gmem(g.arr[HARM_ARR_F3]), gmem(g.arr[HARM_ARR_UI]),
-                        gmem(g.arr[HARM_ARR_UF]), gmem(g.arr[HARM_ARR_UCUM]), gmem(g.geom[HARM_LOC_CENT]),
-                        gmem(g.conn), cuf0, cuf1, cuf2, cun0, cun1, cun2, timeorder, gmem(g.ds), lb);
+                        gmem(g.arr[HARM_ARR_F2]), gmem(g.arr[HARM_ARR_F3]), gmem(g.emf), g.emf_ni, g.emf_nj, g.emf_nk,
+                        gmem(g.arr[HARM_ARR_UI]), gmem(g.arr[HARM_ARR_UF]), gmem(g.arr[HARM_ARR_UCUM]),
+                        gmem(g.geom[HARM_LOC_CENT]), gmem(g.conn), cuf0, cuf1, cuf2, cun0, cun1, cun2, timeorder,
+                        gmem(g.ds), lb);
 }
 
+// inversion of every grid (n blocks), then the grids' substep dt, a thread each
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void kb_invert(
-    const GridRef* __restrict__ G, const int* __restrict__ pre, int ng, int which_pb, int which_pf, int finalstep)
+    const GridRef* __restrict__ G, const int* __restrict__ pre, int ng, int n, int which_pb, int which_pf,
+    int finalstep)
 {
-  BATCH_DECODE(true)
+  if ((int)blockIdx.x >= n) {
+    const int q = ((int)blockIdx.x - n) * kBlock + threadIdx.x;
+    if (q < ng) scal_substep_dt(G[q].ds);
+    return;
+  }
+  int gi, lb;
+  batch_decode(pre, ng, xcd_tile(blockIdx.x, n), gi, lb);
+  const GridRef& g = G[gi];
   invert_body(g.d, g.P, gmem(g.arr[finalstep ? HARM_ARR_UCUM : HARM_ARR_UF]), gmem(g.arr[which_pb]),
               gmem(g.arr[which_pf]), gmem(g.pflag), gmem(g.geom[HARM_LOC_CENT]), finalstep, gmem(g.di), lb);
 }
@@ -1921,11 +2044,11 @@ __global__ __launch_bounds__(kBlock) void kb_fixup_apply(const GridRef* __restri
 // every grid's boundary pass (bounds_body); pre: block counts with the flags'
 template <bool FIX2D>
 __global__ __launch_bounds__(kBlock) void kb_bounds(const GridRef* __restrict__ G, const int* __restrict__ pre, int ng,
-                                                    int which, int finalstep, int cond)
+                                                    int which, int finalstep, int cond, int end)
 {
   BATCH_DECODE(false)
   bounds_body<FIX2D>(g.d, g.P, gmem(g.arr[which]), gmem(g.geom[HARM_LOC_CENT]), gmem(g.rcent), gmem(g.pflag),
-                     gmem(g.pfix), gmem(g.di), finalstep, true, cond, lb);
+                     gmem(g.pfix), gmem(g.di), finalstep, true, cond, lb, end ? gmem(g.ds) : nullptr);
 }
 
 __global__ __launch_bounds__(kBlock) void kb_bound_x1(const GridRef* __restrict__ G, const int* __restrict__ pre,
@@ -1963,37 +2086,16 @@ __global__ __launch_bounds__(kBlock) void kb_bound_x3(const GridRef* __restrict_
   bound_x3_body(g.d, gmem(g.arr[which]), lb);
 }
 
-// one thread per grid
+// a step's begin (0) or end (1), one thread per grid
 __global__ void kb_scal(const GridRef* __restrict__ G, int ng, int what)
 {
   const int gi = blockIdx.x * blockDim.x + threadIdx.x;
   if (gi >= ng) return;
-  double* ds = G[gi].ds;
-  if (what == 0) {  // begin flux
-    ds[DS_NDT1] = kBIG; ds[DS_NDT2] = kBIG; ds[DS_NDT3] = kBIG; ds[DS_ACCDT] = kBIG;
-    G[gi].di[DI_FIX] = 0;
-  } else if (what == 1) {  // begin step
-    ds[DS_LASTNDT] = kBIG;
-    G[gi].di[DI_NSTROKE] = 0;
-    G[gi].di[DI_NFAIL] = 0;
-    G[gi].di[DI_NFALLBACK] = 0;
-  } else if (what == 2) {  // substep dt
-    const double wavedt = 1. / (1. / ds[DS_NDT1] + 1. / ds[DS_NDT2] + 1. / ds[DS_NDT3]);
-    const double nd = 1.0 * fmin(wavedt, ds[DS_ACCDT]);
-    if (nd < ds[DS_LASTNDT]) ds[DS_LASTNDT] = nd;
-  } else {  // end step
-    const double safe = G[gi].P.safe;
-    double fullndt = ds[DS_LASTNDT];
-    const double dt = ds[DS_DT];
-    if (fullndt > safe * dt) fullndt = safe * dt;
-    ds[DS_DTSTEP] = dt;
-    ds[DS_T] = ds[DS_T] + dt;
-    ds[DS_DT] = fullndt;
-    ds[DS_NSTEP] = ds[DS_NSTEP] + 1.0;
-    unsigned long long* di = G[gi].di;
-    di[DI_NSTROKE_SUM] += di[DI_NSTROKE];
-    di[DI_NFAIL_SUM] += di[DI_NFAIL];
-    di[DI_NFALLBACK_SUM] += di[DI_NFALLBACK];
+  if (what == 0) {
+    scal_begin_step(G[gi].ds, G[gi].di);
+    scal_begin_flux(G[gi].ds);
+  } else {
+    scal_end_step(G[gi].ds, G[gi].di, G[gi].P.safe);
   }
 }
 
@@ -2096,43 +2198,34 @@ harm_status enq_batch_substep(harm_batch* b, int to, int nto, const double CUf[4
   int pff[3] = {HARM_ARR_PK0, HARM_ARR_PK1, HARM_ARR_P};
   if (nto == 2) { pbb[1] = HARM_ARR_PK0; pff[1] = HARM_ARR_P; }
   const int finalstep = (to == nto - 1);
-  const unsigned g1 = (unsigned)((ng + 63) / 64);
-  hipLaunchKernelGGL(kb_scal, dim3(g1), dim3(64), 0, s, G, ng, 0);
   // fluxes
   // WENO5BND: every grid's lines of a direction are reconstructed (one
-  // launch per grid) before the batched face kernel of that direction
+  // launch per grid) before the batched face kernels
   const bool weno = b->recon == HARM_RECON_WENO5;
   if (weno)
-    for (harm_handle* h : b->grids) launch_weno_dp(h->d, s, h->arr[pbb[to]], h->geom[HARM_LOC_CENT], h->P, h->wtm, h->wdp);
-#define BFLUX(DIR)                                                                                         \
-  if (b->ntot[BS_FLUX1 + DIR - 1] > 0) {                                                                    \
-    if (weno)                                                                                               \
-      for (harm_handle* h : b->grids)                                                                       \
-        if (h->ft[DIR].nblk > 0 && (DIR == 1 ? h->d.n1 : DIR == 2 ? h->d.n2 : h->d.n3) > 1)                 \
-          launch_weno_recon(DIR, h->d, h->ft[DIR].b, s, h->arr[pbb[to]], h->wdp, wl_dir(h, DIR), wr_dir(h, DIR)); \
-    launch_flux_batch(DIR, b->recon, (unsigned)b->ntot[BS_FLUX1 + DIR - 1], s, G, P(BS_FLUX1 + DIR - 1), ng, \
-                      pbb[to], 1);                                                                          \
-  }
-  BFLUX(1)
-  BFLUX(2)
-  BFLUX(3)
-#undef BFLUX
-  hipLaunchKernelGGL(kb_emf, dim3((unsigned)b->ntot[BS_EMF]), blk, 0, s, G, P(BS_EMF), ng);
-  if (b->ntot[BS_CT]) hipLaunchKernelGGL(kb_ct_all, dim3((unsigned)b->ntot[BS_CT]), blk, 0, s, G, P(BS_CT), ng);
-  if (b->ntot[BS_FACC]) {
-    hipLaunchKernelGGL(kb_fluxacc_part, dim3((unsigned)b->ntot[BS_FACC]), blk, 0, s, G, P(BS_FACC), ng);
-    hipLaunchKernelGGL(kb_fluxacc_final, dim3((unsigned)ng), dim3(64), 0, s, G, wflux[to]);
-  }
+    for (harm_handle* h : b->grids) {
+      launch_weno_dp(h->d, s, h->arr[pbb[to]], h->geom[HARM_LOC_CENT], h->P, h->wtm, h->wdp);
+      for (int dir = 1; dir <= 3; dir++)
+        if ((dir == 1 ? h->d.n1 : dir == 2 ? h->d.n2 : h->d.n3) > 1)
+          launch_weno_recon(dir, h->d, h->ft[dir].b, s, h->arr[pbb[to]], h->wdp, wl_dir(h, dir), wr_dir(h, dir));
+    }
+  const int* pf3[3] = {P(BS_FLUX1), P(BS_FLUX2), P(BS_FLUX3)};
+  launch_flux_batch(b->recon, &b->ntot[BS_FLUX1], pf3, s, G, ng, pbb[to], 1);
+  const int ne = b->ntot[BS_EMF], nz = b->ntot[BS_ZONE];
+  hipLaunchKernelGGL(kb_emf, dim3((unsigned)(ne + b->ntot[BS_FACC])), blk, 0, s, G, P(BS_EMF), P(BS_FACC), ne, ng);
   // update (the reduced-traffic modes: the RK2/RK3 tables keep ucum at zero
   // until the last substep)
   bool zero_ucum = true;
   for (int st = 0; st + 1 < nto; st++)
     zero_ucum = zero_ucum && Cunew[st][0] == 0.0 && Cunew[st][1] == 0.0 && Cunew[st][2] == 0.0;
   const int mode = !zero_ucum ? kUpdAll : to == 0 ? kUpdFirst : finalstep ? kUpdLast : kUpdMiddle;
-  const dim3 gz((unsigned)b->ntot[BS_ZONE]);
+  if (mode == kUpdAll && b->ntot[BS_CT])
+    hipLaunchKernelGGL(kb_ct_all, dim3((unsigned)b->ntot[BS_CT]), blk, 0, s, G, P(BS_CT), ng);
+  const dim3 gz((unsigned)nz);
 #define BUPD(DM, MODE)                                                                                            \
-  hipLaunchKernelGGL((kb_update<DM, MODE>), gz, blk, 0, s, G, P(BS_ZONE), ng, pii[to], pbb[to], CUf[to][0],      \
-                     CUf[to][1], CUf[to][2], Cunew[to][0], Cunew[to][1], Cunew[to][2], to)
+  hipLaunchKernelGGL((kb_update<DM, MODE>), dim3((unsigned)(nz + ng)), blk, 0, s, G, P(BS_ZONE), ng, nz, pii[to], \
+                     pbb[to], CUf[to][0], CUf[to][1], CUf[to][2], Cunew[to][0], Cunew[to][1], Cunew[to][2], to,   \
+                     wflux[to])
 #define BUPD_MODES(DM)                                   \
   switch (mode) {                                        \
     case kUpdFirst: BUPD(DM, kUpdFirst); break;          \
@@ -2145,19 +2238,19 @@ harm_status enq_batch_substep(harm_batch* b, int to, int nto, const double CUf[4
   else { BUPD_MODES(-1); }
 #undef BUPD_MODES
 #undef BUPD
-  hipLaunchKernelGGL(kb_invert, gz, blk, 0, s, G, P(BS_ZONE), ng, pbb[to], pff[to], finalstep);
+  hipLaunchKernelGGL(kb_invert, dim3((unsigned)(nz + (ng + kBlock - 1) / kBlock)), blk, 0, s, G, P(BS_ZONE), ng, nz,
+                     pbb[to], pff[to], finalstep);
   if (finalstep) hipLaunchKernelGGL(kb_floors, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to]);
-  hipLaunchKernelGGL(kb_scal, dim3(g1), dim3(64), 0, s, G, ng, 2);
   // bounds, failure averaging, bounds
   if (b->bnd_merged) {
     const dim3 gb((unsigned)b->ntot[BS_BND]);
     if (b->dm == 3) {
-      hipLaunchKernelGGL(kb_bounds<true>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 0);
+      hipLaunchKernelGGL(kb_bounds<true>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 0, finalstep);
     } else {
-      hipLaunchKernelGGL(kb_bounds<false>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 0);
+      hipLaunchKernelGGL(kb_bounds<false>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 0, 0);
       hipLaunchKernelGGL(kb_post_fixup, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to], finalstep, 1);
       hipLaunchKernelGGL(kb_fixup_apply, gz, blk, 0, s, G, P(BS_ZONE), ng, pff[to], finalstep, 1);
-      hipLaunchKernelGGL(kb_bounds<false>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 1);
+      hipLaunchKernelGGL(kb_bounds<false>, gb, blk, 0, s, G, P(BS_BND), ng, pff[to], finalstep, 1, finalstep);
     }
     return hh::check_launch("batch substep");
   }
@@ -2190,9 +2283,10 @@ harm_status enq_batch_step(harm_batch* b)
   double CUf[4][4], Cunew[4][4], w[4];
   const int nto = rk_tables(b->timeorder, CUf, Cunew);
   rk_flux_weights(b->timeorder, w);
-  hipLaunchKernelGGL(kb_scal, dim3((unsigned)((ng + 63) / 64)), dim3(64), 0, b->stream, b->dref, ng, 1);
+  hipLaunchKernelGGL(kb_scal, dim3((unsigned)((ng + 63) / 64)), dim3(64), 0, b->stream, b->dref, ng, 0);
   for (int to = 0; to < nto; to++) HH_TRY(enq_batch_substep(b, to, nto, CUf, Cunew, w));
-  hipLaunchKernelGGL(kb_scal, dim3((unsigned)((ng + 63) / 64)), dim3(64), 0, b->stream, b->dref, ng, 3);
+  if (!b->bnd_merged)
+    hipLaunchKernelGGL(kb_scal, dim3((unsigned)((ng + 63) / 64)), dim3(64), 0, b->stream, b->dref, ng, 1);
   return hh::check_launch("batch step");
 }
 
@@ -2675,7 +2769,6 @@ harm_status enq_step(harm_handle* h)
   rk_flux_weights(h->cfg.timeorder, w);
   hipLaunchKernelGGL(k_scal_begin_step, dim3(1), dim3(1), 0, h->stream, h->ds, h->di);
   for (int to = 0; to < nto; to++) HH_TRY(enq_substep(h, to, nto, CUf, Cunew, w, true, true));
-  hipLaunchKernelGGL(k_scal_end_step, dim3(1), dim3(1), 0, h->stream, h->ds, h->di, h->P.safe);
   return hh::check_launch("harm_step");
 }
 }  // namespace
