@@ -719,6 +719,105 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
   }
 }
 
+// Faces of storage lines along DIR for one primitive, a zone a thread.  Line
+// index c = 0 .. n-1 is the coordinate m = c - 4 (m = -4 .. N+3); weights exist
+// for c = 2 .. n-3, ratios for the same zones (the left comparison from c = 4,
+// the right one up to c = n-5), faces for c = 3 .. n-4 (m = -1 .. N).  A block
+// holds T consecutive zones, f0-3 .. f0+T-4, of several lines: each thread forms
+// its zone's weights and leaves the two outer ones in LDS, then its ratio from
+// the weights two zones away, then its faces from the ratios one zone away;
+// the T - 6 inner zones own faces.  The lines are 8 consecutive i on 64-byte
+// boundaries (the neighbouring block has the other half of each 128-byte row,
+// on the same XCD).  LDS entries are numbered by thread, so a zone's
+// neighbours along the line are a fixed distance away.
+//
+// For grids whose lines are too few to fill the chip with sweeps, which take a
+// segment's zones one after the other: x2 + x3 take 59 + 62 us at 97x51x22 as
+// sweeps and 31 + 29 so, 54 and 9 (x2) at 200x100x1, 68 + 68 and 53 + 45 at
+// 96x64x32, 111 + 133 and 127 + 103 at 128x64x64.  On large grids its barriers
+// cost more than the sweeps' halo (waves in smooth regions wait for the
+// others): 308 + 347 and 446 + 390 at 256x128x64, where smaller blocks change
+// nothing (391 + 406 with 32 zones a segment).
+constexpr int kLineMax = 1024;  // threads of a block
+constexpr int kCols = 8;        // lines of a block
+struct LinePlan {
+  int T, nseg;   // zones a segment (halo included), segments a line
+  int nt, npl;   // line tiles, transverse planes
+  int threads;
+  long blocks;
+};
+template <int DIR>
+__global__ __launch_bounds__(kLineMax) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_weno_line(
+    Dims d, Box b, LinePlan pl, const double* __restrict__ pb, const double* __restrict__ dpd,
+    double* __restrict__ L, double* __restrict__ R)
+{
+  constexpr int S = kCols;  // distance of neighbours along the line
+  extern __shared__ double lds[];
+  double *ru0 = lds, *ru2 = lds + blockDim.x, *rfd = lds + 2 * blockDim.x;
+  const int tid = threadIdx.x;
+  int q = xcd_tile(blockIdx.x, gridDim.x);
+  const int tile = q % pl.nt;
+  q /= pl.nt;
+  const int sg = q % pl.nseg;
+  q /= pl.nseg;
+  const int plane = q % pl.npl, v = q / pl.npl;
+  const int w = tid % kCols, l = tid / kCols;
+  const int N = DIR == 2 ? d.n2 : d.n3, n = N + 8;
+  const int c = sg * (pl.T - 6) + l;  // line index of this thread's zone
+  const int i = -d.ng1 + tile * kCols + w;
+  const int j = DIR == 2 ? -4 + c : b.js + plane, k = DIR == 2 ? b.ks + plane : -4 + c;
+  const bool act = l < pl.T && c < n && i >= b.is && i < b.is + b.ni;
+  const unsigned st = DIR == 2 ? (unsigned)d.ps1 : (unsigned)d.ps1 * d.ns2;
+  const unsigned o = act ? (unsigned)hd::cidx(d, i, j, k) : 0u;  // (a plane stays below 2^29 elements)
+  const double* __restrict__ a = pb + (long)v * d.ncell;
+  const bool zone = act && c >= 2 && c <= n - 3;
+  double y[5];
+  ZoneW z = {};
+  if (zone) {
+#pragma unroll
+    for (int m = 0; m < 5; m++) y[m] = a[o + (m - 2) * st];
+    zone_weights(y + 2, z);
+  }
+  ru0[tid] = z.u[0];
+  ru2[tid] = z.u[2];
+  __syncthreads();
+  double fd = 0.0;
+  const bool ratio = zone && l >= 2 && l < pl.T - 2;
+  if (ratio) {
+    const bool hl = c >= 4, hr = c <= n - 5;
+    fd = ratio_lof(z.u[2], ru0[hl ? tid - 2 * S : tid], hl, z.u[0], ru2[hr ? tid + 2 * S : tid], hr);
+  }
+  rfd[tid] = fd;
+  __syncthreads();
+  if (zone && l >= 3 && l < pl.T - 3 && c >= 3 && c <= n - 4) {
+    const double dPi = dpd[o];
+    const double ss = wmin((fabs(dPi) - 0.5 * 0.5) / (0.5 * 0.5), 1.);
+    double lof = fd;
+    lof = wmax(lof, ss * rfd[tid + S]);
+    lof = wmax(lof, ss * rfd[tid - S]);
+    double lo, ro;
+    zone_faces(y + 2, z, lof, lo, ro);
+    L[(long)v * d.ncell + o] = lo;
+    R[(long)v * d.ncell + o] = ro;
+  }
+}
+
+// Segments: as few as keep a block within its threads, of equal length, so the
+// halo of six zones costs little (92 % of the threads own faces at 64 zones).
+LinePlan plan_lines(int dir, const Dims& d, const Box& b)
+{
+  LinePlan p{};
+  const int nf = (dir == 2 ? d.n2 : d.n3) + 2;  // faces of zones -1 .. N
+  const int tmax = kLineMax / kCols;
+  p.nseg = (nf + tmax - 7) / (tmax - 6);
+  p.T = (nf + p.nseg - 1) / p.nseg + 6;
+  p.npl = dir == 3 ? b.nj : b.nk;
+  p.nt = (b.is + b.ni + d.ng1 + kCols - 1) / kCols;
+  p.threads = (kCols * p.T + 63) / 64 * 64;
+  p.blocks = (long)p.nt * p.nseg * p.npl * HARM_NPR;
+  return p;
+}
+
 }  // namespace
 
 // dP of every active direction over the zones the face reconstructions read;
@@ -757,6 +856,16 @@ void launch_weno_recon(int dir, const Dims& d, const Box& b, hipStream_t s, cons
   const int N = dir == 2 ? d.n2 : d.n3;
   const int nf = N + 2;  // zones -1 .. N
   const long nl = (long)b.ni * (dir == 3 ? b.nj : b.nk);
+  // a zone a thread where that makes at most 72 waves a SIMD (about 550 000 zones)
+  constexpr long kLineWaves = 73728;
+  if (nl * N * HARM_NPR <= 64 * kLineWaves) {
+    const LinePlan p = plan_lines(dir, d, b);
+    const dim3 grid((unsigned)p.blocks), blk((unsigned)p.threads);
+    const size_t lds = sizeof(double) * 3 * p.threads;
+    if (dir == 2) hipLaunchKernelGGL(k_weno_line<2>, grid, blk, lds, s, d, b, p, pb, dpd, L, R);
+    if (dir == 3) hipLaunchKernelGGL(k_weno_line<3>, grid, blk, lds, s, d, b, p, pb, dpd, L, R);
+    return;
+  }
   const long waves1 = (nl * HARM_NPR + 63) / 64;
   int nseg = (int)std::max(1L, std::min((long)(nf / kMinSeg), (kWaveTarget + waves1 - 1) / waves1));
   const int seg = (nf + nseg - 1) / nseg;
