@@ -325,123 +325,141 @@ __global__ void k_ener_divb_final(const double* __restrict__ part, long n, doubl
   }
 }
 
-// The physics columns of one zone of HARM's main dump (dump_content,
-// dump.c:439-600, CALCFARADAYANDCURRENTS): column c (DC_* order) of zone t =
-// i + n1 (j + n2 k), the dump's row order, at out[c * cs + t * rs].  U is the
-// conserved state the last inversion consumed (udump = unewglobal,
-// initbase.c:885); J^mu from jcon (0 without it) and J_mu = lower_vec.
-__global__ __launch_bounds__(kBlock) void k_dump_cols(Dims d, Params P, const double* __restrict__ p,
-                                                      const double* __restrict__ ucum,
-                                                      const double* __restrict__ gcent,
-                                                      const double* __restrict__ jcon, double* __restrict__ out,
-                                                      long cs, long rs)
+// Rows z0 .. z0 + nz - 1 of HARM's main dump (dump_content, dump.c:439-600,
+// CALCFARADAYANDCURRENTS), row t = i + n1 (j + n2 k): the coordinates from the
+// axes' tables (X1, r of n1 zones, X2, theta of n2, X3, phi of n3), then the
+// physics columns (DC_* order).  U is the conserved state the last inversion
+// consumed (udump = unewglobal, initbase.c:885); J^mu from jcon (0 without it)
+// and J_mu = lower_vec.
+//
+// A wave builds the rows of 64 zones in LDS (an odd row stride: no bank
+// conflicts) and writes them as one contiguous run of 36 KB; straight from the
+// lanes each of the 72 stores would touch 64 lines.
+constexpr int kRowZones = 64, kRowStride = HARM_DUMP_NCOL + 1;
+__global__ __launch_bounds__(kRowZones) void k_dump_rows(Dims d, Params P, const double* __restrict__ p,
+                                                         const double* __restrict__ ucum,
+                                                         const double* __restrict__ gcent,
+                                                         const double* __restrict__ jcon,
+                                                         const double* __restrict__ axes, long z0, long nz,
+                                                         double* __restrict__ rows)
 {
-  const long nz = (long)d.n1 * d.n2 * d.n3;
-  const long t = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (t >= nz) return;
-  const int i = (int)(t % d.n1), j = (int)((t / d.n1) % d.n2), k = (int)(t / ((long)d.n1 * d.n2));
-  const long o = hd::cidx(d, i, j, k), nc = d.ncell;
-  Geom G;
-  hd::load_geom(gcent, hd::pidx(d, i, j), d.nplane, G);
-  double pz[HARM_NPR];
+  __shared__ double S[kRowZones * kRowStride];
+  const long b0 = (long)blockIdx.x * kRowZones;  // the block's first row
+  const int nrow = (int)min((long)kRowZones, nz - b0);
+  const int lane = threadIdx.x;
+  if (lane < nrow) {
+    const long t = z0 + b0 + lane;
+    const int i = (int)(t % d.n1), j = (int)((t / d.n1) % d.n2), k = (int)(t / ((long)d.n1 * d.n2));
+    double* row = S + lane * kRowStride;
+    const double *a2 = axes + 2 * d.n1, *a3 = a2 + 2 * d.n2;
+    row[0] = i;
+    row[1] = j;
+    row[2] = k;
+    row[3] = axes[i];
+    row[4] = a2[j];
+    row[5] = a3[k];
+    row[6] = axes[d.n1 + i];
+    row[7] = a2[d.n2 + j];
+    row[8] = a3[d.n3 + k];
+    const long o = hd::cidx(d, i, j, k), nc = d.ncell;
+    Geom G;
+    hd::load_geom(gcent, hd::pidx(d, i, j), d.nplane, G);
+    double pz[HARM_NPR];
 #pragma unroll
-  for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = p[pl * nc + o];
-  auto put = [&](int c, double v) { out[(long)c * cs + t * rs] = v; };
+    for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = p[pl * nc + o];
+    auto put = [&](int c, double v) { row[kDumpCoordCols + c] = v; };
 #pragma unroll
-  for (int pl = 0; pl < HARM_NPR; pl++) put(DC_P + pl, pz[pl]);
-  // ideal-gas EOS columns (idealgaseos.c:19, 48, 71)
-  const double rho0 = pz[HARM_RHO], u = pz[HARM_UU];
-  const double pressure = (P.gam - 1.) * u;
-  put(DC_PRESS, pressure);
-  put(DC_CS2, P.gam * pressure / (rho0 + u + pressure));
-  const double indexn = 1.0 / (P.gam - 1.);
-  double Sden;
-  if (rho0 < D_SMALL && pressure < D_SMALL) Sden = 0.0;
-  else if (rho0 < D_SMALL) Sden = 0.0;
-  else if (pressure < D_SMALL) Sden = -kBIG;
-  else Sden = rho0 * log(pow(pressure, indexn) / pow(rho0, indexn + 1.0));
-  put(DC_SDEN, Sden);
+    for (int pl = 0; pl < HARM_NPR; pl++) put(DC_P + pl, pz[pl]);
+    // ideal-gas EOS columns (idealgaseos.c:19, 48, 71)
+    const double rho0 = pz[HARM_RHO], u = pz[HARM_UU];
+    const double pressure = (P.gam - 1.) * u;
+    put(DC_PRESS, pressure);
+    put(DC_CS2, P.gam * pressure / (rho0 + u + pressure));
+    const double indexn = 1.0 / (P.gam - 1.);
+    double Sden;
+    if (rho0 < D_SMALL && pressure < D_SMALL) Sden = 0.0;
+    else if (rho0 < D_SMALL) Sden = 0.0;
+    else if (pressure < D_SMALL) Sden = -kBIG;
+    else Sden = rho0 * log(pow(pressure, indexn) / pow(rho0, indexn + 1.0));
+    put(DC_SDEN, Sden);
 #pragma unroll
-  for (int pl = 0; pl < HARM_NPR; pl++) put(DC_U + pl, ucum[pl * nc + o]);
-  put(DC_DIVB, corner_divb(d, P, p, gcent, i, j, k));
-  State q;
-  hd::get_state(pz, G, P.gam, q);
-  double bcon[4], bcov[4];
-  bcon[0] = pz[HARM_B1] * q.ucov[1] + pz[HARM_B2] * q.ucov[2] + pz[HARM_B3] * q.ucov[3];
+    for (int pl = 0; pl < HARM_NPR; pl++) put(DC_U + pl, ucum[pl * nc + o]);
+    put(DC_DIVB, corner_divb(d, P, p, gcent, i, j, k));
+    State q;
+    hd::get_state(pz, G, P.gam, q);
+    double bcon[4], bcov[4];
+    bcon[0] = pz[HARM_B1] * q.ucov[1] + pz[HARM_B2] * q.ucov[2] + pz[HARM_B3] * q.ucov[3];
 #pragma unroll
-  for (int m = 1; m < 4; m++) bcon[m] = (pz[HARM_B1 - 1 + m] + bcon[0] * q.ucon[m]) / q.ucon[0];
-  hd::lower(bcon, G, bcov);
-#pragma unroll
-  for (int m = 0; m < 4; m++) {
-    put(DC_UCON + m, q.ucon[m]);
-    put(DC_UCOV + m, q.ucov[m]);
-    put(DC_BCON + m, bcon[m]);
-    put(DC_BCOV + m, bcov[m]);
-  }
-#pragma unroll
-  for (int dir = 1; dir <= 3; dir++) {
-    double vmax, vmin;
-    hd::vchar(pz, q, dir, G, P.gam, vmax, vmin);
-    put(DC_VCHAR + 2 * (dir - 1), vmin);
-    put(DC_VCHAR + 2 * (dir - 1) + 1, vmax);
-  }
-  put(DC_GDET, G.gdet);
-  {
-    double jc[4] = {0.0, 0.0, 0.0, 0.0}, jl[4];
-    if (jcon) {
-#pragma unroll
-      for (int m = 0; m < 4; m++) jc[m] = jcon[(long)m * nc + o];
-    }
-    hd::lower(jc, G, jl);
+    for (int m = 1; m < 4; m++) bcon[m] = (pz[HARM_B1 - 1 + m] + bcon[0] * q.ucon[m]) / q.ucon[0];
+    hd::lower(bcon, G, bcov);
 #pragma unroll
     for (int m = 0; m < 4; m++) {
-      put(DC_JCON + m, jc[m]);
-      put(DC_JCOV + m, jl[m]);
+      put(DC_UCON + m, q.ucon[m]);
+      put(DC_UCOV + m, q.ucov[m]);
+      put(DC_BCON + m, bcon[m]);
+      put(DC_BCOV + m, bcov[m]);
+    }
+#pragma unroll
+    for (int dir = 1; dir <= 3; dir++) {
+      double vmax, vmin;
+      hd::vchar(pz, q, dir, G, P.gam, vmax, vmin);
+      put(DC_VCHAR + 2 * (dir - 1), vmin);
+      put(DC_VCHAR + 2 * (dir - 1) + 1, vmax);
+    }
+    put(DC_GDET, G.gdet);
+    {
+      double jc[4] = {0.0, 0.0, 0.0, 0.0}, jl[4];
+      if (jcon) {
+#pragma unroll
+        for (int m = 0; m < 4; m++) jc[m] = jcon[(long)m * nc + o];
+      }
+      hd::lower(jc, G, jl);
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        put(DC_JCON + m, jc[m]);
+        put(DC_JCOV + m, jl[m]);
+      }
+    }
+    // Faraday F^{mu nu} at the centre (current_precalc CURTYPEFARADAY,
+    // phys.c:701-708) and F_{mu nu} (lowerf, phys.tools.c:1449)
+    const double ig = -1.0 / G.gdet;
+    double f[6];
+    f[0] = ig * (bcov[3] * q.ucov[2] - bcov[2] * q.ucov[3]);
+    f[1] = ig * (-bcov[3] * q.ucov[1] + bcov[1] * q.ucov[3]);
+    f[2] = ig * (bcov[2] * q.ucov[1] - bcov[1] * q.ucov[2]);
+    f[3] = ig * (bcov[3] * q.ucov[0] - bcov[0] * q.ucov[3]);
+    f[4] = ig * (-bcov[2] * q.ucov[0] + bcov[0] * q.ucov[2]);
+    f[5] = ig * (bcov[1] * q.ucov[0] - bcov[0] * q.ucov[1]);
+    double F[4][4];
+    F[0][0] = F[1][1] = F[2][2] = F[3][3] = 0.0;
+    F[0][1] = f[0]; F[0][2] = f[1]; F[0][3] = f[2]; F[1][2] = f[3]; F[1][3] = f[4]; F[2][3] = f[5];
+    F[1][0] = -f[0]; F[2][0] = -f[1]; F[3][0] = -f[2]; F[2][1] = -f[3]; F[3][1] = -f[4]; F[3][2] = -f[5];
+    const int lo[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+      const int a = lo[c][0], b = lo[c][1];
+      double s = 0.0;
+#pragma unroll
+      for (int jp = 0; jp < 4; jp++)
+#pragma unroll
+        for (int kp = 0; kp < 4; kp++) s += F[jp][kp] * hd::gco(G, a, jp) * hd::gco(G, b, kp);
+      put(DC_FCON + c, f[c]);
+      put(DC_FCOV + c, s);
     }
   }
-  // Faraday F^{mu nu} at the centre (current_precalc CURTYPEFARADAY,
-  // phys.c:701-708) and F_{mu nu} (lowerf, phys.tools.c:1449)
-  const double ig = -1.0 / G.gdet;
-  double f[6];
-  f[0] = ig * (bcov[3] * q.ucov[2] - bcov[2] * q.ucov[3]);
-  f[1] = ig * (-bcov[3] * q.ucov[1] + bcov[1] * q.ucov[3]);
-  f[2] = ig * (bcov[2] * q.ucov[1] - bcov[1] * q.ucov[2]);
-  f[3] = ig * (bcov[3] * q.ucov[0] - bcov[0] * q.ucov[3]);
-  f[4] = ig * (-bcov[2] * q.ucov[0] + bcov[0] * q.ucov[2]);
-  f[5] = ig * (bcov[1] * q.ucov[0] - bcov[0] * q.ucov[1]);
-  double F[4][4];
-  F[0][0] = F[1][1] = F[2][2] = F[3][3] = 0.0;
-  F[0][1] = f[0]; F[0][2] = f[1]; F[0][3] = f[2]; F[1][2] = f[3]; F[1][3] = f[4]; F[2][3] = f[5];
-  F[1][0] = -f[0]; F[2][0] = -f[1]; F[3][0] = -f[2]; F[2][1] = -f[3]; F[3][1] = -f[4]; F[3][2] = -f[5];
-  const int lo[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
-#pragma unroll
-  for (int c = 0; c < 6; c++) {
-    const int a = lo[c][0], b = lo[c][1];
-    double s = 0.0;
-#pragma unroll
-    for (int jp = 0; jp < 4; jp++)
-#pragma unroll
-      for (int kp = 0; kp < 4; kp++) s += F[jp][kp] * hd::gco(G, a, jp) * hd::gco(G, b, kp);
-    put(DC_FCON + c, f[c]);
-    put(DC_FCOV + c, s);
-  }
+  __syncthreads();
+  double* dst = rows + b0 * HARM_DUMP_NCOL;
+  for (int e = lane; e < nrow * HARM_DUMP_NCOL; e += kRowZones)
+    dst[e] = S[e / HARM_DUMP_NCOL * kRowStride + e % HARM_DUMP_NCOL];
 }
 
 }  // namespace
 
-void launch_dump_cols(const hd::Dims& d, const Params& P, const double* p, const double* ucum, const double* gcent,
-                      const double* jcon, double* out, hipStream_t s)
-{
-  const long nz = (long)d.n1 * d.n2 * d.n3;
-  hipLaunchKernelGGL(k_dump_cols, dim3(nblk(nz)), dim3(kBlock), 0, s, d, P, p, ucum, gcent, jcon, out, nz, 1L);
-}
-
 void launch_dump_rows(const hd::Dims& d, const Params& P, const double* p, const double* ucum, const double* gcent,
-                      const double* jcon, double* rows, hipStream_t s)
+                      const double* jcon, const double* axes, long z0, long nz, double* rows, hipStream_t s)
 {
-  const long nz = (long)d.n1 * d.n2 * d.n3;
-  hipLaunchKernelGGL(k_dump_cols, dim3(nblk(nz)), dim3(kBlock), 0, s, d, P, p, ucum, gcent, jcon,
-                     rows + kDumpCoordCols, 1L, (long)HARM_DUMP_NCOL);
+  hipLaunchKernelGGL(k_dump_rows, dim3((unsigned)((nz + kRowZones - 1) / kRowZones)), dim3(kRowZones), 0, s, d, P, p,
+                     ucum, gcent, jcon, axes, z0, nz, rows);
 }
 
 namespace {

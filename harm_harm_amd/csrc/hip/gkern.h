@@ -239,23 +239,20 @@ void launch_ener_reduce(const double* part, long nblk, double* en, const int* ds
 // from the states the inversion kept (fx_*) and the primitives pf after it
 void launch_ener_fix(const hd::Dims& d, const Params& P, const double* pf, const double* gcent, const double* fx_p0,
                      const double* fx_pfl, const uint8_t* fx_flag, double* part, double* en, hipStream_t s);
-// The main dump's physics columns (dump_content, dump.c:439-600), device
-// SoA out[c][nz] in the dump's row order (i fastest, then j, then k): the
-// primitives, pressure, cs2, entropy density, U (from ucum), |div B|, u^mu,
-// u_mu, b^mu, b_mu, (vmin, vmax) per direction, gdet, F^{mu nu}, F_{mu nu}.
-// The coordinates and the current columns are the host's.
+// The main dump's rows (dump_content, dump.c:439-600): rows z0 .. z0 + nz - 1
+// (i fastest, then j, then k) at rows[(z - z0) * HARM_DUMP_NCOL + c].  axes:
+// X1, r of the n1 zones, X2, theta of the n2, X3, phi of the n3.  jcon: J^mu
+// (4 x ncell, harm_currents), or null for zeros.  The columns: i, j, k, X,
+// (r, theta, phi), then (DC_*) the primitives, pressure, cs2, entropy density,
+// U (from ucum), |div B|, u^mu, u_mu, b^mu, b_mu, (vmin, vmax) per direction,
+// gdet, J^mu, J_mu, F^{mu nu}, F_{mu nu}.
 enum { DC_P = 0, DC_PRESS = 8, DC_CS2 = 9, DC_SDEN = 10, DC_U = 11, DC_DIVB = 19, DC_UCON = 20, DC_UCOV = 24,
        DC_BCON = 28, DC_BCOV = 32, DC_VCHAR = 36, DC_GDET = 42, DC_JCON = 43, DC_JCOV = 47, DC_FCON = 51,
        DC_FCOV = 57, DC_N = 63 };
-void launch_dump_cols(const hd::Dims& d, const Params& P, const double* p, const double* ucum, const double* gcent,
-                      const double* jcon, double* out, hipStream_t s);
-// The same columns straight into the dump's rows: rows[z * HARM_DUMP_NCOL +
-// c], columns kDumpCoordCols.. (the coordinate columns before them are left
-// as they are).  jcon: J^mu (4 x ncell, harm_currents), or null for zeros.
 enum { kDumpCoordCols = 9 };
 static_assert(kDumpCoordCols + DC_N == HARM_DUMP_NCOL, "dump row layout");
 void launch_dump_rows(const hd::Dims& d, const Params& P, const double* p, const double* ucum, const double* gcent,
-                      const double* jcon, double* rows, hipStream_t s);
+                      const double* jcon, const double* axes, long z0, long nz, double* rows, hipStream_t s);
 // The main dump's four-current (CURRENTCALC1): the Faraday samples of every
 // storage zone (current_precalc phys.c:622; cf: 18 x ncell, slot * 3 + c) and
 // J^mu of the active zones from them (current_calc_1 phys.c:846; jcon: 4 x

@@ -1354,6 +1354,8 @@ struct harm_handle {
   hipEvent_t evfork = nullptr, evjoin[2] = {nullptr, nullptr};
   double* cf = nullptr;    // the dump's four-current: Faraday samples (18 x ncell) and J^mu (4 x ncell),
   double* jcon = nullptr;  // allocated by the first harm_currents
+  double* axes = nullptr;  // zone-centre coordinates per axis (X1, r | X2, theta | X3, phi), for the dump's rows
+  double* rows = nullptr;  // a chunk of the main dump's rows, allocated by the first harm_dump_columns
   double* xfer = nullptr;  // HARM's interleaved layout of one array (NPR x storage cells), staged for set/get
   long cur_calls = 0;      // current_calc_1's call count and the dt of its last call
   double cur_lastdt = 0.0;
@@ -1509,6 +1511,26 @@ harm_status build_geometry(harm_handle* h)
   HH_TRY(upload(h, h->rcent, h->hrcent.data(), h->hrcent.size()));
   return HARM_OK;
 }
+
+// zone-centre coordinates of each axis as harm_get_coords gives them
+harm_status build_axes(harm_handle* h)
+{
+  const int n[3] = {h->d.n1, h->d.n2, h->d.n3};
+  std::vector<double> a(2 * (size_t)(n[0] + n[1] + n[2]));
+  double* q = a.data();
+  for (int m = 0; m < 3; m++) {
+    for (int c = 0; c < n[m]; c++) {
+      double X[4], V[4];
+      harm_get_coords(h, m == 0 ? c : 0, m == 1 ? c : 0, m == 2 ? c : 0, X, V);
+      q[c] = X[m + 1];
+      q[n[m] + c] = V[m + 1];
+    }
+    q += 2 * n[m];
+  }
+  HH_TRY(alloc((void**)&h->axes, sizeof(double) * a.size()));
+  return upload(h, h->axes, a.data(), a.size());
+}
+
 
 hipEvent_t ev_get(harm_handle* h)
 {
@@ -2377,6 +2399,7 @@ extern "C" harm_status harm_create(const harm_config* cfg, harm_handle** out)
   TRYC(alloc((void**)&h->di, sizeof(unsigned long long) * DI_N));
   TRYC(hh::check_hip(hipMemset(h->di, 0, sizeof(unsigned long long) * DI_N), "hipMemset"));
   TRYC(build_geometry(h));
+  TRYC(build_axes(h));
   for (int dir = 1; dir <= 3; dir++) h->ft[dir] = plan_face_tile(d, dir);
 #undef TRYC
   *out = h;
@@ -2400,7 +2423,7 @@ extern "C" harm_status harm_destroy(harm_handle* h)
   }
   for (hipEvent_t e : h->evpool) (void)hipEventDestroy(e);
   void* bufs[] = {h->pflag, h->pfix, h->gcorn3, h->conn, h->floors, h->rcent, h->emf, h->wl, h->wr, h->wdp, h->wtm, h->facc,
-                  h->cf, h->jcon, h->xfer,
+                  h->cf, h->jcon, h->xfer, h->axes, h->rows,
                   h->en, h->enpart, h->entot, h->fx_p0, h->fx_pfl, h->fx_flag, h->ds, h->di};
   for (void* b : bufs) (void)hipFree(b);
   for (int q = 0; q < 2; q++) {
@@ -2918,29 +2941,25 @@ harm_status write_rows(FILE* f, const double* rows, long nz, int ncol)
 }
 }  // namespace
 
+// The rows are built on the device a chunk at a time (37.7 MB, kept with the
+// handle) and copied straight into the caller's.
+constexpr long kRowChunk = 65536;
 extern "C" harm_status harm_dump_columns(harm_handle* h, int32_t which, double* rows)
 {
   HH_TRY(check_handle(h));
   if (!rows) return hh::set_error(HARM_EINVAL, "harm_dump_columns: null argument");
   if (which < 0 || which >= HARM_NARR) return hh::set_error(HARM_EINVAL, "harm_dump_columns: bad array %d", which);
   const Dims& d = h->d;
-  const long nz = (long)d.n1 * d.n2 * d.n3;
-  double* dcol = nullptr;
-  HH_TRY(alloc((void**)&dcol, sizeof(double) * DC_N * nz));
-  launch_dump_cols(d, h->P, h->arr[which], h->arr[HARM_ARR_UCUM], h->geom[HARM_LOC_CENT], h->jcon, dcol, h->stream);
-  std::vector<double> col((size_t)DC_N * nz);
-  harm_status st = hh::check_launch("k_dump_cols");
-  if (st == HARM_OK) st = hh::check_hip(hipStreamSynchronize(h->stream), "harm_dump_columns");
-  if (st == HARM_OK)
-    st = hh::check_hip(hipMemcpy(col.data(), dcol, sizeof(double) * col.size(), hipMemcpyDeviceToHost), "copy");
-  (void)hipFree(dcol);
-  if (st != HARM_OK) return st;
-  // dump_content's column order: coordinates, then the device columns
-  for (long t = 0; t < nz; t++) {
-    const int i = (int)(t % d.n1), j = (int)((t / d.n1) % d.n2), k = (int)(t / ((long)d.n1 * d.n2));
-    double* r = rows + t * HARM_DUMP_NCOL;
-    dump_coords(h, i, j, k, r);
-    for (int q = 0; q < DC_N; q++) r[kDumpCoordCols + q] = col[(size_t)q * nz + t];
+  const long nz = (long)d.n1 * d.n2 * d.n3, chunk = std::min(nz, kRowChunk);
+  if (!h->rows) HH_TRY(alloc((void**)&h->rows, sizeof(double) * HARM_DUMP_NCOL * chunk));
+  for (long z = 0; z < nz; z += chunk) {
+    const long n = std::min(chunk, nz - z);
+    launch_dump_rows(d, h->P, h->arr[which], h->arr[HARM_ARR_UCUM], h->geom[HARM_LOC_CENT], h->jcon, h->axes, z, n,
+                     h->rows, h->stream);
+    HH_TRY(hh::check_launch("k_dump_rows"));
+    HH_HIP(hipMemcpyAsync(rows + z * HARM_DUMP_NCOL, h->rows, sizeof(double) * HARM_DUMP_NCOL * n,
+                          hipMemcpyDeviceToHost, h->stream));
+    HH_HIP(hipStreamSynchronize(h->stream));
   }
   return HARM_OK;
 }
@@ -2993,18 +3012,12 @@ extern "C" harm_status harm_dump_columns_noalloc(harm_handle* h, int32_t which, 
                          kNoallocZones);
   double* dev = nullptr;
   HH_TRY(scratch_on(h->dev, &dev));
-  // every column of every row the copy takes is written: the kernel fills
-  // the physics columns (the four-current included), the host the
-  // coordinates after the copy
-  launch_dump_rows(d, h->P, h->arr[which], h->arr[HARM_ARR_UCUM], h->geom[HARM_LOC_CENT], h->jcon, dev, h->stream);
-  HH_TRY(hh::check_launch("k_dump_cols"));
+  // every column of every row the copy takes is written by the kernel
+  launch_dump_rows(d, h->P, h->arr[which], h->arr[HARM_ARR_UCUM], h->geom[HARM_LOC_CENT], h->jcon, h->axes, 0, nz,
+                   dev, h->stream);
+  HH_TRY(hh::check_launch("k_dump_rows"));
   HH_HIP(hipMemcpyAsync(rows, dev, sizeof(double) * HARM_DUMP_NCOL * nz, hipMemcpyDeviceToHost, h->stream));
-  HH_HIP(hipStreamSynchronize(h->stream));
-  for (long t = 0; t < nz; t++) {
-    const int i = (int)(t % d.n1), j = (int)((t / d.n1) % d.n2), k = (int)(t / ((long)d.n1 * d.n2));
-    dump_coords(h, i, j, k, rows + t * HARM_DUMP_NCOL);
-  }
-  return HARM_OK;
+  return hh::check_hip(hipStreamSynchronize(h->stream), "harm_dump_columns_noalloc");
 }
 
 // The four-current the main dump carries (CALCFARADAYANDCURRENTS 1,
