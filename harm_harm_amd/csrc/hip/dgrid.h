@@ -136,7 +136,7 @@ constexpr double kBondiC2x = 1.373125, kBondiKx = 1.0;
 // radius r, with u^r the Kerr-Schild radial 4-velocity (spin 0) and
 // T = p/rho, n = 1/(Gamma-1).
 __device__ __forceinline__ void bondi_integrals(const double* pr, const Geom& G, double r, double R0, double gam,
-                                                double& C1, double& C2, double& K)
+                                                double& C1, double& C2, double& K, double& T)
 {
   State q;
   get_state(pr, G, gam, q);
@@ -144,66 +144,79 @@ __device__ __forceinline__ void bondi_integrals(const double* pr, const Geom& G,
   const double n = 1 / (gam - 1);
   const double p = (gam - 1) * pr[HARM_UU];
   const double rho = pr[HARM_RHO];
-  const double T = p / rho;
+  T = p / rho;
+  const double h = 1 + (1 + n) * T;
   C1 = pow(T, n) * ur * r * r;
-  C2 = pow(1 + (1 + n) * T, 2.) * (1 - 2. / r + ur * ur);
+  C2 = h * h * (1 - 2. / r + ur * ur);
   K = p / pow(rho, gam);
+}
+
+// Newton steps on h(T) = T - f(T) (below) from a start that is already close,
+// to a step below 1e-12 of T, which leaves an error of order its square (a
+// tighter test could chase the rounding noise of pow and sqrt).  Returns true
+// only where the reference's iteration from T = 0.1 settles on the same root
+// before its cap of 250.  Inside, T <- T + 0.02 (T - f) multiplies the error
+// by 1 - 0.02 (f' - 1): 8 < f' < 40 gives 0.22 to 0.86, the first step must
+// go towards the root without passing it (f is convex there, so later ones do
+// not pass it either), and below f' = 8 the cap can end it early.  Outside,
+// T <- f(T) falls from 0.1 to the larger of the two roots, f' < 1, by f' a
+// step: 0.87^250 = 8e-16.  A NaN anywhere returns false.
+__device__ __forceinline__ bool bondi_newton(double n, double C1, double C2, double r, double& T)
+{
+  const double r2 = r * r, g = 1 - 2 / r, c = sqrt(C2);
+  const double ua = C1 / (r2 * pow(0.1, n));
+  const double ha = 0.1 - (sqrt(C2 / (g + ua * ua)) - 1) / (1 + n);  // h(0.1)
+  double most = 0.5;
+  for (int k = 0; k < 10; k++) {
+    const double u = C1 / (r2 * pow(T, n));
+    const double w = g + u * u;
+    const double f = (sqrt(C2 / w) - 1) / (1 + n);
+    const double fp = n * c * u * u / ((1 + n) * T * w * sqrt(w));
+    const double Tn = T - (T - f) / (1 - fp), step = fabs(Tn - T);
+    if (!(step <= most * fabs(T)) || !(Tn > 0.0)) return false;  // growing steps, or NaN
+    most = fmax(0.5 * step / fabs(T), 1e-11);
+    T = Tn;
+    if (step <= 1e-12 * Tn) {
+      const double first = 0.1 + 0.02 * ha;
+      if (r < 2.5) return fp > 8 && fp < 40 && (ha > 0 ? first < Tn : first > Tn);
+      return fp < 0.87 && ha > 0 && Tn < 0.1;
+    }
+  }
+  return false;
 }
 
 // bondi_invert_integrals (bounds.sasha.c:1101): the temperature at radius r
 // from the integrals, then rho, u and u^r.  The temperature is the root of
 // h(T) = T - f(T), f(T) = (sqrt(C2/(1 - 2/r + u^2)) - 1)/(1 + n),
-// u = C1/(r^2 T^n).  For r > 9 the reference's plain iteration T <- f(T) is
+// u = C1/(r^2 T^n).  Newton steps from the boundary zone's temperature Tz,
+// a few percent away, find it in four or five.  A step is one dependent chain
+// (pow, sqrt, two divisions) on the few lanes that have a boundary zone, so
+// only fewer steps help: with the reference's 10 to 190 the 30 RK2 steps of a
+// 256 x 130 PARA grid took 6.0 ms, with these 4.6.  Where Newton does not settle, the reference's
+// iterations decide.  For r > 9 its plain iteration T <- f(T) is
 // used as written.  For 0.35 < r < 2.5 the root is a repelling fixed point of
 // f, which the reference reaches by the damped iteration
 // T <- T + 0.02 (T - f(T)), converging linearly (100-170 steps at the inner
-// boundary); here that iteration runs until its steps fall below 1e-4 of T
-// and Newton steps on h finish it (the same root, to 1.3e-14 of the
-// reference's over randomized integrals; about 30 steps).  A Newton
-// step moving T by more than 1 % hands back to the damped iteration to the
-// reference's own tolerance.  Returns false outside those radii or when the
+// boundary).  Returns false outside those radii or when the
 // outer iteration does not decrease monotonically (the reference stops the
 // run there).
-__device__ __forceinline__ bool bondi_invert(double n, double C1, double C2, double K, double r, double& rho,
-                                             double& uu, double& ur)
+__device__ __forceinline__ bool bondi_invert(double n, double C1, double C2, double K, double r, double Tz,
+                                             double& rho, double& uu, double& ur)
 {
   const double relative_accuracy = 1.0e-15;
   const int max_iter = 250;
-  double T0 = 0.2, T1 = 0.1, u1;
+  double T0 = 0.2, T1 = Tz, u1;
   int iter;
-  if (r > 0.35 && r < 2.5) {
-    for (iter = 0; iter < max_iter && fabs((T0 - T1) / T1) > 1.0e-4; iter++) {
+  if (((r > 0.35 && r < 2.5) || r > 9) && bondi_newton(n, C1, C2, r, T1)) {
+  } else if (r > 0.35 && r < 2.5) {
+    T1 = 0.1;
+    for (iter = 0; iter < max_iter && fabs((T0 - T1) / T1) > relative_accuracy; iter++) {
       T0 = T1;
       u1 = C1 / (r * r * pow(T0, n));
       T1 = T0 + 0.02 * (T0 - (sqrt(C2 / (1 - 2 / r + u1 * u1)) - 1) / (1 + n));
     }
-    bool polished = false;
-    double T = T1;
-    for (int k = 0; k < 8; k++) {
-      const double u = C1 / (r * r * pow(T, n));
-      const double w = 1 - 2 / r + u * u;
-      const double f = (sqrt(C2 / w) - 1) / (1 + n);
-      const double fp = n * sqrt(C2) * u * u / ((1 + n) * T * w * sqrt(w));
-      const double Tn = T - (T - f) / (1 - fp);
-      if (!(fabs(Tn - T) <= 1e-2 * fabs(T))) break;  // leaving the basin (or NaN)
-      // a step below 1e-12 of T leaves an error of order its square: T is
-      // converged to the last bits (a tighter test could chase the rounding
-      // noise of pow and sqrt)
-      if (fabs(Tn - T) <= 1e-12 * fabs(Tn)) {
-        T = Tn;
-        polished = true;
-        break;
-      }
-      T = Tn;
-    }
-    if (polished) T1 = T;
-    else
-      for (; iter < max_iter && fabs((T0 - T1) / T1) > relative_accuracy; iter++) {
-        T0 = T1;
-        u1 = C1 / (r * r * pow(T0, n));
-        T1 = T0 + 0.02 * (T0 - (sqrt(C2 / (1 - 2 / r + u1 * u1)) - 1) / (1 + n));
-      }
   } else if (r > 9) {
+    T1 = 0.1;
     for (iter = 0; iter < max_iter && (T0 - T1) / T1 > relative_accuracy; iter++) {
       T0 = T1;
       u1 = C1 / (r * r * pow(T0, n));

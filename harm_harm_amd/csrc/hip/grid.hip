@@ -902,8 +902,8 @@ __device__ void bondi_line(const Dims& d, const Params& P, double* p, const doub
   Geom Gr;
   hd::load_geom(gcent, hd::pidx(d, ri, j), d.nplane, Gr);
   const double rr = P.R0 + exp(P.startx[1] + (ri + 0.5) * P.dx[1]);
-  double C1, C2, K;
-  hd::bondi_integrals(pr, Gr, rr, P.R0, P.gam, C1, C2, K);
+  double C1, C2, K, Tz;
+  hd::bondi_integrals(pr, Gr, rr, P.R0, P.gam, C1, C2, K, Tz);
   if (up) {
     C2 = hd::kBondiC2x;
     K = hd::kBondiKx;
@@ -913,7 +913,7 @@ __device__ void bondi_line(const Dims& d, const Params& P, double* p, const doub
 #pragma unroll
   for (int pl = 0; pl < HARM_NPR; pl++) pi[pl] = 0.0;
   double ur = 0.0;
-  hd::bondi_invert(1 / (P.gam - 1), C1, C2, K, r, pi[HARM_RHO], pi[HARM_UU], ur);
+  hd::bondi_invert(1 / (P.gam - 1), C1, C2, K, r, Tz, pi[HARM_RHO], pi[HARM_UU], ur);
   Geom Gi;
   hd::load_geom(gcent, hd::pidx(d, i, j), d.nplane, Gi);
   hd::radial_ks_to_rel4(ur, r, P.R0, Gi, pi);
