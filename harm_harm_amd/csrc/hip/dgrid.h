@@ -192,12 +192,11 @@ __device__ __forceinline__ bool bondi_newton(double n, double C1, double C2, dou
 // a few percent away, find it in four or five.  A step is one dependent chain
 // (pow, sqrt, two divisions) on the few lanes that have a boundary zone, so
 // only fewer steps help: with the reference's 10 to 190 the 30 RK2 steps of a
-// 256 x 130 PARA grid took 6.0 ms, with these 4.6.  Where Newton does not settle, the reference's
-// iterations decide.  For r > 9 its plain iteration T <- f(T) is
-// used as written.  For 0.35 < r < 2.5 the root is a repelling fixed point of
-// f, which the reference reaches by the damped iteration
-// T <- T + 0.02 (T - f(T)), converging linearly (100-170 steps at the inner
-// boundary).  Returns false outside those radii or when the
+// 256 x 130 PARA grid took 6.0 ms, with these 4.6.  Where Newton does not
+// settle, the reference's iterations decide.  For r > 9 its plain iteration
+// T <- f(T) is used as written.  For 0.35 < r < 2.5 the root is a repelling
+// fixed point of f, which the reference reaches by the damped iteration
+// T <- T + 0.02 (T - f(T)).  Returns false outside those radii or when the
 // outer iteration does not decrease monotonically (the reference stops the
 // run there).
 __device__ __forceinline__ bool bondi_invert(double n, double C1, double C2, double K, double r, double Tz,

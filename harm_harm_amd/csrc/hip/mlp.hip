@@ -1,7 +1,7 @@
 // mlp.hip -- training and inference kernels of the learned inversion guess,
 // and the batched inversion seeded by it.
 //
-// Training runs in one persistent workgroup (4 wavefronts) that loops over
+// Training runs in one persistent workgroup (8 wavefronts) that loops over
 // minibatches of 128 pairs: forward (three BF16 matrix products with FP32
 // accumulation, tanh hidden layers), mean-squared error on the standardised
 // targets, backward (the weight gradients as transposed products X^T G, the
@@ -41,83 +41,84 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kBatch = 128;     // training minibatch
 constexpr int kWaves = kBlock / 64;
+using hm::v4s;
 
 // ---------------------------------------------------------------------------
 // shared pieces
 // ---------------------------------------------------------------------------
 
-// BF16 images of the weights from the FP32 parameters (zero padding).
+// BF16 images of the weights from the FP32 parameters (the rows' padding zero).
 __global__ void k_mlp_pack(const float* __restrict__ w, uint16_t* __restrict__ wbf)
 {
   for (int e = threadIdx.x + blockIdx.x * blockDim.x; e < hm::kNBf; e += blockDim.x * gridDim.x) {
     float v = 0.0f;
     if (e < hm::kBfW2) {
-      const int f = e / hm::kHid, h = e % hm::kHid;
-      if (f < hm::kIn) v = w[hm::kOffW1 + f * hm::kHid + h];
+      const int h = e / hm::kIn, f = e % hm::kIn;
+      v = w[hm::kOffW1 + f * hm::kHid + h];
     } else if (e < hm::kBfW3) {
-      v = w[hm::kOffW2 + (e - hm::kBfW2)];
+      const int x = e - hm::kBfW2, o = x / hm::kStride, h = x % hm::kStride;
+      if (h < hm::kHid) v = w[hm::kOffW2 + h * hm::kHid + o];
     } else {
-      const int x = e - hm::kBfW3, h = x / hm::kOutPad, o = x % hm::kOutPad;
-      if (o < hm::kOut) v = w[hm::kOffW3 + h * hm::kOut + o];
+      const int x = e - hm::kBfW3, o = x / hm::kStride, h = x % hm::kStride;
+      if (h < hm::kHid) v = w[hm::kOffW3 + h * hm::kOut + o];
     }
     wbf[e] = hm::f2bf(v);
   }
 }
 
-// Weights and biases into LDS for the forward products.
-__device__ void stage_weights(const uint16_t* __restrict__ wbf, const float* __restrict__ w32, uint16_t* sW,
-                              float* sBias)
+// What a forward pass reads, in LDS: the weight images and the biases of the
+// three layers.
+constexpr int kNBias = 2 * hm::kHid + 4;
+struct __align__(16) Net {
+  uint16_t w[hm::kNBf];
+  float b[kNBias];
+};
+
+__device__ void stage_net(const uint16_t* __restrict__ wbf, const float* __restrict__ w32, Net& N)
 {
-  for (int e = threadIdx.x; e < hm::kNBf; e += blockDim.x) sW[e] = wbf[e];
+  const uint4* src = (const uint4*)wbf;
+  uint4* dst = (uint4*)N.w;
+  for (int e = threadIdx.x; e < hm::kNBf / 8; e += blockDim.x) dst[e] = src[e];
   for (int e = threadIdx.x; e < hm::kHid; e += blockDim.x) {
-    sBias[e] = w32[hm::kOffB1 + e];
-    sBias[hm::kHid + e] = w32[hm::kOffB2 + e];
+    N.b[e] = w32[hm::kOffB1 + e];
+    N.b[hm::kHid + e] = w32[hm::kOffB2 + e];
   }
-  if (threadIdx.x < hm::kOut) sBias[2 * hm::kHid + threadIdx.x] = w32[hm::kOffB3 + threadIdx.x];
+  if (threadIdx.x < 4) N.b[2 * hm::kHid + threadIdx.x] = threadIdx.x < hm::kOut ? w32[hm::kOffB3 + threadIdx.x] : 0.0f;
 }
 
-// Forward pass of one wavefront's 64 samples.  X (standardised, BF16) is in
-// bufA with row stride 16; the hidden layers go to bufB then bufA (row stride
-// 64); the two standardised outputs of sample m land in y[2*m + o].  Every
-// thread of the block must call it (it synchronises the block between
-// layers); the caller must make X visible first.
-__device__ void wave_forward(uint16_t* bufA, uint16_t* bufB, const uint16_t* sW, const float* sBias, float* y)
+// The network over a wave's 64 samples, lane l's raw features in f (zeros for
+// a lane without one): output o (or, NOUT 1, output 0 alone) of the lane's own
+// sample, standardised, in y[o].  The features pass between lanes through the
+// wave's xs; each 16 samples stay in registers from there on, so the block
+// needs no barrier.
+template <int NOUT>
+__device__ __forceinline__ void wave_net(const float* f, bool act, const float* __restrict__ norm, const Net& N,
+                                         uint16_t (*xs)[hm::kIn], float* y)
 {
   const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-  // layer 1: [64 x 16] x [16 x 64]
-  for (int t = 0; t < 16; t++) {
-    const int mt = t >> 2, nt = t & 3;
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
-    acc = hm::mma16(bufA + mt * 16 * hm::kInPad, hm::kInPad, 1, sW + hm::kBfW1 + nt * 16, hm::kHid, 1, hm::kInPad, acc);
+  v4f lo, hi;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int m = mt * 16 + 4 * q + i, n = nt * 16 + r;
-      bufB[m * hm::kHid + n] = hm::f2bf(tanhf(acc[i] + sBias[n]));
+  for (int k = 0; k < 4; k++) {
+    lo[k] = act ? (f[k] - norm[k]) * norm[hm::kIn + k] : 0.0f;
+    hi[k] = act ? (f[4 + k] - norm[4 + k]) * norm[hm::kIn + 4 + k] : 0.0f;
+  }
+  *(v4s*)&xs[l][0] = hm::f2bf4(lo);
+  *(v4s*)&xs[l][4] = hm::f2bf4(hi);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+  for (int m = 0; m < 4; m++) {
+    v4s x = hm::frag(&xs[m * 16 + r][4 * (q & 1)]), h1[4], h2[4];
+    if (q > 1) x = (v4s){0, 0, 0, 0};
+    hm::layer1(x, N.w + hm::kBfW1, N.b, h1);
+    hm::layer<4>(h1, N.w + hm::kBfW2, hm::kStride, N.b + hm::kHid, h2);
+    const v4f acc = hm::layer3(h2, N.w + hm::kBfW3);
+#pragma unroll
+    for (int o = 0; o < NOUT; o++) {
+      const float v = __shfl(acc[o] + N.b[2 * hm::kHid + o], r);
+      if (q == m) y[o] = v;
     }
   }
-  __syncthreads();
-  // layer 2: [64 x 64] x [64 x 64]
-  for (int t = 0; t < 16; t++) {
-    const int mt = t >> 2, nt = t & 3;
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
-    acc = hm::mma16(bufB + mt * 16 * hm::kHid, hm::kHid, 1, sW + hm::kBfW2 + nt * 16, hm::kHid, 1, hm::kHid, acc);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int m = mt * 16 + 4 * q + i, n = nt * 16 + r;
-      bufA[m * hm::kHid + n] = hm::f2bf(tanhf(acc[i] + sBias[hm::kHid + n]));
-    }
-  }
-  __syncthreads();
-  // layer 3: [64 x 64] x [64 x 16 (2 used)]
-  for (int mt = 0; mt < 4; mt++) {
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
-    acc = hm::mma16(bufA + mt * 16 * hm::kHid, hm::kHid, 1, sW + hm::kBfW3, hm::kOutPad, 1, hm::kHid, acc);
-    if (r < hm::kOut) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) y[(mt * 16 + 4 * q + i) * 2 + r] = acc[i] + sBias[2 * hm::kHid + r];
-    }
-  }
-  __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -178,222 +179,347 @@ struct TrainArgs {
   int nsteps;
   long t0;             // Adam steps before this launch
   float lr, beta1, beta2, eps;
-  int update;          // 0: write gradients of one batch to grad_out instead of stepping
-  float* grad_out;
+  float* grad_out;     // UPDATE false: one batch's gradients, nothing else changed
   float* loss_out;     // mean loss over the launch's steps
 };
 
-__global__ __launch_bounds__(kBlock) void k_mlp_train(TrainArgs a)
-{
-  __shared__ uint16_t sX[kBatch * hm::kInPad];
-  __shared__ uint16_t sH1[kBatch * hm::kHid];
-  __shared__ uint16_t sH2[kBatch * hm::kHid];
-  __shared__ uint16_t sG1[kBatch * hm::kHid];
-  __shared__ uint16_t sG2[kBatch * hm::kHid];
-  __shared__ uint16_t sDY[kBatch * hm::kOutPad];
-  __shared__ float sT[kBatch * hm::kOut];
-  __shared__ float sErr[kBatch * hm::kOut];
-  __shared__ float sDYf[kBatch * hm::kOut];
-  __shared__ uint16_t sW[hm::kNBf];
-  __shared__ float sBias[2 * hm::kHid + hm::kOut];
+constexpr int kTrainBlock = 512;
+constexpr int kRow = kBatch + 8;  // a row of a transposed layer: 68 words, rows 4 banks apart
+constexpr int kChunk = 16;        // steps whose loss sums and bias corrections are formed together
 
+struct __align__(16) TrainLds {
+  Net N;
+  uint16_t w2[hm::kHid * hm::kStride];   // W2 [in][out], for the input gradients
+  uint16_t w3[hm::kHid * hm::kOut];      // W3 [in][out]
+  uint16_t x[2][kBatch * hm::kIn];       // this batch and the next: [sample][feature]
+  uint16_t xT[2][hm::kIn * kRow];        // [feature][sample]
+  uint16_t h1T[hm::kHid * kRow], h2T[hm::kHid * kRow];  // hidden layers, [unit][sample]
+  uint16_t g1T[hm::kHid * kRow], g2T[hm::kHid * kRow];  // their gradients
+  uint16_t dyT[hm::kOut * kRow];
+  float dyf[hm::kOut][kBatch + 4];
+  float t[2][kBatch * hm::kOut];
+  float err[kChunk][kBatch * hm::kOut + 1];
+  double bc[2 * kChunk][2];              // 1/(1 - beta^t) of two chunks
+};
+
+// sum of a row of 128 BF16 values in order
+__device__ __forceinline__ float row_sum(const uint16_t* row)
+{
+  float s = 0.0f;
+#pragma unroll
+  for (int c = 0; c < kBatch / 8; c++) {
+    const uint4 v = ((const uint4*)row)[c];
+    const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      s += __uint_as_float(u[i] << 16);
+      s += __uint_as_float(u[i] & 0xffff0000u);
+    }
+  }
+  return s;
+}
+
+// A step is two phases with one barrier after each.  First each wave carries
+// its 16 samples forward and back through the network in registers (hm::layer)
+// and leaves the layers and their gradients transposed, sample fastest, in LDS;
+// then 24 products over the 128 samples (16 of dW2, 4 of dW1, 4 of dW3), three
+// a wave, the bias sums on one wave each, and Adam: parameters and moments stay
+// in their lane's registers for the whole launch, LDS gets the BF16 images.
+// The next batch's rows are fetched during the first phase and put into LDS in
+// the second.  One compute unit works, so a step is bound by its issue slots
+// (the hidden layers' 256 tanhs and Adam's 100 updates a wave) and by the
+// latency of the chain through the two phases.
+// 2000 steps over 2^18 pairs: 46 us a step with a 4-wave block that kept
+// every layer in LDS at a stride of 64 (rows on one bank, two bytes a load) and
+// the parameters in memory, 8.4 now.
+template <bool UPDATE>
+__global__ __launch_bounds__(kTrainBlock) void k_mlp_train(TrainArgs a)
+{
+  __shared__ TrainLds S;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, r = l & 15, q = l >> 4;
-  stage_weights(a.wbf, a.w32, sW, sBias);
-  for (int e = tid; e < kBatch * hm::kOutPad; e += kBlock) sDY[e] = 0;
+  stage_net(a.wbf, a.w32, S.N);
+
+  // ---- the parameters this lane owns ----
+  // W2 tiles 2w, 2w + 1: (in, out) = (16 (w/2) + 4 q + i, 16 (2 w % 4 + u) + r);
+  // waves 0-3 W3: (in, out) = (16 w + 4 q + i, r), r < 2;
+  // waves 4-7 W1: (feature, unit) = (4 q + i, 16 (w - 4) + r), q < 2;
+  // waves 1, 2, 3: the biases of layers 1, 2, 3, one a lane
+  const int in2 = 16 * (w >> 1) + 4 * q, out2 = 16 * (2 * w & 3) + r;
+  const bool own3 = w < 4 && r < hm::kOut, own1 = w >= 4 && q < 2;
+  const int off = w < 4 ? hm::kOffW3 + (16 * w + 4 * q) * hm::kOut + r : hm::kOffW1 + 4 * q * hm::kHid + 16 * (w - 4) + r;
+  const int inc = w < 4 ? hm::kOut : hm::kHid;
+  const bool ownb = w == 1 || w == 2 || (w == 3 && l < hm::kOut);
+  const int offb = w == 1 ? hm::kOffB1 + l : w == 2 ? hm::kOffB2 + l : hm::kOffB3 + l;
+  float w2[2][4], m2[2][4], v2[2][4], wo[4], mo[4], vo[4], wb = 0.f, mb = 0.f, vb = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int e = hm::kOffW2 + (in2 + i) * hm::kHid + out2 + 16 * u;
+      w2[u][i] = a.w32[e];
+      m2[u][i] = a.am[e];
+      v2[u][i] = a.av[e];
+      S.w2[(in2 + i) * hm::kStride + out2 + 16 * u] = hm::f2bf(w2[u][i]);
+    }
+    wo[i] = mo[i] = vo[i] = 0.f;
+    if (own3 || own1) {
+      wo[i] = a.w32[off + i * inc];
+      mo[i] = a.am[off + i * inc];
+      vo[i] = a.av[off + i * inc];
+    }
+    if (own3) S.w3[(16 * w + 4 * q + i) * hm::kOut + r] = hm::f2bf(wo[i]);
+  }
+  if (ownb) {
+    wb = a.w32[offb];
+    mb = a.am[offb];
+    vb = a.av[offb];
+  }
+
+  // ---- the batch: sample tid - 384 in waves 6 and 7, a step ahead ----
+  const int bs = tid - (kTrainBlock - kBatch);
+  float fx[hm::kIn], ft[hm::kOut];
+  long pos = 0, sidx = 0;
+  const long hop = kBatch % a.nidx;
+  auto next_index = [&]() {  // out-of-range indices are rejected on the host
+    sidx = a.idx[pos];
+    if (sidx < 0 || sidx >= a.nx) sidx = 0;
+    pos += hop;
+    if (pos >= a.nidx) pos -= a.nidx;
+  };
+  auto fetch = [&]() {
+#pragma unroll
+    for (int k = 0; k < hm::kIn; k++) fx[k] = a.X[sidx * hm::kIn + k];
+#pragma unroll
+    for (int o = 0; o < hm::kOut; o++) ft[o] = a.T[sidx * hm::kOut + o];
+  };
+  auto stage = [&](int b) {
+    v4f lo, hi;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      lo[k] = (fx[k] - a.norm[k]) * a.norm[hm::kIn + k];
+      hi[k] = (fx[4 + k] - a.norm[4 + k]) * a.norm[hm::kIn + 4 + k];
+    }
+    const v4s xl = hm::f2bf4(lo), xh = hm::f2bf4(hi);
+    *(v4s*)&S.x[b][bs * hm::kIn] = xl;
+    *(v4s*)&S.x[b][bs * hm::kIn + 4] = xh;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      S.xT[b][k * kRow + bs] = (uint16_t)xl[k];
+      S.xT[b][(4 + k) * kRow + bs] = (uint16_t)xh[k];
+    }
+#pragma unroll
+    for (int o = 0; o < hm::kOut; o++)
+      S.t[b][bs * hm::kOut + o] = (ft[o] - a.norm[2 * hm::kIn + o]) / a.norm[2 * hm::kIn + hm::kOut + o];
+  };
+  auto corrections = [&](int step) {  // lane j: those of step + j
+    if (l < kChunk) {
+      const float t = (float)(a.t0 + step + l + 1);
+      S.bc[(step + l) % (2 * kChunk)][0] = 1.0 / (1.0f - powf(a.beta1, t));
+      S.bc[(step + l) % (2 * kChunk)][1] = 1.0 / (1.0f - powf(a.beta2, t));
+    }
+  };
+  if (bs >= 0) {
+    pos = (a.first + bs) % a.nidx;
+    next_index();
+    fetch();
+    next_index();
+    stage(0);
+  }
+  if (w == 0) corrections(0);
   float loss_acc = 0.0f;
   __syncthreads();
 
   for (int step = 0; step < a.nsteps; step++) {
-    // ---- batch ----
-    if (tid < kBatch) {
-      const long pos = (a.first + (long)step * kBatch + tid) % a.nidx;
-      long sidx = a.idx[pos];
-      if (sidx < 0 || sidx >= a.nx) sidx = 0;  // out-of-range indices are rejected on the host
-#pragma unroll
-      for (int k = 0; k < hm::kIn; k++)
-        sX[tid * hm::kInPad + k] = hm::f2bf((a.X[sidx * hm::kIn + k] - a.norm[k]) * a.norm[hm::kIn + k]);
-#pragma unroll
-      for (int k = hm::kIn; k < hm::kInPad; k++) sX[tid * hm::kInPad + k] = 0;
-#pragma unroll
-      for (int o = 0; o < hm::kOut; o++)
-        sT[tid * 2 + o] = (a.T[sidx * 2 + o] - a.norm[2 * hm::kIn + o]) / a.norm[2 * hm::kIn + hm::kOut + o];
+    const int b = step & 1, slot = step % kChunk;
+    if (bs >= 0) {
+      fetch();
+      next_index();
     }
-    __syncthreads();
-    // ---- layer 1 ----
-    for (int t = w * 8; t < w * 8 + 8; t++) {
-      const int mt = t >> 2, nt = t & 3;
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      acc = hm::mma16(sX + mt * 16 * hm::kInPad, hm::kInPad, 1, sW + hm::kBfW1 + nt * 16, hm::kHid, 1, hm::kInPad,
-                      acc);
+    // ---- this wave's 16 samples, forward ----
+    const int m = 16 * w + r;  // the lane's sample
+    v4s x = hm::frag(&S.x[b][m * hm::kIn + 4 * (q & 1)]), h1[4], h2[4], g2[4];
+    if (q > 1) x = (v4s){0, 0, 0, 0};
+    auto put = [&](uint16_t* T, int t, v4s v) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int m = mt * 16 + 4 * q + i, n = nt * 16 + r;
-        sH1[m * hm::kHid + n] = hm::f2bf(tanhf(acc[i] + sBias[n]));
+      for (int i = 0; i < 4; i++) T[(16 * t + 4 * q + i) * kRow + m] = (uint16_t)v[i];
+    };
+    hm::layer1(x, S.N.w + hm::kBfW1, S.N.b, h1);
+    hm::layer<4>(h1, S.N.w + hm::kBfW2, hm::kStride, S.N.b + hm::kHid, h2);
+    const v4f y = hm::layer3(h2, S.N.w + hm::kBfW3);
+    // ---- the loss and its gradient: lanes q = 0, outputs in elements 0 and 1 ----
+    v4f dyv = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int o = 0; o < hm::kOut; o++) {
+      const float d = y[o] + S.N.b[2 * hm::kHid + o] - S.t[b][m * hm::kOut + o];
+      dyv[o] = d * (2.0f / (kBatch * hm::kOut));
+      if (q == 0) {
+        S.err[slot][m * hm::kOut + o] = d * d;
+        S.dyf[o][m] = dyv[o];
       }
     }
-    __syncthreads();
-    // ---- layer 2 ----
-    for (int t = w * 8; t < w * 8 + 8; t++) {
-      const int mt = t >> 2, nt = t & 3;
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      acc = hm::mma16(sH1 + mt * 16 * hm::kHid, hm::kHid, 1, sW + hm::kBfW2 + nt * 16, hm::kHid, 1, hm::kHid, acc);
+    v4s dy = hm::f2bf4(dyv);
+    if (q > 0) dy = (v4s){0, 0, 0, 0};
+    else {
+      S.dyT[m] = (uint16_t)dy[0];
+      S.dyT[kRow + m] = (uint16_t)dy[1];
+    }
+    // ---- back: dH2 = dY W3^T, dH1 = dZ2 W2^T ----
+    auto through_tanh = [&](v4f g, v4s h) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int m = mt * 16 + 4 * q + i, n = nt * 16 + r;
-        sH2[m * hm::kHid + n] = hm::f2bf(tanhf(acc[i] + sBias[hm::kHid + n]));
+        const float hf = hm::bf2f((uint16_t)h[i]);
+        g[i] = g[i] * (1.0f - hf * hf);
       }
+      return hm::f2bf4(g);
+    };
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const uint32_t pair = *(const uint32_t*)&S.w3[(16 * t + r) * hm::kOut];
+      v4s c = {(short)(pair & 0xffffu), (short)(pair >> 16), 0, 0};
+      if (q > 0) c = (v4s){0, 0, 0, 0};
+      v4f acc = {0.f, 0.f, 0.f, 0.f};
+      acc = hm::mfma(c, dy, acc);
+      g2[t] = through_tanh(acc, h2[t]);
+      put(S.h1T, t, h1[t]);
+      put(S.h2T, t, h2[t]);
+      put(S.g2T, t, g2[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 4; c++) acc = hm::mfma(hm::frag(&S.w2[(16 * t + r) * hm::kStride + 16 * c + 4 * q]), g2[c], acc);
+      put(S.g1T, t, through_tanh(acc, h1[t]));
     }
     __syncthreads();
-    // ---- layer 3 and the loss gradient ----
-    for (int mt = 2 * w; mt < 2 * w + 2; mt++) {
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      acc = hm::mma16(sH2 + mt * 16 * hm::kHid, hm::kHid, 1, sW + hm::kBfW3, hm::kOutPad, 1, hm::kHid, acc);
-      if (r < hm::kOut) {
+    // ---- gradients over the batch ----
+    v4f d2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, dO = {0.f, 0.f, 0.f, 0.f};
+    const uint16_t* ra = w < 4 ? &S.h2T[(16 * w + r) * kRow] : &S.xT[b][(r & 7) * kRow];
+    const uint16_t* rb = w < 4 ? &S.dyT[(r & 1) * kRow] : &S.g1T[(16 * (w - 4) + r) * kRow];
+#pragma unroll
+    for (int c = 0; c < kBatch / 16; c++) {
+      const int k = 16 * c + 4 * q;
+      const v4s h = hm::frag(&S.h1T[(16 * (w >> 1) + r) * kRow + k]);
+      d2[0] = hm::mfma(h, hm::frag(&S.g2T[out2 * kRow + k]), d2[0]);
+      d2[1] = hm::mfma(h, hm::frag(&S.g2T[(out2 + 16) * kRow + k]), d2[1]);
+      dO = hm::mfma(hm::frag(ra + k), hm::frag(rb + k), dO);
+    }
+    float gb = 0.0f;
+    if (w == 1) gb = row_sum(&S.g1T[l * kRow]);
+    else if (w == 2) gb = row_sum(&S.g2T[l * kRow]);
+    else if (w == 3) {
+      if (l < hm::kOut)
+        for (int k = 0; k < kBatch; k++) gb += S.dyf[l][k];
+    } else if (w == 0 && (slot == kChunk - 1 || step == a.nsteps - 1)) {
+      float sl = 0.0f;
+      if (l <= slot)
+        for (int e = 0; e < kBatch * hm::kOut; e++) sl += S.err[l][e];
+      for (int j = 0; j <= slot; j++) loss_acc += __shfl(sl, j) / (kBatch * hm::kOut);
+      corrections(step + 1);
+    }
+    // ---- parameter step ----
+    if constexpr (UPDATE) {
+      const double rc1 = S.bc[step % (2 * kChunk)][0], rc2 = S.bc[step % (2 * kChunk)][1];
+      // (float)(m rc) is m / (1 - beta^t) rounded once: a quotient of two 24-bit
+      // numbers is never within 2^-49 of a tie, the product's error is 2^-52
+      auto adam = [&](float& p, float& pm, float& pv, float g) {
+        pm = a.beta1 * pm + (1.0f - a.beta1) * g;
+        pv = a.beta2 * pv + (1.0f - a.beta2) * g * g;
+        p = p - a.lr * (float)(pm * rc1) / (sqrtf((float)(pv * rc2)) + a.eps);
+      };
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        v4f n;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const int m = mt * 16 + 4 * q + i;
-          const float d = acc[i] + sBias[2 * hm::kHid + r] - sT[m * 2 + r];
-          const float dy = d * (2.0f / (kBatch * hm::kOut));
-          sErr[m * 2 + r] = d * d;
-          sDYf[m * 2 + r] = dy;
-          sDY[m * hm::kOutPad + r] = hm::f2bf(dy);
+          adam(w2[u][i], m2[u][i], v2[u][i], d2[u][i]);
+          n[i] = w2[u][i];
+        }
+        const v4s nb = hm::f2bf4(n);
+        *(v4s*)&S.N.w[hm::kBfW2 + (out2 + 16 * u) * hm::kStride + in2] = nb;
+#pragma unroll
+        for (int i = 0; i < 4; i++) S.w2[(in2 + i) * hm::kStride + out2 + 16 * u] = (uint16_t)nb[i];
+      }
+      if (own3 || own1) {
+        v4f n;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          adam(wo[i], mo[i], vo[i], dO[i]);
+          n[i] = wo[i];
+        }
+        const v4s nb = hm::f2bf4(n);
+        if (own3) {
+          *(v4s*)&S.N.w[hm::kBfW3 + r * hm::kStride + 16 * w + 4 * q] = nb;
+#pragma unroll
+          for (int i = 0; i < 4; i++) S.w3[(16 * w + 4 * q + i) * hm::kOut + r] = (uint16_t)nb[i];
+        } else {
+          *(v4s*)&S.N.w[hm::kBfW1 + (16 * (w - 4) + r) * hm::kIn + 4 * q] = nb;
         }
       }
-    }
-    __syncthreads();
-    // ---- dW3 = H2^T dY (one 16x16 tile per wave); dH2 = dY W3^T ----
-    v4f g3 = {0.f, 0.f, 0.f, 0.f};
-    g3 = hm::mma16(sH2 + w * 16, 1, hm::kHid, sDY, hm::kOutPad, 1, kBatch, g3);
-    for (int t = w * 8; t < w * 8 + 8; t++) {
-      const int mt = t >> 2, nt = t & 3;
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      acc = hm::mma16(sDY + mt * 16 * hm::kOutPad, hm::kOutPad, 1, sW + hm::kBfW3 + nt * 16 * hm::kOutPad, 1,
-                      hm::kOutPad, hm::kOutPad, acc);
+      if (ownb) {
+        adam(wb, mb, vb, gb);
+        S.N.b[hm::kHid * (w - 1) + l] = wb;
+      }
+    } else {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int m = mt * 16 + 4 * q + i, n = nt * 16 + r;
-        const float h = hm::bf2f(sH2[m * hm::kHid + n]);
-        sG2[m * hm::kHid + n] = hm::f2bf(acc[i] * (1.0f - h * h));
-      }
-    }
-    __syncthreads();
-    // ---- dW2 = H1^T dZ2 (four tiles per wave); dH1 = dZ2 W2^T ----
-    v4f g2[4];
-    for (int u = 0; u < 4; u++) {
-      const int t = 4 * w + u, mt = t >> 2, nt = t & 3;
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      g2[u] = hm::mma16(sH1 + mt * 16, 1, hm::kHid, sG2 + nt * 16, hm::kHid, 1, kBatch, acc);
-    }
-    for (int t = w * 8; t < w * 8 + 8; t++) {
-      const int mt = t >> 2, nt = t & 3;
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      acc = hm::mma16(sG2 + mt * 16 * hm::kHid, hm::kHid, 1, sW + hm::kBfW2 + nt * 16 * hm::kHid, 1, hm::kHid, hm::kHid,
-                      acc);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int m = mt * 16 + 4 * q + i, n = nt * 16 + r;
-        const float h = hm::bf2f(sH1[m * hm::kHid + n]);
-        sG1[m * hm::kHid + n] = hm::f2bf(acc[i] * (1.0f - h * h));
+        for (int u = 0; u < 2; u++) a.grad_out[hm::kOffW2 + (in2 + i) * hm::kHid + out2 + 16 * u] = d2[u][i];
+        if (own3 || own1) a.grad_out[off + i * inc] = dO[i];
       }
+      if (ownb) a.grad_out[offb] = gb;
     }
-    __syncthreads();
-    // ---- dW1 = X^T dZ1 (one tile per wave) and the bias gradients ----
-    v4f g1 = {0.f, 0.f, 0.f, 0.f};
-    g1 = hm::mma16(sX, 1, hm::kInPad, sG1 + w * 16, hm::kHid, 1, kBatch, g1);
-    float gb = 0.0f;  // bias gradient owned by this thread
-    if (tid < hm::kHid) {
-      for (int m = 0; m < kBatch; m++) gb += hm::bf2f(sG1[m * hm::kHid + tid]);
-    } else if (tid < 2 * hm::kHid) {
-      for (int m = 0; m < kBatch; m++) gb += hm::bf2f(sG2[m * hm::kHid + tid - hm::kHid]);
-    } else if (tid < 2 * hm::kHid + hm::kOut) {
-      for (int m = 0; m < kBatch; m++) gb += sDYf[m * 2 + tid - 2 * hm::kHid];
-    }
-    if (tid == 0) {
-      float sl = 0.0f;
-      for (int e = 0; e < kBatch * hm::kOut; e++) sl += sErr[e];
-      loss_acc += sl / (kBatch * hm::kOut);
-    }
-    __syncthreads();  // every read of the current weights is done
-    // ---- parameter step ----
-    const long tstep = a.t0 + step + 1;
-    const float bc1 = 1.0f - powf(a.beta1, (float)tstep), bc2 = 1.0f - powf(a.beta2, (float)tstep);
-    auto apply = [&](int pidx, float g) {
-      if (!a.update) { a.grad_out[pidx] = g; return a.w32[pidx]; }
-      const float m = a.beta1 * a.am[pidx] + (1.0f - a.beta1) * g;
-      const float v = a.beta2 * a.av[pidx] + (1.0f - a.beta2) * g * g;
-      a.am[pidx] = m;
-      a.av[pidx] = v;
-      const float wn = a.w32[pidx] - a.lr * (m / bc1) / (sqrtf(v / bc2) + a.eps);
-      a.w32[pidx] = wn;
-      return wn;
-    };
-    if (r < hm::kOut) {  // W3 tile of wave w: rows h = 16w + 4q + i
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int h = w * 16 + 4 * q + i;
-        const float wn = apply(hm::kOffW3 + h * hm::kOut + r, g3[i]);
-        sW[hm::kBfW3 + h * hm::kOutPad + r] = hm::f2bf(wn);
-      }
-    }
-    for (int u = 0; u < 4; u++) {
-      const int t = 4 * w + u, mt = t >> 2, nt = t & 3;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int hin = mt * 16 + 4 * q + i, hout = nt * 16 + r;
-        const float wn = apply(hm::kOffW2 + hin * hm::kHid + hout, g2[u][i]);
-        sW[hm::kBfW2 + hin * hm::kHid + hout] = hm::f2bf(wn);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int f = 4 * q + i, h = w * 16 + r;
-      if (f < hm::kIn) {
-        const float wn = apply(hm::kOffW1 + f * hm::kHid + h, g1[i]);
-        sW[hm::kBfW1 + f * hm::kHid + h] = hm::f2bf(wn);
-      }
-    }
-    if (tid < hm::kHid) sBias[tid] = apply(hm::kOffB1 + tid, gb);
-    else if (tid < 2 * hm::kHid) sBias[tid] = apply(hm::kOffB2 + tid - hm::kHid, gb);
-    else if (tid < 2 * hm::kHid + hm::kOut) sBias[tid] = apply(hm::kOffB3 + tid - 2 * hm::kHid, gb);
+    if (bs >= 0) stage(b ^ 1);
     __syncthreads();
   }
-  // the BF16 images of the final weights
-  for (int e = tid; e < hm::kNBf; e += kBlock) a.wbf[e] = sW[e];
-  if (tid == 0) a.loss_out[0] = loss_acc / (a.nsteps > 0 ? a.nsteps : 1);
+  if (tid == 0) a.loss_out[0] = loss_acc / a.nsteps;
+  if constexpr (UPDATE) {
+    // the parameters, their moments and the BF16 images back to memory
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int e = hm::kOffW2 + (in2 + i) * hm::kHid + out2 + 16 * u;
+        a.w32[e] = w2[u][i];
+        a.am[e] = m2[u][i];
+        a.av[e] = v2[u][i];
+      }
+      if (own3 || own1) {
+        a.w32[off + i * inc] = wo[i];
+        a.am[off + i * inc] = mo[i];
+        a.av[off + i * inc] = vo[i];
+      }
+    }
+    if (ownb) {
+      a.w32[offb] = wb;
+      a.am[offb] = mb;
+      a.av[offb] = vb;
+    }
+    for (int e = tid; e < hm::kNBf / 8; e += kTrainBlock) ((uint4*)a.wbf)[e] = ((const uint4*)S.N.w)[e];
+  }
 }
 
 // ---------------------------------------------------------------------------
 // inference
 // ---------------------------------------------------------------------------
-struct Fwd {
-  uint16_t sW[hm::kNBf];
-  float sBias[2 * hm::kHid + hm::kOut];
-  uint16_t bufA[kWaves][64 * hm::kHid];
-  uint16_t bufB[kWaves][64 * hm::kHid];
-  float y[kWaves][64 * 2];
-};
-
 // X[n][8] raw features -> Y[n][2] raw predictions (log W'/D, log u~^2)
 __global__ __launch_bounds__(kBlock) void k_mlp_forward(const uint16_t* __restrict__ wbf,
                                                         const float* __restrict__ w32, const float* __restrict__ norm,
                                                         const float* __restrict__ X, float* __restrict__ Y, long n)
 {
-  __shared__ Fwd S;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  stage_weights(wbf, w32, S.sW, S.sBias);
-  const long z = (long)blockIdx.x * kBlock + threadIdx.x;
-#pragma unroll
-  for (int k = 0; k < hm::kInPad; k++) {
-    float v = 0.0f;
-    if (z < n && k < hm::kIn) v = (X[z * hm::kIn + k] - norm[k]) * norm[hm::kIn + k];
-    S.bufA[w][l * hm::kInPad + k] = hm::f2bf(v);
-  }
+  __shared__ Net N;
+  __shared__ uint16_t xs[kWaves][64][hm::kIn];
+  stage_net(wbf, w32, N);
   __syncthreads();
-  wave_forward(S.bufA[w], S.bufB[w], S.sW, S.sBias, S.y[w]);
+  const long z = (long)blockIdx.x * kBlock + threadIdx.x;
+  float f[hm::kIn], y[hm::kOut];
+#pragma unroll
+  for (int k = 0; k < hm::kIn; k++) f[k] = z < n ? X[z * hm::kIn + k] : 0.0f;
+  wave_net<hm::kOut>(f, z < n, norm, N, xs[threadIdx.x >> 6], y);
   if (z < n) {
 #pragma unroll
     for (int o = 0; o < hm::kOut; o++)
-      Y[z * 2 + o] = S.y[w][l * 2 + o] * norm[2 * hm::kIn + hm::kOut + o] + norm[2 * hm::kIn + o];
+      Y[z * 2 + o] = y[o] * norm[2 * hm::kIn + hm::kOut + o] + norm[2 * hm::kIn + o];
   }
 }
 
@@ -408,12 +534,14 @@ __global__ __launch_bounds__(kBlock) void k_invert_batch_mlp(const uint16_t* __r
                                                              long n, double gam, double gammafail,
                                                              unsigned long long* __restrict__ nfallback)
 {
-  __shared__ Fwd S;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  stage_weights(wbf, w32, S.sW, S.sBias);
+  __shared__ Net N;
+  __shared__ uint16_t xs[kWaves][64][hm::kIn];
+  stage_net(wbf, w32, N);
+  __syncthreads();
   const long z = (long)blockIdx.x * kBlock + threadIdx.x;
   const bool act = z < n;
   double D = 1.0;
+  float y[1];
   {
     float f[hm::kIn] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (act) {
@@ -429,18 +557,11 @@ __global__ __launch_bounds__(kBlock) void k_invert_batch_mlp(const uint16_t* __r
       hm::features(s, f);
       D = s.D;
     }
-#pragma unroll
-    for (int k = 0; k < hm::kInPad; k++) {
-      float v = 0.0f;
-      if (act && k < hm::kIn) v = (f[k] - norm[k]) * norm[hm::kIn + k];
-      S.bufA[w][l * hm::kInPad + k] = hm::f2bf(v);
-    }
+    wave_net<1>(f, act, norm, N, xs[threadIdx.x >> 6], y);
   }
-  __syncthreads();
-  wave_forward(S.bufA[w], S.bufB[w], S.sW, S.sBias, S.y[w]);
   int fb = 0;
   if (act) {
-    const float y0 = S.y[w][l * 2] * norm[2 * hm::kIn + hm::kOut] + norm[2 * hm::kIn];
+    const float y0 = y[0] * norm[2 * hm::kIn + hm::kOut] + norm[2 * hm::kIn];
     const double seed = D * exp((double)fminf(fmaxf(y0, -60.0f), 60.0f));
     hd::Geom g;
     hd::load_geom(geom, z, n, g);
@@ -527,14 +648,16 @@ __global__ __launch_bounds__(kBlock) void k_invert_grid_mlp(const uint16_t* __re
                                                             double* __restrict__ fx_p0, double* __restrict__ fx_pfl,
                                                             uint8_t* __restrict__ fx_flag)
 {
-  __shared__ Fwd S;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  stage_weights(wbf, w32, S.sW, S.sBias);
+  __shared__ Net N;
+  __shared__ uint16_t xs[kWaves][64][hm::kIn];
+  stage_net(wbf, w32, N);
+  __syncthreads();
   const int lb = hk::xcd_tile(blockIdx.x, gridDim.x);
   const int t = lb * kBlock + threadIdx.x;
   const bool act = t < d.n1 * d.n2 * d.n3;
   long o = 0, pp = 0;
   double D = 1.0;
+  float y[1];
   {
     float f[hm::kIn] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (act) {
@@ -554,18 +677,11 @@ __global__ __launch_bounds__(kBlock) void k_invert_grid_mlp(const uint16_t* __re
       hm::features(s, f);
       D = s.D;
     }
-#pragma unroll
-    for (int k = 0; k < hm::kInPad; k++) {
-      float v = 0.0f;
-      if (act && k < hm::kIn) v = (f[k] - norm[k]) * norm[hm::kIn + k];
-      S.bufA[w][l * hm::kInPad + k] = hm::f2bf(v);
-    }
+    wave_net<1>(f, act, norm, N, xs[threadIdx.x >> 6], y);
   }
-  __syncthreads();
-  wave_forward(S.bufA[w], S.bufB[w], S.sW, S.sBias, S.y[w]);
   int ns = 0, nf = 0, fb = 0;
   if (act) {
-    const float y0 = S.y[w][l * 2] * norm[2 * hm::kIn + hm::kOut] + norm[2 * hm::kIn];
+    const float y0 = y[0] * norm[2 * hm::kIn + hm::kOut] + norm[2 * hm::kIn];
     const double seed = D * exp((double)fminf(fmaxf(y0, -60.0f), 60.0f));
     double Uz[HARM_NPR];
 #pragma unroll
@@ -712,8 +828,8 @@ extern "C" harm_status harm_mlp_train(harm_mlp* m, const float* X, const float* 
   a.w32 = m->w32; a.am = m->adam_m; a.av = m->adam_v; a.wbf = m->wbf; a.norm = m->norm;
   a.X = X; a.T = T; a.nx = (long)nx; a.idx = order; a.nidx = (long)norder; a.first = (long)first; a.nsteps = nsteps;
   a.t0 = (long)m->t;
-  a.lr = lr; a.beta1 = 0.9f; a.beta2 = 0.999f; a.eps = 1e-8f; a.update = 1; a.grad_out = nullptr; a.loss_out = m->loss;
-  hipLaunchKernelGGL(k_mlp_train, dim3(1), dim3(kBlock), 0, (hipStream_t)stream, a);
+  a.lr = lr; a.beta1 = 0.9f; a.beta2 = 0.999f; a.eps = 1e-8f; a.grad_out = nullptr; a.loss_out = m->loss;
+  hipLaunchKernelGGL(k_mlp_train<true>, dim3(1), dim3(kTrainBlock), 0, (hipStream_t)stream, a);
   HH_TRY(hh::check_launch("k_mlp_train"));
   m->t += nsteps;
   if (loss) {
@@ -730,8 +846,8 @@ extern "C" harm_status harm_mlp_grad(harm_mlp* m, const float* X, const float* T
   TrainArgs a{};
   a.w32 = m->w32; a.am = m->adam_m; a.av = m->adam_v; a.wbf = m->wbf; a.norm = m->norm;
   a.X = X; a.T = T; a.nx = (long)nx; a.idx = order; a.nidx = kBatch; a.first = 0; a.nsteps = 1; a.t0 = 0;
-  a.lr = 0.0f; a.beta1 = 0.9f; a.beta2 = 0.999f; a.eps = 1e-8f; a.update = 0; a.grad_out = grad; a.loss_out = m->loss;
-  hipLaunchKernelGGL(k_mlp_train, dim3(1), dim3(kBlock), 0, nullptr, a);
+  a.lr = 0.0f; a.beta1 = 0.9f; a.beta2 = 0.999f; a.eps = 1e-8f; a.grad_out = grad; a.loss_out = m->loss;
+  hipLaunchKernelGGL(k_mlp_train<false>, dim3(1), dim3(kTrainBlock), 0, nullptr, a);
   HH_TRY(hh::check_launch("k_mlp_train"));
   HH_HIP(hipDeviceSynchronize());
   if (loss) HH_HIP(hipMemcpy(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost));
