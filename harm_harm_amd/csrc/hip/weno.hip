@@ -119,12 +119,20 @@ __device__ __forceinline__ double limit_weight_q(double w)
   return w < w1 ? 0.0 : r;
 }
 
-// Whether the indicator sum n of a zone lies in the range of the unscaled
-// quotients (dphys.h).  Its terms are then at least 1e-28 of it: each holds
-// WENO_EPSILON (1.2e-26) times the window's sum of squares, and n is at most
-// 60 times that sum.  Outside (fields that have decayed to 1e-100, infinities
-// and NaN) the plain divisions are used.
-__device__ __forceinline__ bool plain_range(double n) { return n > 1e-200 && n < 1e200; }
+// Whether the unscaled quotients (dphys.h) of the indicators by their sum n can
+// be used, with the factor sc for both.  Above 1e-200 the indicators are at
+// least 1e-28 of n: each holds WENO_EPSILON (1.2e-26) times the window's sum of
+// squares, and n is at most 60 times that sum.  Below (a field's front falls by
+// some 1e-7 a zone, so most waves at it hold such a zone) the indicators and n,
+// which is at least DBL_MIN, are brought up by a power of two, which leaves
+// their quotients as they are (with the plain divisions there 30 steps of the
+// 256x128x64 torus took 213.7 ms, so 206.1).  Beyond 1e200, infinities and NaN take the plain
+// divisions.
+__device__ __forceinline__ bool unscaled(double n, double& sc)
+{
+  sc = n < 1e-200 ? 0x1p600 : 1.0;
+  return n < 1e200;
+}
 
 // The weights of the two uniform cases, formed by the same operations as the
 // general code below (constant-folded, round to nearest):
@@ -162,12 +170,12 @@ __device__ __forceinline__ void weights3(const double* u, double* w)
   s0 += err;
   s1 += err;
   s2 += err;
-  double n = sym3(s0, s1, s2) + kMinNum;
-  if (plain_range(n)) {
-    // the quotients below stay between 1e-53 and 1e52 (s/n >= 1e-28, t between
-    // WENO_EPSILON^2 = 1.5e-52 and about 1)
-    const hd::Recip rn = hd::recip(n);
-    double t0 = hd::quot(s0, rn) + kWeps, t1 = hd::quot(s1, rn) + kWeps, t2 = hd::quot(s2, rn) + kWeps;
+  double n = sym3(s0, s1, s2) + kMinNum, sc;
+  if (unscaled(n, sc)) {
+    // the quotients below stay between 1e-53 and 1e52 (t between WENO_EPSILON^2
+    // = 1.5e-52 and about 1)
+    const hd::Recip rn = hd::recip(n * sc);
+    double t0 = hd::quot(s0 * sc, rn) + kWeps, t1 = hd::quot(s1 * sc, rn) + kWeps, t2 = hd::quot(s2 * sc, rn) + kWeps;
     t0 *= t0;
     t1 *= t1;
     t2 *= t2;
@@ -210,10 +218,10 @@ __device__ __forceinline__ void weights2(const double* u, double* L2, double* R2
   const double err = sym3(u[-1] * u[-1], u[0] * u[0], u[1] * u[1]) * kWeps;
   s0 += err;
   s1 += err;
-  double n = sym2(s0, s1) + kMinNum;
-  if (plain_range(n)) {  // as in weights3
-    const hd::Recip rn = hd::recip(n);
-    double t0 = hd::quot(s0, rn) + kWeps, t1 = hd::quot(s1, rn) + kWeps;
+  double n = sym2(s0, s1) + kMinNum, sc;
+  if (unscaled(n, sc)) {  // as in weights3
+    const hd::Recip rn = hd::recip(n * sc);
+    double t0 = hd::quot(s0 * sc, rn) + kWeps, t1 = hd::quot(s1 * sc, rn) + kWeps;
     t0 *= t0;
     t1 *= t1;
     const double w0 = hd::inv1(t0), w1 = hd::inv1(t1);
