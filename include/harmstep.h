@@ -173,8 +173,9 @@ enum { HARM_ARR_P = 0,     /* pglobal (primitives)                           */
        HARM_ARR_F1 = 6, HARM_ARR_F2 = 7, HARM_ARR_F3 = 8, /* face fluxes     */
        HARM_NARR = 9 };
 /* Both copy the whole storage box over PCIe and convert between this layout
- * and the device planes with a kernel (a staging buffer of the box's size is
- * allocated by the first call); both return when the copy is complete. */
+ * and the device planes with a kernel (a device buffer of the box's size and up
+ * to three pinned pieces of at most 16 MB are allocated by the first calls and
+ * kept with the handle); both return when the copy is complete. */
 harm_status harm_set_array(harm_handle* h, int32_t which, const double* host_aos);
 harm_status harm_get_array(harm_handle* h, int32_t which, double* host_aos);
 /* pflag[k][j][i] (FLAGUTOPRIMFAIL) over the storage box */
@@ -320,7 +321,8 @@ enum { HARM_DUMP_NCOL = 72, HARM_GDUMP_NCOL = 126 };
  * its arrays on the first call. */
 harm_status harm_currents(harm_handle* h, int32_t at_start);
 /* Replaces dump_content() over the grid: rows[z * HARM_DUMP_NCOL + c] from
- * primitives `which` (HARM_ARR_*) on the host. */
+ * primitives `which` (HARM_ARR_*) on the host.  Built on the device 65536 zones
+ * at a time (up to 37.7 MB, kept with the handle from the first call on). */
 harm_status harm_dump_columns(harm_handle* h, int32_t which, double* rows);
 /* No counterpart in the reference: harm_dump_columns for callers that cannot
  * allocate (code under graph capture, tight serving loops, harnesses that
