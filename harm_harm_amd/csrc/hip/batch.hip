@@ -129,13 +129,8 @@ extern "C" harm_status harm_invert_batch(const double* U, const double* geom, do
   if (n <= 0 || !U || !geom || !p_inout || !pflag) return hh::set_error(HARM_EINVAL, "invert_batch: bad arguments");
   const long nr = (long)((n + kBlock - 1) / kBlock);
   if (nr > 0x7fffffffL) return hh::set_error(HARM_EINVAL, "invert_batch: n too large");
-  // The chip holds kResident blocks (four waves a SIMD), so the rounds a block
-  // takes are chosen for whole passes of that many blocks with at most 16
-  // rounds each; up to kResident runs of 256 zones every run is a block of its
-  // own and its solves run through (their length is the call's latency).
-  constexpr long kResident = 1024;
-  const long passes = (nr + kResident * 16 - 1) / (kResident * 16);
-  const int rounds = (int)((nr + kResident * passes - 1) / (kResident * passes));
+  constexpr long kResident = 1024;  // blocks the chip holds (four waves a SIMD)
+  const int rounds = hh::inversion_rounds(nr, kResident);
   const long nb = (nr + rounds - 1) / rounds;
   hipLaunchKernelGGL(k_invert_batch, dim3((unsigned)nb), dim3(kBlock), 0, (hipStream_t)stream, U, geom, p_inout, pflag,
                      niter, (long)n, gam, gammafail, rounds);

@@ -41,7 +41,13 @@ __device__ __forceinline__ void fix_delta_to(const Params& P, const Geom& G, con
 // Returns the flag; the floors' Newton strokes are added to ns.  *changed
 // reports whether pz differs from pf, which is not written.  The geometry and
 // the primitives are read again after the solve (an L1/L2 hit) instead of
-// holding 86 registers through the Newton iterations.  DIAG: as invert_zone.
+// holding 86 registers through the Newton iterations.
+// DIAG (final substep): the states each fix started from are kept for the
+// energy-file accounting (diag_fixup, fixup.c:220): fx_flag[o] gets bit 0
+// when the floors changed the zone (fixup.c:766) and bit 1 when the gamma
+// limit did (fixup.c:784); fx_p0 (SoA, stride ncell) then holds the
+// primitives ahead of both fixes and, when the floors changed them, fx_pfl
+// the primitives after the floors.  Only fixed zones store their states.
 template <bool DIAG = false>
 __device__ __forceinline__ int floors_zone(const Dims& d, const Params& P, const double* __restrict__ gcent,
                                            const double* __restrict__ floors, const double* pf,
@@ -128,77 +134,59 @@ __device__ __forceinline__ int floors_zone(const Dims& d, const Params& P, const
   return fl;
 }
 
-// One zone: conserved Uz (with gdet) in registers, the guess read from pg at
-// offset o, the result written to pf and pflag.  Returns the flag; the Newton
-// stroke count is added to ns.
+// One zone's solve: conserved U (with gdet) and the guess pg read at offset o,
+// the result written to pf and pflag.  Returns the flag; the Newton stroke
+// count is added to ns.  The floors and the Lorentz-factor limit of the final
+// substep are a pass of their own (floors_zone), so that this solve keeps its
+// registers.
 //
 // SEEDED: the Newton solve starts from W' = wp_seed (the learned guess); when
 // that solve fails, the zone is solved again from the primitives' guess as
 // the plain inversion does (Newton from the previous primitives is the
 // fallback and decides), and *fellback is set.
-// DIAG (final substep): the states each fix started from are kept for the
-// energy-file accounting (diag_fixup, fixup.c:220): fx_flag[o] gets bit 0
-// when the floors changed the zone (fixup.c:766) and bit 1 when the gamma
-// limit did (fixup.c:784); fx_p0 (SoA, stride ncell) then holds the
-// primitives ahead of both fixes and, when the floors changed them, fx_pfl
-// the primitives after the floors.  Only fixed zones store their states.
-//
-// FLOORS = false: the floors and the Lorentz-factor limit are left to a
-// separate pass over the zones (floors_zone), as the plain grid inversion
-// does on the final substep so that this solve keeps its registers.
-//
-// Ug: the conserved state in global memory (Uz's source, SoA at o); the rare
-// checks and retries after the hot solve read it again rather than keeping
-// Uz in registers through the Newton iterations.
-template <bool SEEDED = false, bool DIAG = false, bool FLOORS = true>
-__device__ __forceinline__ int invert_zone(const Dims& d, const Params& P, double* Uz, const double* __restrict__ Ug,
-                                           const double* __restrict__ pg, double* pf,
-                                           int32_t* __restrict__ pflag, const double* __restrict__ gcent,
-                                           const double* __restrict__ floors, int finalstep, long o, long pp, int& ns,
-                                           double wp_seed = 0.0, int* fellback = nullptr,
-                                           double* __restrict__ fx_p0 = nullptr, double* __restrict__ fx_pfl = nullptr,
-                                           uint8_t* __restrict__ fx_flag = nullptr)
+template <bool SEEDED = false>
+__device__ __forceinline__ int invert_zone(const Dims& d, const Params& P, const double* __restrict__ U,
+                                           const double* __restrict__ pg, double* __restrict__ pf,
+                                           int32_t* __restrict__ pflag, const double* __restrict__ gcent, long o,
+                                           long pp, int& ns, double wp_seed = 0.0, int* fellback = nullptr)
 {
   const long nc = d.ncell;
   Geom G;
-  hd::load_geom(gcent, pp, d.nplane, G);
   double pz[HARM_NPR];
-#pragma unroll
-  for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = pg[pl * nc + o];  // guess: the substep's starting primitives
   bool solved;
-  int fl = hd::utoprimgen(Uz, G, P.gam, P.gammafail, pz, ns, SEEDED ? wp_seed : __builtin_nan(""), 200, &solved);
+  int fl;
+#pragma unroll 1
+  for (int pass = 0;; pass++) {
+    const double *Ur = pass ? hd::fresh(U) : U, *pgr = pass ? hd::fresh(pg) : pg;
+    hd::load_geom(pass ? hd::fresh(gcent) : gcent, pp, d.nplane, G);
+    double Uz[HARM_NPR];
+#pragma unroll
+    for (int pl = 0; pl < HARM_NPR; pl++) {
+      Uz[pl] = Ur[pl * nc + o];
+      pz[pl] = pgr[pl * nc + o];  // guess: the substep's starting primitives
+    }
+    fl = hd::utoprimgen(Uz, G, P.gam, P.gammafail, pz, ns, SEEDED && !pass ? wp_seed : __builtin_nan(""), 200, &solved);
+    if (!SEEDED || pass || fl == 0) break;
+    *fellback = 1;
+  }
   if (!solved) {  // the guess stands (read again rather than kept through the iterations)
     const double* pgr = hd::fresh(pg);
 #pragma unroll
     for (int pl = 0; pl <= HARM_U3; pl++) pz[pl] = pgr[pl * nc + o];
   }
-  if (SEEDED && fl != 0) {
-    *fellback = 1;
-#pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = pg[pl * nc + o];
-    fl = hd::utoprimgen(Uz, G, P.gam, P.gammafail, pz, ns, __builtin_nan(""));
-  }
-  // The geometry is needed again only for the floors below.  Reloading it
-  // through a pointer the compiler cannot see through frees its 54
-  // registers during the Newton iterations (they come back from L1/L2).
-  hd::load_geom(hd::fresh(gcent), pp, d.nplane, G);
   if (hd::needs_after_hot(fl, P.hot2cold, P.checkinv)) {
+    // The rare checks and retries read the state and the geometry again,
+    // through pointers the compiler cannot see through, rather than keeping
+    // 70 registers through the Newton iterations (they come from L1/L2).
+    hd::load_geom(hd::fresh(gcent), pp, d.nplane, G);
     double Ur[HARM_NPR], Ugf[HARM_NPR], p0[HARM_NPR];
 #pragma unroll
     for (int pl = 0; pl < HARM_NPR; pl++) {
-      Ur[pl] = Ug[pl * nc + o];
+      Ur[pl] = U[pl * nc + o];
       p0[pl] = pg[pl * nc + o];
     }
     hd::geometry_free(Ur, G, Ugf);
     fl = hd::after_hot(fl, Ugf, G, P.gam, P.gammafail, p0, pz, ns, P.hot2cold, P.checkinv);
-  }
-  if (FLOORS && finalstep) {
-    bool changed;
-#pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) pf[pl * nc + o] = pz[pl];
-    fl = floors_zone<DIAG>(d, P, gcent, floors, pf, pz, fl, o, pp, ns, &changed, fx_p0, fx_pfl, fx_flag);
-  } else if (FLOORS && DIAG) {
-    fx_flag[o] = 0;
   }
 #pragma unroll
   for (int pl = 0; pl < HARM_NPR; pl++) pf[pl * nc + o] = pz[pl];

@@ -218,13 +218,11 @@ __device__ __forceinline__ void zone_ijk(const Dims& d, int t, int& i, int& j, i
 }
 
 // The step's inversion started from a learned W' (mlp.hip): harm_step's
-// k_invert with the network in front of the Newton solve.
-// With fx_p0, the states the final substep's fixes started from are kept
-// as k_invert<true> keeps them (invert_zone).
+// k_invert with the network in front of the Newton solve (the final substep's
+// floors follow as after k_invert).
 harm_status launch_invert_grid_mlp(const harm_mlp* m, const hd::Dims& d, const Params& P, const double* U,
-                                   const double* pg, double* pf, int32_t* pflag, const double* gcent,
-                                   const double* floors, int finalstep, unsigned long long* di, hipStream_t s,
-                                   double* fx_p0 = nullptr, double* fx_pfl = nullptr, uint8_t* fx_flag = nullptr);
+                                   const double* pg, double* pf, int32_t* pflag, const double* gcent, int finalstep,
+                                   unsigned long long* di, hipStream_t s);
 
 // Energy-file diagnostics (ener.hip).  `part` holds per-block partial sums:
 // at least 4 * ener_part_blocks(d) * 8 doubles.

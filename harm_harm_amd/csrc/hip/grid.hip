@@ -460,11 +460,7 @@ __device__ __forceinline__ void invert_body(Dims d, Params P, const double* __re
     zone_ijk(d, t, i, j, k);
     const long o = hd::cidx(d, i, j, k);
     const long pp = hd::pidx(d, i, j);
-    const long nc = d.ncell;
-    double Uz[HARM_NPR];
-#pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) Uz[pl] = U[pl * nc + o];
-    const int fl = invert_zone<false, false, false>(d, P, Uz, U, pg, pf, pflag, gcent, nullptr, finalstep, o, pp, ns);
+    const int fl = invert_zone(d, P, U, pg, pf, pflag, gcent, o, pp, ns);
     nf = !finalstep && fl > 0;
   }
   newton_counts_to(ns, nf, di);
@@ -1755,20 +1751,19 @@ harm_status enq_invert(harm_handle* h, int which_pb, int which_pf, int finalstep
   prof_begin(h);
   if (h->guess) {
     HH_TRY(launch_invert_grid_mlp(h->guess, d, h->P, U, h->arr[which_pb], h->arr[which_pf], h->pflag,
-                                  h->geom[HARM_LOC_CENT], h->floors, finalstep, h->di, h->stream,
-                                  diag ? h->fx_p0 : nullptr, h->fx_pfl, h->fx_flag));
+                                  h->geom[HARM_LOC_CENT], finalstep, h->di, h->stream));
     if (substep_dt) hipLaunchKernelGGL(k_scal_substep_dt, dim3(1), dim3(1), 0, h->stream, h->ds);
   } else {
     hipLaunchKernelGGL(k_invert, dim3(nb + (substep_dt ? 1 : 0)), dim3(kBlock), 0, h->stream, d, h->P, U,
                        h->arr[which_pb], h->arr[which_pf], h->pflag, h->geom[HARM_LOC_CENT], finalstep, h->di,
                        substep_dt ? h->ds : nullptr);
-    if (finalstep && diag)
-      hipLaunchKernelGGL(k_floors<true>, dim3(nb), dim3(kBlock), 0, h->stream, d, h->P, h->arr[which_pf], h->pflag,
-                         h->geom[HARM_LOC_CENT], h->floors, h->di, h->fx_p0, h->fx_pfl, h->fx_flag);
-    else if (finalstep)
-      hipLaunchKernelGGL(k_floors<false>, dim3(nb), dim3(kBlock), 0, h->stream, d, h->P, h->arr[which_pf], h->pflag,
-                         h->geom[HARM_LOC_CENT], h->floors, h->di, nullptr, nullptr, nullptr);
   }
+  if (finalstep && diag)
+    hipLaunchKernelGGL(k_floors<true>, dim3(nb), dim3(kBlock), 0, h->stream, d, h->P, h->arr[which_pf], h->pflag,
+                       h->geom[HARM_LOC_CENT], h->floors, h->di, h->fx_p0, h->fx_pfl, h->fx_flag);
+  else if (finalstep)
+    hipLaunchKernelGGL(k_floors<false>, dim3(nb), dim3(kBlock), 0, h->stream, d, h->P, h->arr[which_pf], h->pflag,
+                       h->geom[HARM_LOC_CENT], h->floors, h->di, nullptr, nullptr, nullptr);
   prof_end(h, HARM_K_INVERT);
   if (diag)
     launch_ener_fix(d, h->P, h->arr[which_pf], h->geom[HARM_LOC_CENT], h->fx_p0, h->fx_pfl, h->fx_flag, h->enpart,

@@ -523,81 +523,142 @@ __global__ __launch_bounds__(kBlock) void k_mlp_forward(const uint16_t* __restri
   }
 }
 
+// One zone's solve from W' = seed, or from the primitives' guess when plain:
+// 0 done, 1 unfinished after `limit` iterations (ns unchanged), 2 the seeded
+// solve failed (its strokes in ns) and the plain guess decides.
+__device__ __forceinline__ int seeded_one(const double* __restrict__ U, const double* __restrict__ geom,
+                                          double* __restrict__ p, int32_t* __restrict__ pflag,
+                                          int32_t* __restrict__ niter, long n, double gam, double gammafail, long z,
+                                          double seed, bool plain, int limit, int& ns)
+{
+  hd::Geom g;
+  hd::load_geom(geom, z, n, g);
+  double Uz[HARM_NPR], pz[HARM_NPR];
+#pragma unroll
+  for (int pl = 0; pl < HARM_NPR; pl++) {
+    Uz[pl] = U[pl * n + z];
+    pz[pl] = p[pl * n + z];
+  }
+  const int ns0 = ns;
+  bool solved;
+  int fl = hd::utoprimgen<true>(Uz, g, gam, gammafail, pz, ns, plain ? __builtin_nan("") : seed, limit, &solved);
+  if (fl == hd::kUnfinishedFlag) {
+    ns = ns0;
+    return 1;
+  }
+  if (!plain && fl != 0) return 2;
+  if (!solved) {  // the guess stands (read again rather than kept through the iterations)
+    const double* pr = hd::fresh(p);
+#pragma unroll
+    for (int pl = 0; pl <= HARM_U3; pl++) pz[pl] = pr[pl * n + z];
+  }
+  if (hd::needs_after_hot(fl, true, false)) {  // the cold retry, as harm_invert_batch
+    double Ugf[HARM_NPR], p0[HARM_NPR];
+    const double *pr = hd::fresh(p), *Ur = hd::fresh(U);
+#pragma unroll
+    for (int pl = 0; pl < HARM_NPR; pl++) {
+      Ugf[pl] = Ur[pl * n + z];
+      p0[pl] = pr[pl * n + z];
+    }
+    hd::load_geom(hd::fresh(geom), z, n, g);
+    hd::geometry_free(Ugf, g, Ugf);
+    fl = hd::after_hot(fl, Ugf, g, gam, gammafail, p0, pz, ns, true, false);
+  }
+#pragma unroll
+  for (int pl = 0; pl < HARM_NPR; pl++) p[pl * n + z] = pz[pl];
+  pflag[z] = fl;
+  if (niter) niter[z] = ns;
+  return 0;
+}
+
 // Batched inversion started from the network's W' (harm_invert_batch's
-// arguments, plus the count of zones that fell back to the plain guess).
-__global__ __launch_bounds__(kBlock) void k_invert_batch_mlp(const uint16_t* __restrict__ wbf,
-                                                             const float* __restrict__ w32,
-                                                             const float* __restrict__ norm,
-                                                             const double* __restrict__ U,
-                                                             const double* __restrict__ geom, double* __restrict__ p,
-                                                             int32_t* __restrict__ pflag, int32_t* __restrict__ niter,
-                                                             long n, double gam, double gammafail,
-                                                             unsigned long long* __restrict__ nfallback)
+// arguments, plus the count of zones that fell back to the plain guess), in
+// rounds as k_invert_batch: a zone whose seeded solve is unfinished after
+// kFirst iterations, or has failed, goes into the block's list with its seed
+// and the strokes so far, and is solved in a full wave of such zones.
+// 2^20 zones of a log-uniform sample take 0.84 ms (2.39 one zone a lane to the
+// end, the plain solve in the same lane).
+constexpr int kFirst = 16;
+constexpr long kResident = 768;  // blocks the chip holds (three waves a SIMD)
+constexpr int kPlain = 1 << 30;  // in a list entry: the seeded solve has failed
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_invert_batch_mlp(
+    const uint16_t* __restrict__ wbf, const float* __restrict__ w32, const float* __restrict__ norm,
+    const double* __restrict__ U, const double* __restrict__ geom, double* __restrict__ p,
+    int32_t* __restrict__ pflag, int32_t* __restrict__ niter, long n, double gam, double gammafail, int rounds,
+    unsigned long long* __restrict__ nfallback)
 {
   __shared__ Net N;
   __shared__ uint16_t xs[kWaves][64][hm::kIn];
+  __shared__ double lseed[2 * kBlock];
+  __shared__ int list[2 * kBlock], lns[2 * kBlock];  // zones (from z0) to come back to, at most 255 + 256
+  __shared__ int cnt;
+  __shared__ unsigned int nfb;
+  const int tid = threadIdx.x;
+  const long z0 = (long)blockIdx.x * kBlock * rounds;
+  const int first = rounds > 1 ? kFirst : 200;
   stage_net(wbf, w32, N);
+  if (tid == 0) cnt = nfb = 0;
   __syncthreads();
-  const long z = (long)blockIdx.x * kBlock + threadIdx.x;
-  const bool act = z < n;
-  double D = 1.0;
-  float y[1];
-  {
-    float f[hm::kIn] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (act) {
-      hd::Geom g;
-      hd::load_geom(geom, z, n, g);
-      const double ig = (g.gdet >= 0.0 ? 1.0 : -1.0) / (fabs(g.gdet) + D_SMALL);
-      double Ut[HARM_NPR];
-#pragma unroll
-      for (int pl = 0; pl < HARM_NPR; pl++) Ut[pl] = g.alpha * (U[pl * n + z] * ig);
-      hd::Inv s;
-      double Qtcon[4], Bcon[4];
-      hd::inv_setup(Ut, g, gam, gammafail, s, Qtcon, Bcon);
-      hm::features(s, f);
-      D = s.D;
+  int round = 0;
+#pragma clang loop unroll(disable)
+  while (true) {
+    const int c = __builtin_amdgcn_readfirstlane(cnt);  // the same in every thread: cnt changes between barriers only
+    const bool more = round < rounds && z0 + (long)round * kBlock < n;
+    if (!more && c == 0) break;
+    const bool full = c >= kBlock || !more;
+    int loc = -1, ns = 0;
+    bool plain = false;
+    double seed = 0.0;
+    if (full) {
+      if (tid < min(c, kBlock)) {
+        const int e = c - 1 - tid;
+        loc = list[e] & (kPlain - 1);
+        plain = (list[e] & kPlain) != 0;
+        seed = lseed[e];
+        ns = lns[e];
+      }
+    } else {
+      if (z0 + (long)round * kBlock + tid < n) loc = round * kBlock + tid;
+      round++;
     }
-    wave_net<1>(f, act, norm, N, xs[threadIdx.x >> 6], y);
-  }
-  int fb = 0;
-  if (act) {
-    const float y0 = y[0] * norm[2 * hm::kIn + hm::kOut] + norm[2 * hm::kIn];
-    const double seed = D * exp((double)fminf(fmaxf(y0, -60.0f), 60.0f));
-    hd::Geom g;
-    hd::load_geom(geom, z, n, g);
-    double Uz[HARM_NPR], pz[HARM_NPR], pg[HARM_NPR];
-#pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) {
-      Uz[pl] = U[pl * n + z];
-      pg[pl] = p[pl * n + z];
-      pz[pl] = pg[pl];
-    }
-    int ns = 0;
-    int fl = hd::utoprimgen(Uz, g, gam, gammafail, pz, ns, seed);
-    if (fl != 0) {  // the plain guess decides
-      fb = 1;
-#pragma unroll
-      for (int pl = 0; pl < HARM_NPR; pl++) pz[pl] = pg[pl];
-      fl = hd::utoprimgen(Uz, g, gam, gammafail, pz, ns, __builtin_nan(""));
-    }
-    if (hd::needs_after_hot(fl, true, false)) {  // the cold retry, as harm_invert_batch
-      double Ugf[HARM_NPR];
-      hd::geometry_free(Uz, g, Ugf);
-      fl = hd::after_hot(fl, Ugf, g, gam, gammafail, pg, pz, ns, true, false);
-    }
-#pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) p[pl * n + z] = pz[pl];
-    pflag[z] = fl;
-    if (niter) niter[z] = ns;
-  }
-  if (nfallback) {
-    __shared__ unsigned int cnt;
-    if (threadIdx.x == 0) cnt = 0;
+    __syncthreads();  // the list's entries and cnt have been read
+    if (full && tid == 0) cnt = c - min(c, kBlock);
     __syncthreads();
-    if (fb) atomicAdd(&cnt, 1u);
+    if (!full) {  // the whole wave, for the matrix instructions
+      float f[hm::kIn] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, y[1];
+      double D = 1.0;
+      if (loc >= 0) {
+        const long z = z0 + loc;
+        hd::Geom g;
+        hd::load_geom(geom, z, n, g);
+        const double ig = (g.gdet >= 0.0 ? 1.0 : -1.0) / (fabs(g.gdet) + D_SMALL);
+        double Ut[HARM_NPR];
+#pragma unroll
+        for (int pl = 0; pl < HARM_NPR; pl++) Ut[pl] = g.alpha * (U[pl * n + z] * ig);
+        hd::Inv s;
+        double Qtcon[4], Bcon[4];
+        hd::inv_setup(Ut, g, gam, gammafail, s, Qtcon, Bcon);
+        hm::features(s, f);
+        D = s.D;
+      }
+      wave_net<1>(f, loc >= 0, norm, N, xs[tid >> 6], y);
+      const float y0 = y[0] * norm[2 * hm::kIn + hm::kOut] + norm[2 * hm::kIn];
+      seed = D * exp((double)fminf(fmaxf(y0, -60.0f), 60.0f));
+    }
+    if (loc >= 0) {
+      const int left = seeded_one(U, geom, p, pflag, niter, n, gam, gammafail, z0 + loc, seed, plain,
+                                  full ? 200 : first, ns);
+      if (left) {
+        if (left == 2) atomicAdd(&nfb, 1u);
+        const int e = atomicAdd(&cnt, 1);
+        list[e] = loc | (left == 2 ? kPlain : 0);
+        lseed[e] = seed;
+        lns[e] = ns;
+      }
+    }
     __syncthreads();
-    if (threadIdx.x == 0 && cnt) atomicAdd(nfallback, (unsigned long long)cnt);
   }
+  if (nfallback && tid == 0 && nfb) atomicAdd(nfallback, (unsigned long long)nfb);
 }
 
 // deterministic host initialisation: Glorot-uniform weights, zero biases
@@ -632,21 +693,14 @@ harm_status pack(harm_mlp* m, hipStream_t s)
 // the zones of k_invert in the same order; per wave the features of 64 zones
 // go through the network on the matrix cores, each zone's Newton solve then
 // starts from the predicted W' (falling back to the previous primitives when
-// it fails), and the final substep's floors follow in the same kernel
-// (floors_zone, as the plain inversion's floors pass applies them; DIAG:
-// keeping the states the fixes started from).
-template <bool DIAG>
-__global__ __launch_bounds__(kBlock) void k_invert_grid_mlp(const uint16_t* __restrict__ wbf,
-                                                            const float* __restrict__ w32,
-                                                            const float* __restrict__ norm, hd::Dims d, hk::Params P,
-                                                            const double* __restrict__ U,
-                                                            const double* __restrict__ pg, double* pf,
-                                                            int32_t* __restrict__ pflag,
-                                                            const double* __restrict__ gcent,
-                                                            const double* __restrict__ floors, int finalstep,
-                                                            unsigned long long* __restrict__ di,
-                                                            double* __restrict__ fx_p0, double* __restrict__ fx_pfl,
-                                                            uint8_t* __restrict__ fx_flag)
+// it fails).  Bound by issue, the network's tanhs about as much as the Newton
+// iterations; without the floors and with the fallback as a second pass of one
+// loop the solve fits three waves a SIMD (145 registers, 229 before): 12 steps
+// of 128x64x64 28.6 -> 28.1 ms.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_invert_grid_mlp(
+    const uint16_t* __restrict__ wbf, const float* __restrict__ w32, const float* __restrict__ norm, hd::Dims d,
+    hk::Params P, const double* __restrict__ U, const double* __restrict__ pg, double* __restrict__ pf,
+    int32_t* __restrict__ pflag, const double* __restrict__ gcent, int finalstep, unsigned long long* __restrict__ di)
 {
   __shared__ Net N;
   __shared__ uint16_t xs[kWaves][64][hm::kIn];
@@ -683,11 +737,8 @@ __global__ __launch_bounds__(kBlock) void k_invert_grid_mlp(const uint16_t* __re
   if (act) {
     const float y0 = y[0] * norm[2 * hm::kIn + hm::kOut] + norm[2 * hm::kIn];
     const double seed = D * exp((double)fminf(fmaxf(y0, -60.0f), 60.0f));
-    double Uz[HARM_NPR];
-#pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) Uz[pl] = U[pl * d.ncell + o];
-    nf = hk::invert_zone<true, DIAG>(d, P, Uz, U, pg, pf, pflag, gcent, floors, finalstep, o, pp, ns, seed, &fb,
-                                     fx_p0, fx_pfl, fx_flag) > 0;
+    const int fl = hk::invert_zone<true>(d, P, U, pg, pf, pflag, gcent, o, pp, ns, seed, &fb);
+    nf = !finalstep && fl > 0;
   }
   hk::newton_counts_to(ns, nf, di);
   __shared__ unsigned int nfb;
@@ -871,22 +922,19 @@ extern "C" harm_status harm_invert_batch_mlp(harm_mlp* m, const double* U, const
     return hh::set_error(HARM_EINVAL, "harm_invert_batch_mlp: bad arguments");
   const long nb = (long)((n + kBlock - 1) / kBlock);
   if (nb > 0x7fffffffL) return hh::set_error(HARM_EINVAL, "harm_invert_batch_mlp: n too large");
-  hipLaunchKernelGGL(k_invert_batch_mlp, dim3((unsigned)nb), dim3(kBlock), 0, (hipStream_t)stream, m->wbf, m->w32,
-                     m->norm, U, geom, p_inout, pflag, niter, (long)n, gam, gammafail, nfallback);
+  const int rounds = hh::inversion_rounds(nb, kResident);
+  hipLaunchKernelGGL(k_invert_batch_mlp, dim3((unsigned)((nb + rounds - 1) / rounds)), dim3(kBlock), 0,
+                     (hipStream_t)stream, m->wbf, m->w32, m->norm, U, geom, p_inout, pflag, niter, (long)n, gam,
+                     gammafail, rounds, nfallback);
   return hh::check_launch("k_invert_batch_mlp");
 }
 
 harm_status hk::launch_invert_grid_mlp(const harm_mlp* m, const hd::Dims& d, const hk::Params& P, const double* U,
                                        const double* pg, double* pf, int32_t* pflag, const double* gcent,
-                                       const double* floors, int finalstep, unsigned long long* di, hipStream_t s,
-                                       double* fx_p0, double* fx_pfl, uint8_t* fx_flag)
+                                       int finalstep, unsigned long long* di, hipStream_t s)
 {
   const long nb = ((long)d.n1 * d.n2 * d.n3 + kBlock - 1) / kBlock;
-  if (fx_p0)
-    hipLaunchKernelGGL(k_invert_grid_mlp<true>, dim3((unsigned)nb), dim3(kBlock), 0, s, m->wbf, m->w32, m->norm, d, P,
-                       U, pg, pf, pflag, gcent, floors, finalstep, di, fx_p0, fx_pfl, fx_flag);
-  else
-    hipLaunchKernelGGL(k_invert_grid_mlp<false>, dim3((unsigned)nb), dim3(kBlock), 0, s, m->wbf, m->w32, m->norm, d,
-                       P, U, pg, pf, pflag, gcent, floors, finalstep, di, nullptr, nullptr, nullptr);
+  hipLaunchKernelGGL(k_invert_grid_mlp, dim3((unsigned)nb), dim3(kBlock), 0, s, m->wbf, m->w32, m->norm, d, P, U, pg,
+                     pf, pflag, gcent, finalstep, di);
   return hh::check_launch("k_invert_grid_mlp");
 }
