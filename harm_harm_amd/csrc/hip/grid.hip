@@ -974,69 +974,69 @@ __global__ __launch_bounds__(kBlock) void k_x2_reflect(Dims d, double* __restric
   x2_reflect_body(d, p, side, blockIdx.x);
 }
 
-// pole death of one column col = (i + ng1) + ns1 * k at one pole: the first
-// active row and the first ghost row are rebuilt from the second active row.
-// The field components of the ghost row are kept as the reflection left
-// them; with mirror_ghost they are taken from the mirrored first active row
-// directly (the reflection of that ghost row has not run).
-__device__ __forceinline__ void x2_poledeath_col(const Dims& d, const Params& P, double* __restrict__ p,
+// pole death of one row of one column col = (i + ng1) + ns1 * k at one pole:
+// the first ghost row (ghost) or the first active row is rebuilt from the
+// second active row.  The field components of the ghost row are kept as the
+// reflection left them; with mirror_ghost they are taken from the mirrored
+// first active row directly (the reflection of that ghost row has not run).
+// Neither row reads what the other's thread changes: fields of the first
+// active row are rewritten with the values they have, but for B3 in 2-D, which
+// both rows take from the second active row.
+__device__ __forceinline__ void x2_poledeath_row(const Dims& d, const Params& P, double* __restrict__ p,
                                                  const double* __restrict__ gcent, const double* __restrict__ rcent,
-                                                 int side, long col, bool mirror_ghost = false, long img = 0)
+                                                 int side, bool ghost, long col, bool mirror_ghost = false,
+                                                 long img = 0)
 {
   const int i = (int)(col % d.ns1) - d.ng1, k = (int)(col / d.ns1);
   const int n2 = d.n2, n3 = d.n3;
   const long nc = d.ncell;
   const double x2c0 = P.startx[2];
   const int rj = side == 0 ? 1 : n2 - 2;
-  const int js = side == 0 ? -1 : n2 - 1;
-  const int je = side == 0 ? 0 : n2;
+  const int j0 = side == 0 ? 0 : n2 - 1, j = ghost ? (side == 0 ? -1 : n2) : j0;
   const double X0 = side == 0 ? x2c0 : x2c0 + n2 * P.dx[2];
   const double Xr = x2c0 + (rj + 0.5) * P.dx[2];
-  const long ro = hd::cidx(d, i, rj, k);
-  double pref[HARM_NPR];
+  const long ro = hd::cidx(d, i, rj, k), o = hd::cidx(d, i, j, k);
+  double pref[HARM_NPR], pj[HARM_NPR];
 #pragma unroll
   for (int pl = 0; pl < HARM_NPR; pl++) pref[pl] = p[pl * nc + ro];
-  for (int j = js; j <= je; j++) {
-    const long o = hd::cidx(d, i, j, k);
-    double pj[HARM_NPR];
+  if (mirror_ghost && ghost) {
+    // x2_reflect_zone of this ghost row, field components only (pole death
+    // replaces the rest, and never writes the fields of the mirrored row)
+    const int rk = (n3 > 1) ? (k + n3 / 2) % n3 : k;
+    const long so = hd::cidx(d, i, j0, rk);
+    pj[HARM_B1] = p[HARM_B1 * nc + so];
+    pj[HARM_B2] = -p[HARM_B2 * nc + so];
+    pj[HARM_B3] = p[HARM_B3 * nc + so];
+  } else {
 #pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) pj[pl] = p[pl * nc + o];
-    if (mirror_ghost && j == (side == 0 ? js : je)) {
-      // x2_reflect_zone of this ghost row, field components only (pole death
-      // replaces the rest, and never writes the fields of the mirrored row)
-      const int rk = (n3 > 1) ? (k + n3 / 2) % n3 : k;
-      const long so = hd::cidx(d, i, side == 0 ? 0 : n2 - 1, rk);
-      pj[HARM_B1] = p[HARM_B1 * nc + so];
-      pj[HARM_B2] = -p[HARM_B2 * nc + so];
-      pj[HARM_B3] = p[HARM_B3 * nc + so];
-    }
-    const double X = x2c0 + (j + 0.5) * P.dx[2];
-    for (int pl = HARM_RHO; pl <= HARM_U3; pl++) {
-      if (pl == HARM_U2) continue;
-      pj[pl] = pref[pl];
-    }
-    double ftemp = pref[HARM_U2];
-    if ((side == 0 && ftemp > 0.0) || (side == 1 && ftemp < 0.0)) ftemp = 0.0;
-    pj[HARM_U2] = ftemp + (X - Xr) * (ftemp - 0.0) / (Xr - X0);
-    if (n3 == 1) pj[HARM_B3] = pref[HARM_B3];
-    Geom Gj;
-    hd::load_geom(gcent, hd::pidx(d, i, j), d.nplane, Gj);
-    State q;
-    hd::get_state(pj, Gj, P.gam, q);
-    if (q.ucon[1] > 0.0) {
-      const double r = rcent[i + d.ng1];
-      double lim;
-      if (r <= 10.0) lim = 1.1;
-      else lim = 1.1 * pow(r / 10.0, 1.0);
-      hd::limit_gamma(lim, pj, Gj);
-    } else {
-      hd::limit_gamma(P.gammamax, pj, Gj);
-    }
+    for (int pl = HARM_B1; pl <= HARM_B3; pl++) pj[pl] = p[pl * nc + o];
+  }
+  const double X = x2c0 + (j + 0.5) * P.dx[2];
+  for (int pl = HARM_RHO; pl <= HARM_U3; pl++) {
+    if (pl == HARM_U2) continue;
+    pj[pl] = pref[pl];
+  }
+  double ftemp = pref[HARM_U2];
+  if ((side == 0 && ftemp > 0.0) || (side == 1 && ftemp < 0.0)) ftemp = 0.0;
+  pj[HARM_U2] = ftemp + (X - Xr) * (ftemp - 0.0) / (Xr - X0);
+  if (n3 == 1) pj[HARM_B3] = pref[HARM_B3];
+  Geom Gj;
+  hd::load_geom(gcent, hd::pidx(d, i, j), d.nplane, Gj);
+  State q;
+  hd::get_state(pj, Gj, P.gam, q);
+  if (q.ucon[1] > 0.0) {
+    const double r = rcent[i + d.ng1];
+    double lim;
+    if (r <= 10.0) lim = 1.1;
+    else lim = 1.1 * pow(r / 10.0, 1.0);
+    hd::limit_gamma(lim, pj, Gj);
+  } else {
+    hd::limit_gamma(P.gammamax, pj, Gj);
+  }
 #pragma unroll
-    for (int pl = 0; pl < HARM_NPR; pl++) {
-      p[pl * nc + o] = pj[pl];
-      if (img) p[pl * nc + o + img] = pj[pl];
-    }
+  for (int pl = 0; pl < HARM_NPR; pl++) {
+    p[pl * nc + o] = pj[pl];
+    if (img) p[pl * nc + o + img] = pj[pl];
   }
 }
 
@@ -1047,7 +1047,8 @@ __device__ __forceinline__ void x2_poledeath_body(Dims d, Params P, double* __re
   const long t = (long)blk * kBlock + threadIdx.x;
   const long ncol = (long)d.ns1 * d.n3;
   if (t >= ncol || P.bc == HARM_PROBLEM_BONDI) return;  // Bondi: plain reflection only
-  x2_poledeath_col(d, P, p, gcent, rcent, side, t);
+  x2_poledeath_row(d, P, p, gcent, rcent, side, side == 0, t);
+  x2_poledeath_row(d, P, p, gcent, rcent, side, side != 0, t);
 }
 
 // Both poles in one pass, for n2 > ng2: the pole-death columns (rows -1, 0
@@ -1069,7 +1070,8 @@ __device__ __forceinline__ void x2_poles_body(Dims d, Params P, double* __restri
     if (P.bc == HARM_PROBLEM_BONDI)  // plain polar reflection (POLARAXIS): rows -1 and n2 too
       x2_reflect_zone(d, p, side, side == 0 ? d.ng2 - 1 : 0, t - side * ncol);
     else
-      x2_poledeath_col(d, P, p, gcent, rcent, side, t - side * ncol, true);
+      for (int row = 0; row < 2; row++)
+        x2_poledeath_row(d, P, p, gcent, rcent, side, (row == 0) == (side == 0), t - side * ncol, true);
     return;
   }
   const long u = t - 2 * ncol, nside = ncol * (d.ng2 - 1);
@@ -1157,7 +1159,7 @@ __host__ __device__ __forceinline__ BoundPlan bound_plan(const Dims& d, bool fla
   b.nchunk = (d.n2 + rows - 1) / rows;
   while (b.nchunk > 1 && d.n2 / b.nchunk < d.ng2) b.nchunk--;  // a pole's rows in one chunk
   b.nA = 2 * b.nchunk * (d.n3 > 1 ? d.n3 / 2 : 1);
-  b.nB = (int)((2L * (d.n1 - 6) * d.n3 * d.ng2 + kBlock - 1) / kBlock);
+  b.nB = (int)((2L * (d.n1 - 6) * d.n3 * (d.ng2 + 1) + kBlock - 1) / kBlock);
   b.nC = d.n3 > 1 ? (int)(((long)d.n1 * (d.n2 - 2) * 2 * d.ng3 + kBlock - 1) / kBlock) : 0;
   b.nD = flags ? (int)((pflag_items(d) + kBlock - 1) / kBlock) : 0;
   return b;
@@ -1170,15 +1172,18 @@ __device__ __forceinline__ long phi_image(const Dims& d, int k)
   return k < d.ng3 ? d.n3 * d.nplane : k >= d.n3 - d.ng3 ? -d.n3 * d.nplane : 0;
 }
 
-// polar item g of column (i, k) at one pole: 0 the rows next to the pole
-// (pole death; Bondi: the first ghost row), 1 .. ng2-1 the ghost rows beyond
+// polar item g of column (i, k) at one pole: 0 the first ghost row (pole death;
+// Bondi: the reflection), 1 .. ng2-1 the ghost rows beyond, ng2 the first active
+// row (pole death).  A thread for each: rebuilding a row is a chain of loads and
+// a few hundred dependent instructions, and two of them one after the other made
+// the launch 15.8 us at 64x64, 13.8 so.
 __device__ __forceinline__ void polar_item(const Dims& d, const Params& P, double* p, const double* gcent,
                                            const double* rcent, int side, int g, int i, int k)
 {
   const long col = (i + d.ng1) + (long)d.ns1 * k, img = phi_image(d, k);
-  if (g > 0) x2_reflect_zone(d, p, side, g - 1 + side, col, img);
-  else if (P.bc == HARM_PROBLEM_BONDI) x2_reflect_zone(d, p, side, side == 0 ? d.ng2 - 1 : 0, col, img);
-  else x2_poledeath_col(d, P, p, gcent, rcent, side, col, true, img);
+  if (g > 0 && g < d.ng2) x2_reflect_zone(d, p, side, g - 1 + side, col, img);
+  else if (P.bc != HARM_PROBLEM_BONDI) x2_poledeath_row(d, P, p, gcent, rcent, side, g == 0, col, true, img);
+  else if (g == 0) x2_reflect_zone(d, p, side, side == 0 ? d.ng2 - 1 : 0, col, img);
 }
 
 __device__ __forceinline__ void bounds_prims(const Dims& d, const Params& P, const BoundPlan& b, double* p,
@@ -1205,13 +1210,14 @@ __device__ __forceinline__ void bounds_prims(const Dims& d, const Params& P, con
   if (blk < b.nA + b.nB) {
     // polar items: of a block's edge columns (A), or one a thread of the others (B)
     const int m = A ? d.ng1 + 3 : d.n1 - 6, np = A ? (d.n3 > 1 ? 2 : 1) : d.n3, i0 = A ? (up ? d.n1 - 3 : -d.ng1) : 3;
-    const long n = (long)m * np * d.ng2 * (lo + hi);
+    const int ni = d.ng2 + 1;
+    const long n = (long)m * np * ni * (lo + hi);
     const long t0 = A ? 0 : (long)(blk - b.nA) * kBlock, t1 = A ? n : min(n, t0 + kBlock);
     for (long t = t0 + tid; t < t1; t += kBlock) {
       const int i = i0 + (int)(t % m);
       const long r = t / m;
       const int kk = (int)(r % np), u = (int)(r / np);
-      polar_item(d, P, p, gcent, rcent, lo && hi ? u / d.ng2 : hi, u % d.ng2, i, A ? pr + kk * (d.n3 / 2) : kk);
+      polar_item(d, P, p, gcent, rcent, lo && hi ? u / ni : hi, u % ni, i, A ? pr + kk * (d.n3 / 2) : kk);
     }
     return;
   }
