@@ -283,9 +283,8 @@ void launch_flux_batch(int recon, const int* n, const int* const* pre, hipStream
                        int which, int do_ct);
 // WENO5BND (weno.hip): the dP measure of every active direction, then the
 // face values of one direction's lines
-// (tm: 10 x ncell doubles of per-zone terms, dp: 3 x ncell)
-void launch_weno_dp(const Dims& d, hipStream_t s, const double* pb, const double* gcent, const Params& P, double* tm,
-                    double* dp);
+// (dp: 3 x ncell)
+void launch_weno_dp(const Dims& d, hipStream_t s, const double* pb, const double* gcent, const Params& P, double* dp);
 void launch_weno_recon(int dir, const Dims& d, const Box& b, hipStream_t s, const double* pb, const double* dp,
                        double* L, double* R);
 

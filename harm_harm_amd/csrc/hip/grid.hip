@@ -1368,7 +1368,6 @@ struct harm_handle {
   long cur_calls = 0;      // current_calc_1's call count and the dt of its last call
   double cur_lastdt = 0.0;
   double* wdp = nullptr;   // WENO5BND: dP measure per direction (3 x ncell)
-  double* wtm = nullptr;   // WENO5BND: per-zone terms of dP (10 x ncell)
   double* facc = nullptr;  // boundary-flux partial sums
   double* en = nullptr;      // energy-file accumulators (EN_*)
   double* enpart = nullptr;  // their per-block partial sums
@@ -1645,7 +1644,7 @@ harm_status enq_fluxcalc(harm_handle* h, int which_p, int do_ct, bool in_step = 
   const bool weno = recon == HARM_RECON_WENO5;
   if (weno) {
     prof_begin(h);
-    launch_weno_dp(d, s, pb, h->geom[HARM_LOC_CENT], h->P, h->wtm, h->wdp);
+    launch_weno_dp(d, s, pb, h->geom[HARM_LOC_CENT], h->P, h->wdp);
     prof_end(h, HARM_K_RECON);
   }
   // WENO5BND: each direction's lines are reconstructed into its own block of
@@ -2233,7 +2232,7 @@ harm_status enq_batch_substep(harm_batch* b, int to, int nto, const double CUf[4
   const bool weno = b->recon == HARM_RECON_WENO5;
   if (weno)
     for (harm_handle* h : b->grids) {
-      launch_weno_dp(h->d, s, h->arr[pbb[to]], h->geom[HARM_LOC_CENT], h->P, h->wtm, h->wdp);
+      launch_weno_dp(h->d, s, h->arr[pbb[to]], h->geom[HARM_LOC_CENT], h->P, h->wdp);
       for (int dir = 1; dir <= 3; dir++)
         if ((dir == 1 ? h->d.n1 : dir == 2 ? h->d.n2 : h->d.n3) > 1)
           launch_weno_recon(dir, h->d, h->ft[dir].b, s, h->arr[pbb[to]], h->wdp, wl_dir(h, dir), wr_dir(h, dir));
@@ -2391,7 +2390,6 @@ extern "C" harm_status harm_create(const harm_config* cfg, harm_handle** out)
     }
     TRYC(hh::check_hip(hipEventCreateWithFlags(&h->evfork, hipEventDisableTiming), "hipEventCreate"));
     TRYC(alloc((void**)&h->wdp, sizeof(double) * 3 * d.ncell));
-    TRYC(alloc((void**)&h->wtm, sizeof(double) * 10 * d.ncell));
     TRYC(hh::check_hip(hipMemset(h->wl, 0, sizeof(double) * 3 * HARM_NPR * d.ncell), "hipMemset"));
     TRYC(hh::check_hip(hipMemset(h->wr, 0, sizeof(double) * 3 * HARM_NPR * d.ncell), "hipMemset"));
     TRYC(hh::check_hip(hipMemset(h->wdp, 0, sizeof(double) * 3 * d.ncell), "hipMemset"));
@@ -2442,7 +2440,7 @@ extern "C" harm_status harm_destroy(harm_handle* h)
     (void)hipEventDestroy(r.second.second);
   }
   for (hipEvent_t e : h->evpool) (void)hipEventDestroy(e);
-  void* bufs[] = {h->pflag, h->pfix, h->gcorn3, h->conn, h->floors, h->rcent, h->emf, h->wl, h->wr, h->wdp, h->wtm, h->facc,
+  void* bufs[] = {h->pflag, h->pfix, h->gcorn3, h->conn, h->floors, h->rcent, h->emf, h->wl, h->wr, h->wdp, h->facc,
                   h->cf, h->jcon, h->xfer, h->axes, h->rows,
                   h->en, h->enpart, h->entot, h->fx_p0, h->fx_pfl, h->fx_flag, h->ds, h->di};
   for (void* b : bufs) (void)hipFree(b);
@@ -3483,7 +3481,7 @@ extern "C" harm_status harm_tune(harm_handle* h, int32_t reps, int32_t td_out[4]
       double* F = h->arr[HARM_ARR_F1 + dir - 1];
       const double* G = h->geom[dir];
       if (recon == HARM_RECON_WENO5) {  // the face kernel reads this direction's line reconstruction
-        launch_weno_dp(d, s, pb, h->geom[HARM_LOC_CENT], h->P, h->wtm, h->wdp);
+        launch_weno_dp(d, s, pb, h->geom[HARM_LOC_CENT], h->P, h->wdp);
         launch_weno_recon(dir, d, T.b, s, pb, h->wdp, wl_dir(h, dir), wr_dir(h, dir));
       }
       auto launch = [&]() {

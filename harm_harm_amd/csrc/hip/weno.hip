@@ -19,7 +19,7 @@
 //   * the optimal face weights and the blend of WENO5, WENO3 and SMONO values
 //     (choose_weno_order :2442, eno_cvt :884, eno_line_reconstruct :538).
 //
-// Device layout.  k_weno_terms and k_weno_dp form dP for every direction at
+// Device layout.  k_weno_dp forms dP for every direction at
 // every zone that a face reconstruction needs (compute_df_line_new
 // interpline.c:3557, from the zone's state and its two neighbours' along the
 // direction).  Along x1, where a line is contiguous in memory,
@@ -523,52 +523,85 @@ __device__ __forceinline__ void load_prim(const double* __restrict__ p, long nce
   for (int v = 0; v < HARM_NPR; v++) pr[v] = p[v * ncell + c];
 }
 
-// The zone terms of the dP measure for every active direction: tm[0] = rho,
-// then (par, veff, upar) of direction d at tm[1 + 3 (d-1) ..].  One state
-// per zone, over the zones -2 .. N+1 of every active direction.
-__global__ __launch_bounds__(kBlock) void k_weno_terms(Dims d, Box z, const double* __restrict__ pb,
-                                                         const double* __restrict__ gcent, double gam,
-                                                         double* __restrict__ tm)
+// dP of every active direction at the zones of z, -1 .. N of every active
+// direction (the zones whose faces are reconstructed).  A zone's measure takes
+// its own terms and those of its two neighbours along the direction.  A block
+// marches through the k planes of a chunk with a tile of kDpI x kDpJ zones in
+// (i, j), a halo zone on each active side included: every plane each thread
+// forms the terms of its zone, the neighbours' of directions 1 and 2 come from
+// LDS, the planes before and after from registers.
+//
+// Bound by the latency of a plane's chain at four waves a SIMD.  In two passes,
+// the terms of every zone through memory (10 doubles written, 18 read), this
+// took 94 + 54 us at 256x128x64, 23 + 16 at 128x64x64 and 8.4 + 5.2 at 97x51x22;
+// so it takes 66, 26 and 11.4, though 40 % more terms are formed.  Tiles of
+// 32 x 16 and 64 x 8: 76, 26, 11 and 86, 29, 11.  With the geometry read again
+// every plane 108 us at four waves, 126 to 300 at six and eight (spills).
+constexpr int kDpI = 32, kDpJ = 8;
+struct DpPlan {
+  int ti, tj, tk, nk;  // tiles along i, j; chunks along k, of nk planes
+};
+__global__ __launch_bounds__(kDpI* kDpJ) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_weno_dp(
+    Dims d, Box z, DpPlan pl, const double* __restrict__ pb, const double* __restrict__ gcent, double gam,
+    double* __restrict__ dp)
 {
-  int i, j, k;
-  if (!z.at((long)blockIdx.x * kBlock + threadIdx.x, i, j, k)) return;
+  __shared__ double lds[2][4][kDpI * kDpJ];  // by plane: veff, upar of direction 1, of direction 2
+  const int e1 = d.n1 > 1, e2 = d.n2 > 1, e3 = d.n3 > 1;
+  const int tid = threadIdx.x, ti = tid % kDpI, tj = tid / kDpI;
+  int q = xcd_tile(blockIdx.x, gridDim.x);
+  const int bi = q % pl.ti;
+  q /= pl.ti;
+  const int bk = q % pl.tk, bj = q / pl.tk;
+  const int i = z.is - e1 + bi * (kDpI - 2 * e1) + ti, j = z.js - e2 + bj * (kDpJ - 2 * e2) + tj;
+  const int k0 = z.ks + bk * pl.nk, k1 = min(k0 + pl.nk, z.ks + z.nk);  // planes k0 .. k1 - 1
+  const bool act = i < z.is + z.ni + e1 && j < z.js + z.nj + e2;
+  const bool out = act && ti >= e1 && ti < kDpI - e1 && tj >= e2 && tj < kDpJ - e2 && i < z.is + z.ni &&
+                   j < z.js + z.nj;
+  const long pp = act ? hd::pidx(d, i, j) : 0, nc = d.ncell;
+  auto measure = [&](double rho, double par, double upar, double vp, double vm, double up, double um) {
+    const double dv = vp - vm;
+    return (fabs(rho * dv * dv) + fabs(up - um)) / (fabs(rho * par) + fabs(upar) + D_SMALL);
+  };
   Geom G;
-  hd::load_geom(gcent, hd::pidx(d, i, j), d.nplane, G);
+  hd::load_geom(gcent, pp, d.nplane, G);
+  double rho1 = 0, par1 = 0, v1 = 0, u1 = 0, v2 = 0, u2 = 0;  // direction 3: the plane before, and the one before that
   double pr[HARM_NPR];
-  const long c = hd::cidx(d, i, j, k);
-  load_prim(pb, d.ncell, c, pr);
-  State q;
-  hd::get_state<false>(pr, G, gam, q);
-  tm[c] = pr[HARM_RHO];
+  long c = act ? hd::cidx(d, i, j, k0 - e3) : 0;
+  load_prim(pb, nc, c, pr);
+#pragma clang loop unroll(disable)
+  for (int k = k0 - e3; k < k1 + e3; k++) {
+    const int b = k & 1;
+    DpTerms t[3];
+    {
+      State s;
+      hd::get_state<false>(pr, G, gam, s);
 #pragma unroll
-  for (int dir = 1; dir <= 3; dir++) {
-    if ((dir == 1 ? d.n1 : dir == 2 ? d.n2 : d.n3) <= 1) continue;
-    const DpTerms t = dp_terms(q, pr, G, gam, dir);
-    tm[(1 + 3 * (dir - 1)) * d.ncell + c] = t.par;
-    tm[(2 + 3 * (dir - 1)) * d.ncell + c] = t.veff;
-    tm[(3 + 3 * (dir - 1)) * d.ncell + c] = t.upar;
-  }
-}
-
-// dP of every active direction at the zones -1 .. N of every active direction
-// (the zones whose faces are reconstructed), from the terms of the zone and
-// its two neighbours along the direction.
-__global__ __launch_bounds__(kBlock) void k_weno_dp(Dims d, Box z, const double* __restrict__ tm,
-                                                      double* __restrict__ dp)
-{
-  int i, j, k;
-  if (!z.at((long)blockIdx.x * kBlock + threadIdx.x, i, j, k)) return;
-  const long c = hd::cidx(d, i, j, k);
-  const double rho = tm[c];
-#pragma unroll
-  for (int dir = 1; dir <= 3; dir++) {
-    if ((dir == 1 ? d.n1 : dir == 2 ? d.n2 : d.n3) <= 1) continue;
-    const long st = dir == 1 ? 1 : dir == 2 ? (long)d.ps1 : (long)d.ps1 * d.ns2;
-    const double* T = tm + (1 + 3 * (dir - 1)) * d.ncell;
-    const double par = T[c], upar = T[2 * d.ncell + c];
-    const double dv = T[d.ncell + c + st] - T[d.ncell + c - st];
-    dp[(dir - 1) * d.ncell + c] = (fabs(rho * dv * dv) + fabs(T[2 * d.ncell + c + st] - T[2 * d.ncell + c - st])) /
-                                  (fabs(rho * par) + fabs(upar) + D_SMALL);
+      for (int dir = 1; dir <= 3; dir++) t[dir - 1] = dp_terms(s, pr, G, gam, dir);
+    }
+    const long cn = act ? c + (long)d.ps1 * d.ns2 : 0;
+    if (k + 1 < k1 + e3) load_prim(pb, nc, cn, pr);
+    lds[b][0][tid] = t[0].veff;
+    lds[b][1][tid] = t[0].upar;
+    lds[b][2][tid] = t[1].veff;
+    lds[b][3][tid] = t[1].upar;
+    __syncthreads();
+    if (out && k >= k0 && k < k1) {
+      if (e1)
+        dp[c] = measure(t[0].rho, t[0].par, t[0].upar, lds[b][0][tid + 1], lds[b][0][tid - 1], lds[b][1][tid + 1],
+                        lds[b][1][tid - 1]);
+      if (e2)
+        dp[nc + c] = measure(t[1].rho, t[1].par, t[1].upar, lds[b][2][tid + kDpI], lds[b][2][tid - kDpI],
+                             lds[b][3][tid + kDpI], lds[b][3][tid - kDpI]);
+    }
+    if (e3 && out && k - 1 >= k0 && k - 1 < k1)
+      dp[2 * nc + c - (long)d.ps1 * d.ns2] = measure(rho1, par1, u1, t[2].veff, v2, t[2].upar, u2);
+    v2 = v1;
+    u2 = u1;
+    rho1 = t[2].rho;
+    par1 = t[2].par;
+    v1 = t[2].veff;
+    u1 = t[2].upar;
+    c = cn;
   }
 }
 
@@ -832,18 +865,22 @@ LinePlan plan_lines(int dir, const Dims& d, const Box& b)
 
 }  // namespace
 
-// dP of every active direction over the zones the face reconstructions read;
-// tm: 10 x ncell doubles of zone terms
-void launch_weno_dp(const Dims& d, hipStream_t s, const double* pb, const double* gcent, const Params& P, double* tm,
-                    double* dp)
+// dP of every active direction over the zones the face reconstructions read
+void launch_weno_dp(const Dims& d, hipStream_t s, const double* pb, const double* gcent, const Params& P, double* dp)
 {
-  const int e0 = d.n1 > 1, e1 = d.n2 > 1, e2 = d.n3 > 1;
-  Box zt{-2 * e0, -2 * e1, -2 * e2, d.n1 + 4 * e0, d.n2 + 4 * e1, d.n3 + 4 * e2};
-  hipLaunchKernelGGL(k_weno_terms, dim3((unsigned)((zt.count() + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d, zt,
-                     pb, gcent, P.gam, tm);
-  Box z{-e0, -e1, -e2, d.n1 + 2 * e0, d.n2 + 2 * e1, d.n3 + 2 * e2};
-  hipLaunchKernelGGL(k_weno_dp, dim3((unsigned)((z.count() + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d, z, tm,
-                     dp);
+  const int e1 = d.n1 > 1, e2 = d.n2 > 1, e3 = d.n3 > 1;
+  const Box z{-e1, -e2, -e3, d.n1 + 2 * e1, d.n2 + 2 * e2, d.n3 + 2 * e3};
+  DpPlan pl;
+  pl.ti = (z.ni + kDpI - 2 * e1 - 1) / (kDpI - 2 * e1);
+  pl.tj = (z.nj + kDpJ - 2 * e2 - 1) / (kDpJ - 2 * e2);
+  // chunks of at least two planes (a chunk forms the terms of two more), as
+  // many as give the chip four blocks a CU
+  const int want = (1024 + pl.ti * pl.tj - 1) / (pl.ti * pl.tj);
+  pl.tk = std::max(1, std::min(want, z.nk / 2));
+  pl.nk = (z.nk + pl.tk - 1) / pl.tk;
+  pl.tk = (z.nk + pl.nk - 1) / pl.nk;
+  hipLaunchKernelGGL(k_weno_dp, dim3((unsigned)(pl.ti * pl.tj * pl.tk)), dim3(kDpI * kDpJ), 0, s, d, z, pl, pb, gcent,
+                     P.gam, dp);
 }
 
 // face values L, R (SoA like pb) of zones -1 .. N along dir over the
