@@ -779,10 +779,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 // For grids whose lines are too few to fill the chip with sweeps, which take a
 // segment's zones one after the other: x2 + x3 take 59 + 62 us at 97x51x22 as
 // sweeps and 31 + 29 so, 54 and 9 (x2) at 200x100x1, 68 + 68 and 53 + 45 at
-// 96x64x32, 111 + 133 and 127 + 103 at 128x64x64.  On large grids its barriers
-// cost more than the sweeps' halo (waves in smooth regions wait for the
-// others): 308 + 347 and 446 + 390 at 256x128x64, where smaller blocks change
-// nothing (391 + 406 with 32 zones a segment).
+// 96x64x32.  On large grids its barriers cost more than the sweeps' halo (waves
+// in smooth regions wait for the others): 308 + 347 and 446 + 390 at 256x128x64,
+// where smaller blocks change nothing (391 + 406 with 32 zones a segment).
+// Whole RK3 steps of an evolved torus, where the directions share the chip, as
+// sweeps and so: 96x64x32 981 and 953 us, 128x64x40 1349 and 1349, 200x40x50
+// 1525 and 1507, 128x64x48 1523 and 1535, 128x64x64 1881 and 1968.
 constexpr int kLineMax = 1024;  // threads of a block
 constexpr int kCols = 8;        // lines of a block
 struct LinePlan {
@@ -905,8 +907,8 @@ void launch_weno_recon(int dir, const Dims& d, const Box& b, hipStream_t s, cons
   const int N = dir == 2 ? d.n2 : d.n3;
   const int nf = N + 2;  // zones -1 .. N
   const long nl = (long)b.ni * (dir == 3 ? b.nj : b.nk);
-  // a zone a thread where that makes at most 72 waves a SIMD (about 550 000 zones)
-  constexpr long kLineWaves = 73728;
+  // a zone a thread where that makes at most 50 waves a SIMD (about 400 000 zones)
+  constexpr long kLineWaves = 51200;
   if (nl * N * HARM_NPR <= 64 * kLineWaves) {
     const LinePlan p = plan_lines(dir, d, b);
     const dim3 grid((unsigned)p.blocks), blk((unsigned)p.threads);
