@@ -901,8 +901,12 @@ void launch_weno_recon(int dir, const Dims& d, const Box& b, hipStream_t s, cons
     return;
   }
   // directions 2 and 3: lines cut into segments of at least kMinSeg faces,
-  // about kWaveTarget waves in all (a few per SIMD)
-  constexpr long kWaveTarget = 16384;  // measured: 4 segments along x3, 8 along x2 at 256x128x64
+  // about kWaveTarget waves in all: few enough that the five zones a segment
+  // forms ahead of its faces cost little, and the other directions' passes fill
+  // its last waves' place.  Steps of an evolved 256x128x64 torus with 2048,
+  // 4096, 6144, 8192 and 16384: 5802, 5858, 5815, 5828 and 5940 us; of
+  // 128x128x64: 3535, 3257, 3261, 3297 and 3299.
+  constexpr long kWaveTarget = 6144;
   constexpr int kMinSeg = 16;
   const int N = dir == 2 ? d.n2 : d.n3;
   const int nf = N + 2;  // zones -1 .. N
