@@ -12,7 +12,7 @@
 //                    dump_ener.c:680, SETFDIVBFLUXCTTOTHPRIM)
 //   k_ener_reduce    fixed-order sums of per-block partials, one block per
 //                    channel
-//   k_dump_cols      the physics columns of HARM's main dump (dump.c:439)
+//   k_dump_rows      the rows of HARM's main dump (dump.c:439)
 //   k_current_*      the dump's four-current (phys.c:552-1000)
 //
 //   k_ener_fix       the final substep's floor and gamma-limit changes from

@@ -35,13 +35,14 @@
 // in this translation unit, correctly rounded quotients), so the face values
 // agree bit for bit.
 //
-// The passes are bound by instruction issue (0.56-0.72 of the vector issue
-// slots, 360 instructions a wave of 52 faces along x1).  Quotients are the
-// largest part of it, so the weights of a zone share one reciprocal per
-// normalisation (hd::recip, hd::quot), 7 + 3 + 3 instructions for three
-// quotients instead of 33, and the SMONO and ratio tests settle clear cases
-// without a quotient.  At 256x128x64 the x1, x2 and x3 passes take 265, 301
-// and 337 us (311, 405 and 450 with the compiler's divisions, same steps).
+// The passes are bound by instruction issue: about 500 instructions a zone and
+// primitive with 0.62 of the lanes active, 0.84 (x1), 0.75 and 0.63 (the sweeps
+// alone on the chip) of the vector issue slots, an FP64 reciprocal taking four.
+// Quotients are the largest part of it, so the weights of a zone share one
+// reciprocal per normalisation (hd::recip, hd::quot), 7 + 3 + 3 instructions for
+// three quotients instead of 33, and the SMONO and ratio tests settle clear
+// cases without a quotient.  At 256x128x64 the x1, x2 and x3 passes take 265, 301
+// and 337 us so, 311, 405 and 450 with the compiler's divisions.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <float.h>
