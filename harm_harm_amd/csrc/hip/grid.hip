@@ -1333,6 +1333,55 @@ inline unsigned nblocks(long n) { return (unsigned)((n + kBlock - 1) / kBlock); 
 
 constexpr int kSlots = 3;  // pinned pieces of a handle's host copies
 
+// A step is a fixed sequence of kernel launches with arguments that do not
+// change between steps, so it is captured in a hipGraph (kernel nodes only) and
+// replayed, from kGraphSteps steps in a call on as graphs of that many: the gap
+// between two graphs is about 8 us, 119 us a step of the 64x64 RK2 torus with
+// one step a graph, 112.7 with 4, 111.8 with 8 and 112.6 with 16, whose capture
+// costs a grid's first 40 steps more than it saves (5.2 ms, 5.0 with 4).
+constexpr int kGraphSteps = 4;
+struct StepGraph {
+  hipGraph_t graph[2] = {nullptr, nullptr};  // one step, kGraphSteps steps
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
+  void drop()
+  {
+    for (int q = 0; q < 2; q++) {
+      if (exec[q]) (void)hipGraphExecDestroy(exec[q]);
+      if (graph[q]) (void)hipGraphDestroy(graph[q]);
+      exec[q] = nullptr;
+      graph[q] = nullptr;
+    }
+  }
+  // nsteps steps on stream s, each enqueued by step(); line: a step's kernels
+  // follow one another.  (WENO5BND's three branches take the gap's place: the
+  // longer graph gives nothing, 415 us a step of 97x51x22 either way, and its
+  // capture takes 0.2 ms more.)
+  template <class STEP>
+  harm_status run(hipStream_t s, int nsteps, bool line, STEP step)
+  {
+    for (int q = line ? 1 : 0; q >= 0; q--) {
+      const int len = q ? kGraphSteps : 1;
+      if (nsteps < len) continue;
+      if (!exec[q]) {
+        HH_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        harm_status st = HARM_OK;
+        for (int n = 0; n < len && st == HARM_OK; n++) st = step();
+        hipGraph_t g = nullptr;
+        const hipError_t e = hipStreamEndCapture(s, &g);
+        if (st != HARM_OK) {
+          if (g) (void)hipGraphDestroy(g);
+          return st;
+        }
+        HH_HIP(e);
+        graph[q] = g;
+        HH_HIP(hipGraphInstantiate(&exec[q], g, nullptr, nullptr, 0));
+      }
+      for (; nsteps >= len; nsteps -= len) HH_HIP(hipGraphLaunch(exec[q], s));
+    }
+    return HARM_OK;
+  }
+};
+
 }  // namespace
 
 // ===========================================================================
@@ -1378,8 +1427,7 @@ struct harm_handle {
   uint8_t* fx_flag = nullptr;
   const harm_mlp* guess = nullptr;  // learned inversion guess (harm_set_inversion_guess), or none
   int tile_td[4] = {0, 0, 0, 0};  // sweep depth of the face tiles of dirs 2,3 (0: cost model)
-  hipGraph_t sgraph = nullptr;      // one full step, captured on first use when not profiling
-  hipGraphExec_t sexec = nullptr;
+  StepGraph sgraph;                 // full steps, captured on first use when not profiling
   FaceTile ft[4];                 // planned face tiles per direction (index 1..3)
   double* ds = nullptr;
   unsigned long long* di = nullptr;
@@ -1572,10 +1620,7 @@ harm_status check_handle(const harm_handle* h) { return h ? HARM_OK : hh::set_er
 
 void drop_step_graph(harm_handle* h)
 {
-  if (h->sexec) (void)hipGraphExecDestroy(h->sexec);
-  if (h->sgraph) (void)hipGraphDestroy(h->sgraph);
-  h->sexec = nullptr;
-  h->sgraph = nullptr;
+  h->sgraph.drop();
 }
 harm_status check_which(int which)
 {
@@ -2165,8 +2210,7 @@ struct harm_batch {
   int recon = 0, timeorder = 0, dm = 0;
   bool x2_merged = true;  // every grid has n2 > ng2 (or no polar boundary): both poles in one launch
   bool bnd_merged = true; // every grid takes the boundary pass in one launch (bounds_merge)
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
+  StepGraph graph;
 };
 
 namespace {
@@ -2895,10 +2939,8 @@ harm_status enq_step(harm_handle* h)
 }
 }  // namespace
 
-// A step is a fixed sequence of ~75 kernel launches with arguments that do not
-// change between steps, so it is captured once in a hipGraph (kernel nodes
-// only) and replayed; with kernel timing enabled the launches go out one by one
-// so that the timing events can bracket them.
+// With kernel timing enabled the launches go out one by one, so that the timing
+// events can bracket them.
 extern "C" harm_status harm_step(harm_handle* h, int32_t nsteps)
 {
   HH_TRY(check_handle(h));
@@ -2907,22 +2949,7 @@ extern "C" harm_status harm_step(harm_handle* h, int32_t nsteps)
     for (int n = 0; n < nsteps; n++) HH_TRY(enq_step(h));
     return HARM_OK;
   }
-  if (nsteps == 0) return HARM_OK;
-  if (!h->sexec) {
-    HH_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    const harm_status st = enq_step(h);
-    hipGraph_t g = nullptr;
-    const hipError_t e = hipStreamEndCapture(h->stream, &g);
-    if (st != HARM_OK) {
-      if (g) (void)hipGraphDestroy(g);
-      return st;
-    }
-    HH_HIP(e);
-    h->sgraph = g;
-    HH_HIP(hipGraphInstantiate(&h->sexec, h->sgraph, nullptr, nullptr, 0));
-  }
-  for (int n = 0; n < nsteps; n++) HH_HIP(hipGraphLaunch(h->sexec, h->stream));
-  return HARM_OK;
+  return h->sgraph.run(h->stream, nsteps, h->cfg.recon != HARM_RECON_WENO5, [&] { return enq_step(h); });
 }
 
 extern "C" harm_status harm_get_boundary_fluxes(harm_handle* h, double out[4])
@@ -3518,8 +3545,7 @@ extern "C" harm_status harm_batch_destroy(harm_batch* b)
 {
   if (!b) return HARM_OK;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
+  b->graph.drop();
   for (harm_handle* h : b->grids) {
     if (!h) continue;
     h->stream = nullptr;  // the batch's stream, destroyed below
@@ -3578,8 +3604,7 @@ extern "C" harm_status harm_batch_tune(harm_batch* b, int32_t reps)
   if (!b) return hh::set_error(HARM_EINVAL, "harm_batch_tune: null batch");
   for (harm_handle* h : b->grids) HH_TRY(harm_tune(h, reps, nullptr));
   HH_HIP(hipStreamSynchronize(b->stream));
-  if (b->exec) { (void)hipGraphExecDestroy(b->exec); b->exec = nullptr; }
-  if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
+  b->graph.drop();
   return batch_build(b);
 }
 
@@ -3590,21 +3615,7 @@ extern "C" harm_status harm_batch_step(harm_batch* b, int32_t nsteps, int32_t us
     for (int n = 0; n < nsteps; n++) HH_TRY(enq_batch_step(b));
     return hh::check_launch("harm_batch_step");
   }
-  if (!b->exec) {
-    HH_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    const harm_status st = enq_batch_step(b);
-    hipGraph_t g = nullptr;
-    const hipError_t e = hipStreamEndCapture(b->stream, &g);
-    if (st != HARM_OK) {
-      if (g) (void)hipGraphDestroy(g);
-      return st;
-    }
-    HH_HIP(e);
-    b->graph = g;
-    HH_HIP(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
-  }
-  for (int n = 0; n < nsteps; n++) HH_HIP(hipGraphLaunch(b->exec, b->stream));
-  return HARM_OK;
+  return b->graph.run(b->stream, nsteps, b->recon != HARM_RECON_WENO5, [&] { return enq_batch_step(b); });
 }
 
 extern "C" harm_status harm_batch_sync(harm_batch* b)
