@@ -1136,8 +1136,10 @@ __global__ __launch_bounds__(kBlock) void k_bound_x3(Dims d, double* __restrict_
 //  D: the flags' ghost layer (bound_pflag), both phases: the flags phase 0
 //     copies along phi before phase 1 rewrites them are copied by the thread
 //     that then rewrites them.
-// Needs n2 > ng2 (as x2_poles) and n1 >= 8 (the two radial ends' columns are
-// disjoint); other grids take the direction-by-direction launches.
+// Needs an x2 direction with n2 > ng2 (as x2_poles) and n1 >= 8 (the two radial
+// ends' columns are disjoint); other grids take the direction-by-direction
+// launches.  With n2 = 1 there are no polar rows (ng2 is 0), and rows -1 and 1
+// would lie outside the grid's planes.
 // On such grids the pass applied twice gives the same values as once: the rows
 // it reads are rows it does not write, except the first active row's fields in
 // 2-D and its other variables, which both come from the second active row
@@ -1147,7 +1149,10 @@ struct BoundPlan {
   int nchunk, nA, nB, nC, nD;
   __host__ __device__ int total() const { return nA + nB + nC + nD; }
 };
-__host__ __device__ __forceinline__ bool bounds_merge(const Dims& d) { return d.n1 >= 8 && d.n2 > d.ng2; }
+__host__ __device__ __forceinline__ bool bounds_merge(const Dims& d)
+{
+  return d.n1 >= 8 && d.n2 > 1 && d.n2 > d.ng2;
+}
 __host__ __device__ __forceinline__ long pflag_items(const Dims& d)
 {
   return (long)d.n2 * d.n3 + (long)(d.n1 + 2) * d.n3 + (d.n3 > 1 ? (long)(d.n1 + 1) * d.n2 : 0);
@@ -1839,7 +1844,7 @@ harm_status enq_bound(harm_handle* h, int which, bool flags = false, bool cond =
   if (d.n1 > 1)
     hipLaunchKernelGGL(k_bound_x1, dim3(nblocks(2L * d.ng1 * d.n2 * d.n3)), dim3(kBlock), 0, s, d, h->P, p,
                        h->geom[HARM_LOC_CENT]);
-  if (d.n2 > d.ng2) {
+  if (d.n2 > 1 && d.n2 > d.ng2) {
     hipLaunchKernelGGL(k_x2_poles, dim3(nblocks(2L * d.ns1 * d.n3 * d.ng2)), dim3(kBlock), 0, s, d, h->P, p,
                        h->geom[HARM_LOC_CENT], h->rcent);
   } else if (d.n2 > 1) {  // so few rows that the two poles' stencils overlap: one pole after the other
