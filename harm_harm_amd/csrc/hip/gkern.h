@@ -22,10 +22,13 @@ enum { DS_DT = 0, DS_T = 1, DS_NDT1 = 2, DS_NDT2 = 3, DS_NDT3 = 4, DS_ACCDT = 5,
 // the time was last set
 // and the zones whose learned-guess solve fell back to the plain guess
 // DI_FIX: zones of the current substep that its inversion left with pflag > 0
-// (what failure averaging will change); DI_TICKET: blocks of the 2-D boundary
-// launch that are done, 0 between launches
+// (what failure averaging will change); DI_DRAWN, DI_DONE, DI_LEFT: the queue of
+// the 2-D boundary launch (items drawn, items done, blocks that have left it), 0
+// between launches.  On 2-D grids the list of the DI_FIX zones follows (i + n1 j,
+// 32 bits each, fail_list_cap of them).
 enum { DI_NSTROKE = 0, DI_NFAIL = 1, DI_NSTROKE_SUM = 2, DI_NFAIL_SUM = 3, DI_NFALLBACK = 4, DI_NFALLBACK_SUM = 5,
-       DI_FIX = 6, DI_TICKET = 7, DI_N = 8 };
+       DI_FIX = 6, DI_DRAWN = 7, DI_DONE = 8, DI_LEFT = 9, DI_N = 10 };
+__host__ __device__ __forceinline__ int fail_list_cap(const Dims& d) { return d.n3 == 1 ? d.n1 * d.n2 : 0; }
 // Energy-file accumulators (dump_ener.c:391-407), per grid: boundary flux
 // sums of the last substep (pdot) and their time integral (pcum), six
 // boundaries X1UP, X1DN, X2UP, X2DN, X3UP, X3DN by eight variables; the

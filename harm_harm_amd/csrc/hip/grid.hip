@@ -463,7 +463,7 @@ __device__ __forceinline__ void invert_body(Dims d, Params P, const double* __re
     const int fl = invert_zone(d, P, U, pg, pf, pflag, gcent, o, pp, ns);
     nf = !finalstep && fl > 0;
   }
-  newton_counts_to(ns, nf, di);
+  newton_counts_to(ns, nf, di, t, fail_list_cap(d));
 }
 
 // DIAG: also keeps the states the fixes started from (floors_zone; fx = {p0,
@@ -497,7 +497,7 @@ __device__ __forceinline__ void floors_body(Dims d, Params P, double* pf, int32_
     if (fl != fl0) pflag[o] = fl;
     nf = fl > 0;
   }
-  newton_counts_to(ns, nf, di);
+  newton_counts_to(ns, nf, di, t, fail_list_cap(d));
 }
 
 // Bound by issue: about 1000 instructions a wave around the Newton iterations
@@ -619,15 +619,15 @@ __device__ __forceinline__ bool accounted(int f, int finalstep)
 //    velocity the normal observer's (set_atmosphere VELREL4, init.tools.c:797);
 //  - after a velocity average the Lorentz factor is capped at the zone's own
 //    pre-average value, itself capped at GAMMAMAX (:1290-1322).
+// t: the zone, i + n1 (j + n2 k).
 // DIAG (final substep): an accounted zone's change dV (U(after) - U(before))
 // goes to dfl and `true` is returned, *cat being its category slot.
 template <bool DIAG = false>
 __device__ __forceinline__ bool post_fixup_body(Dims d, Params P, const double* __restrict__ pf,
                                                 const int32_t* __restrict__ pflag, double* __restrict__ pout,
-                                                const double* __restrict__ gcent, int finalstep, const int blk,
+                                                const double* __restrict__ gcent, int finalstep, const long t,
                                                 double* dfl = nullptr, int* cat = nullptr)
 {
-  const long t = (long)blk * kBlock + threadIdx.x;
   const long nact = (long)d.n1 * d.n2 * d.n3;
   if (t >= nact) return false;
   const int i = (int)(t % d.n1), j = (int)((t / d.n1) % d.n2), k = (int)(t / ((long)d.n1 * d.n2));
@@ -728,7 +728,8 @@ __global__ __launch_bounds__(kBlock) void k_post_fixup(Dims d, Params P, const d
   if (!DIAG && di && di[DI_FIX] == 0) return;  // di: inside a step, where the inversion counted the failed zones
   double dfl[HARM_NPR] = {0, 0, 0, 0, 0, 0, 0, 0};
   int cat = 0;
-  const bool ch = post_fixup_body<DIAG>(d, P, pf, pflag, pout, gcent, finalstep, blockIdx.x, dfl, &cat);
+  const bool ch = post_fixup_body<DIAG>(d, P, pf, pflag, pout, gcent, finalstep, (long)blockIdx.x * kBlock + threadIdx.x,
+                                        dfl, &cat);
   if (DIAG && !__syncthreads_or(ch)) {  // no accounted zone in the block
     if (threadIdx.x < 32) fl_part[(long)(threadIdx.x >> 3) * gridDim.x * 8 + (long)blockIdx.x * 8 + (threadIdx.x & 7)] = 0.0;
     return;
@@ -747,9 +748,8 @@ __global__ __launch_bounds__(kBlock) void k_post_fixup(Dims d, Params P, const d
 // primitives, and accounted zones (also the fixed-flag ones, whose
 // accounting changes nothing) get UTOPRIMFAILFIXEDUTOPRIM.
 __device__ __forceinline__ void fixup_apply_body(const Dims& d, double* __restrict__ pf, int32_t* __restrict__ pflag,
-                                                 const double* __restrict__ pin, int finalstep, const int blk)
+                                                 const double* __restrict__ pin, int finalstep, const long t)
 {
-  const long t = (long)blk * kBlock + threadIdx.x;
   const long nact = (long)d.n1 * d.n2 * d.n3;
   if (t >= nact) return;
   const int i = (int)(t % d.n1), j = (int)((t / d.n1) % d.n2), k = (int)(t / ((long)d.n1 * d.n2));
@@ -769,7 +769,7 @@ __global__ __launch_bounds__(kBlock) void k_fixup_apply(Dims d, double* __restri
                                                         const unsigned long long* __restrict__ di)
 {
   if (di && di[DI_FIX] == 0) return;
-  fixup_apply_body(d, pf, pflag, pin, finalstep, blockIdx.x);
+  fixup_apply_body(d, pf, pflag, pin, finalstep, (long)blockIdx.x * kBlock + threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1115,6 +1115,13 @@ __global__ __launch_bounds__(kBlock) void k_bound_x3(Dims d, double* __restrict_
   bound_x3_body(d, p, blockIdx.x);
 }
 
+// one thread waits until a count that other blocks raise has reached n
+__device__ __forceinline__ void wait_count(unsigned long long* count, int n)
+{
+  while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (unsigned long long)n)
+    __builtin_amdgcn_s_sleep(2);
+}
+
 // ---------------------------------------------------------------------------
 // The whole boundary pass in one launch
 // ---------------------------------------------------------------------------
@@ -1270,10 +1277,30 @@ __device__ __forceinline__ void bounds_flags(const Dims& d, int bc, int32_t* __r
 
 // cond: the second pass, only where failure averaging changed zones and
 // without the flags (a batch counts their blocks for both passes).  ds_end
-// (or null): the step's last launch, which also ends the step.  FIX2D (2-D grids, flags
-// bounded in the same launch): the block that ends last goes on with failure
-// averaging and the second pass when there are failed zones; they are few, so
-// one block is enough.  Its zones come from every block, hence the fences.
+// (or null): the step's last launch, which also ends the step.
+//
+// FIX2D (2-D grids, flags bounded in the same launch): with failed zones the
+// launch goes on with failure averaging of the zones that the inversion listed
+// and the second pass.  Its blocks then draw their work from one queue in di: the
+// boundary pass, averaging into pfix, the write-back, the boundary pass again.  A
+// block that has drawn an item waits until every item of the phases before it is
+// done.  Those were drawn before it, by blocks that run, and the first phase waits
+// for nothing, so the waits end whatever number of blocks the chip holds at a time
+// (blocks yet to start have drawn nothing).  A phase reads what other blocks
+// wrote, hence the fences.  The last block to leave clears the queue for the next
+// launch.
+// RK2 steps of a torus with a tenth of its zones failed take 2.2 ms at 256x256 and
+// 5.1 at 512x512 (most of it their solves); with averaging every zone's run and
+// the second pass in the block that ends last they took 7.2 and 22.9.
+//
+// Blocks of the launch: those of the boundary pass, on grids of many zones enough
+// to average a quarter of them at once (a block without work ends at once), up to
+// one a CU.
+__host__ __device__ __forceinline__ int finish_blocks(const Dims& d)
+{
+  const int n = bound_plan(d, true).total(), h = (d.n1 * d.n2 / 4 + kBlock - 1) / kBlock;
+  return n > h ? n : h < 256 ? h : 256;
+}
 template <bool FIX2D>
 __device__ __forceinline__ void bounds_body(const Dims& d, const Params& P, double* p, const double* gcent,
                                             const double* rcent, int32_t* pflag, double* pfix,
@@ -1285,28 +1312,52 @@ __device__ __forceinline__ void bounds_body(const Dims& d, const Params& P, doub
   if (cond && !fix) return;
   const BoundPlan b = bound_plan(d, flags);
   const int nprim = b.nA + b.nB + b.nC;
-  if (blk >= nprim && !cond) bounds_flags(d, P.bc, pflag, (long)(blk - nprim) * kBlock + threadIdx.x);
-  int v0 = blk, v1 = blk < nprim ? blk + 1 : blk;
-  for (bool again = false;; again = true) {
-    for (int v = v0; v < v1; v++) bounds_prims(d, P, b, p, gcent, rcent, v);
-    if (!FIX2D || !fix) return;
-    if (again) break;
-    __shared__ bool last;
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(&di[DI_TICKET], 1ull) == (unsigned long long)(b.total() - 1);
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    const int nz = (d.n1 * d.n2 * d.n3 + kBlock - 1) / kBlock;
-    for (int z = 0; z < nz; z++) post_fixup_body(d, P, p, pflag, pfix, gcent, finalstep, z);
-    __syncthreads();
-    for (int z = 0; z < nz; z++) fixup_apply_body(d, p, pflag, pfix, finalstep, z);
-    __syncthreads();
-    v0 = 0;
-    v1 = nprim;
+  auto bound = [&](int v) {
+    if (v < nprim) bounds_prims(d, P, b, p, gcent, rcent, v);
+    else if (v < b.total() && !cond) bounds_flags(d, P.bc, pflag, (long)(v - nprim) * kBlock + threadIdx.x);
+  };
+  if (!FIX2D || !fix) {
+    bound(blk);
+    return;
   }
-  if (threadIdx.x == 0) di[DI_TICKET] = 0;
+  __shared__ int drawn;
+  const int nf = __builtin_amdgcn_readfirstlane((int)di[DI_FIX]), ni = (nf + kBlock - 1) / kBlock;
+  const int nblk = min(finish_blocks(d), max(b.total(), ni));
+  if (blk >= nblk) return;
+  const int32_t* list = (const int32_t*)(di + DI_N);
+  const int average = b.total(), apply = average + ni, again = apply + ni, end = again + nprim;
+  if (threadIdx.x == 0) drawn = (int)atomicAdd(&di[DI_DRAWN], 1ull);
+  __syncthreads();
+  // Every pass ends in a barrier that all threads meet, with the thread that
+  // draws among them: with its work behind the last barrier the compiler made
+  // the other threads' way round a loop of its own, which that thread had left.
+#pragma clang loop unroll(disable)
+  while (true) {
+    const int v = __builtin_amdgcn_readfirstlane(drawn);  // the same in every thread
+    if (v >= end) break;
+    const int before = v < average ? 0 : v < apply ? average : v < again ? apply : again;  // items of earlier phases
+    if (before > 0) {
+      if (threadIdx.x == 0) wait_count(&di[DI_DONE], before);
+      __syncthreads();
+      __threadfence();
+    }
+    if (v < average) bound(v);
+    else if (v >= again) bound(v - again);
+    else {
+      const int e = (v < apply ? v - average : v - apply) * kBlock + threadIdx.x;
+      if (e < nf && v < apply) post_fixup_body(d, P, p, pflag, pfix, gcent, finalstep, list[e]);
+      else if (e < nf) fixup_apply_body(d, p, pflag, pfix, finalstep, list[e]);
+    }
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      atomicAdd(&di[DI_DONE], 1ull);
+      drawn = (int)atomicAdd(&di[DI_DRAWN], 1ull);
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && atomicAdd(&di[DI_LEFT], 1ull) == (unsigned long long)(nblk - 1))
+    di[DI_DRAWN] = di[DI_DONE] = di[DI_LEFT] = 0;
 }
 
 template <bool FIX2D>
@@ -1904,7 +1955,7 @@ harm_status enq_finish(harm_handle* h, int which, int finalstep, bool ener, bool
   const bool merge = bounds_merge(d);
   if (merge && d.n3 == 1 && !ener) {
     prof_begin(h);
-    hipLaunchKernelGGL(k_bounds<true>, dim3((unsigned)bound_plan(d, true).total()), dim3(kBlock), 0, h->stream, d,
+    hipLaunchKernelGGL(k_bounds<true>, dim3((unsigned)finish_blocks(d)), dim3(kBlock), 0, h->stream, d,
                        h->P, h->arr[which], h->geom[HARM_LOC_CENT], h->rcent, h->pflag, h->pfix, h->di, finalstep, 1,
                        0, end ? h->ds : nullptr);
     prof_end(h, HARM_K_BOUND);
@@ -2108,7 +2159,7 @@ __global__ __launch_bounds__(kBlock) void kb_post_fixup(const GridRef* __restric
   BATCH_DECODE(false)
   if (cond && gmem(g.di)[DI_FIX] == 0) return;
   post_fixup_body(g.d, g.P, gmem(g.arr[which]), gmem(g.pflag), gmem(g.pfix), gmem(g.geom[HARM_LOC_CENT]), finalstep,
-                  lb);
+                  (long)lb * kBlock + threadIdx.x);
 }
 
 __global__ __launch_bounds__(kBlock) void kb_fixup_apply(const GridRef* __restrict__ G, const int* __restrict__ pre,
@@ -2116,7 +2167,7 @@ __global__ __launch_bounds__(kBlock) void kb_fixup_apply(const GridRef* __restri
 {
   BATCH_DECODE(false)
   if (cond && gmem(g.di)[DI_FIX] == 0) return;
-  fixup_apply_body(g.d, gmem(g.arr[which]), gmem(g.pflag), gmem(g.pfix), finalstep, lb);
+  fixup_apply_body(g.d, gmem(g.arr[which]), gmem(g.pflag), gmem(g.pfix), finalstep, (long)lb * kBlock + threadIdx.x);
 }
 
 // every grid's boundary pass (bounds_body); pre: block counts with the flags'
@@ -2246,7 +2297,7 @@ harm_status batch_build(harm_batch* b)
     cnt[BS_BX3] = e2 ? nblocks(d.nplane * 2L * d.ng3) : 0;
     cnt[BS_ONE] = 1;
     cnt[BS_PFB] = nblocks(std::max(bound_pflag_items(d, 0), bound_pflag_items(d, 1)));
-    if (bounds_merge(d)) cnt[BS_BND] = bound_plan(d, true).total();
+    if (bounds_merge(d)) cnt[BS_BND] = d.n3 == 1 ? finish_blocks(d) : bound_plan(d, true).total();
     else b->bnd_merged = false;
     for (int st = 0; st < BS_N; st++) {
       const long nx = (long)pre[(size_t)st * (ng + 1) + gi] + cnt[st];
@@ -2450,7 +2501,7 @@ extern "C" harm_status harm_create(const harm_config* cfg, harm_handle** out)
   TRYC(alloc((void**)&h->enpart, sizeof(double) * 4 * 8 * ener_part_blocks(d)));  // 4 channels
   TRYC(alloc((void**)&h->entot, sizeof(double) * 10));
   TRYC(hh::check_hip(hipMemset(h->ds, 0, sizeof(double) * DS_N), "hipMemset"));
-  TRYC(alloc((void**)&h->di, sizeof(unsigned long long) * DI_N));
+  TRYC(alloc((void**)&h->di, sizeof(unsigned long long) * DI_N + sizeof(int32_t) * fail_list_cap(d)));
   TRYC(hh::check_hip(hipMemset(h->di, 0, sizeof(unsigned long long) * DI_N), "hipMemset"));
   TRYC(build_geometry(h));
   TRYC(build_axes(h));

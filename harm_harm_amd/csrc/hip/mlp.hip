@@ -740,7 +740,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) 
     const int fl = hk::invert_zone<true>(d, P, U, pg, pf, pflag, gcent, o, pp, ns, seed, &fb);
     nf = !finalstep && fl > 0;
   }
-  hk::newton_counts_to(ns, nf, di);
+  hk::newton_counts_to(ns, nf, di, t, hk::fail_list_cap(d));
   __shared__ unsigned int nfb;
   if (threadIdx.x == 0) nfb = 0;
   __syncthreads();
