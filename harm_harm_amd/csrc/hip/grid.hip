@@ -1289,9 +1289,9 @@ __device__ __forceinline__ void bounds_flags(const Dims& d, int bc, int32_t* __r
 // (blocks yet to start have drawn nothing).  A phase reads what other blocks
 // wrote, hence the fences.  The last block to leave clears the queue for the next
 // launch.
-// RK2 steps of a torus with a tenth of its zones failed take 2.2 ms at 256x256 and
-// 5.1 at 512x512 (most of it their solves); with averaging every zone's run and
-// the second pass in the block that ends last they took 7.2 and 22.9.
+// RK2 steps of a torus with a tenth of its zones failed take 1.8 ms at 256x256 and
+// 3.8 at 512x512 (most of it their solves); with averaging every zone's run and
+// the second pass in the block that ends last they took 5 and 18 more.
 //
 // Blocks of the launch: those of the boundary pass, on grids of many zones enough
 // to average a quarter of them at once (a block without work ends at once), up to
