@@ -23,10 +23,8 @@ def test_accepted_roots_are_the_iterations(newton, wide, least):  # noqa: F811
         Ts = -n * V2 / ((n + 1) * (n * V2 - 1))
         C1 = us * rs * rs * Ts**n * rng.uniform(1 - wide, 1 + wide)
         C2 = (1 + (1 + n) * Ts) ** 2 * (1 - 2 / rs + us * us) * rng.uniform(1 - wide, 1 + wide)
-        start = Ts * rng.uniform(1 - wide, 1 + wide)
         ref, settled = iterate(n, C1, C2, r)
-        if settled and ref > 0 and rng.uniform() < 0.5:
-            start = ref * rng.uniform(1 - wide, 1 + wide)
+        start = (ref if settled and ref > 0 else Ts) * rng.uniform(1 - wide, 1 + wide)
         T = ctypes.c_double(start)
         if newton(n, C1, C2, r, ctypes.byref(T)):
             taken += 1
