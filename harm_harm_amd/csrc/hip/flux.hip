@@ -361,6 +361,7 @@ void launch_flux_batch(int recon, const int* n, const int* const* pre, hipStream
                        int which, int do_ct)
 {
   const dim3 grid((unsigned)(n[0] + n[1] + n[2])), blk(kBlock);
+  if (grid.x == 0) return;  // grids of one zone have no faces
 #define LB(RECON)                                                                                                  \
   hipLaunchKernelGGL(kb_flux_all<RECON>, grid, blk, 0, s, G, pre[0], pre[1], pre[2], n[0], n[1], n[2], ng, which, \
                      do_ct)
