@@ -92,11 +92,6 @@ __device__ __forceinline__ double quot(double n, const Recip& R)
   const double q = n * R.r;
   return fma(fma(-R.d, q, n), R.r, q);
 }
-// n / d with IEEE's zeros, infinities and NaN for either operand
-__device__ __forceinline__ double quot_any(double n, const Recip& R)
-{
-  return __builtin_amdgcn_div_fixup(quot(n, R), R.d, n);
-}
 // 1 / d
 __device__ __forceinline__ double inv1(double d)
 {

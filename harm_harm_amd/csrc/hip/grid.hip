@@ -2007,13 +2007,9 @@ harm_status enq_substep(harm_handle* h, int to, int nto, const double CUf[4][4],
                          h->stream);
   }
   const bool facc = diag && h->d.n1 > 1;
-  // The reduced-traffic modes rely on the tables keeping ucum at zero until
-  // the last substep (true of the RK2 and RK3 tables); otherwise run the
-  // reference loop as is.
-  bool zero_ucum = in_step;
-  for (int s = 0; s + 1 < nto; s++)
-    zero_ucum = zero_ucum && Cunew[s][0] == 0.0 && Cunew[s][1] == 0.0 && Cunew[s][2] == 0.0;
-  const int mode = !zero_ucum ? kUpdAll : to == 0 ? kUpdFirst : finalstep ? kUpdLast : kUpdMiddle;
+  // The reduced-traffic modes rely on rk_tables keeping ucum at zero until the
+  // last substep; a lone substep runs the reference loop as is.
+  const int mode = !in_step ? kUpdAll : to == 0 ? kUpdFirst : finalstep ? kUpdLast : kUpdMiddle;
   // the update of a step forms the field fluxes itself; the energy sums read them ahead of it
   HH_TRY(enq_fluxcalc(h, pbb[to], 1, in_step, facc, mode == kUpdAll || ener));
   if (ener)
@@ -2050,8 +2046,8 @@ void rk_flux_weights(int timeorder, double* w)
 // A whole RK step is captured once in a hipGraph (kernel nodes only) and
 // replayed.
 // ---------------------------------------------------------------------------
-enum { BS_FLUX1 = 0, BS_FLUX2, BS_FLUX3, BS_EMF, BS_CT, BS_FACC, BS_ZONE, BS_BX1, BS_X2R, BS_X2P,
-       BS_X2M, BS_BX3, BS_ONE, BS_PFB, BS_BND, BS_N };
+enum { BS_FLUX1 = 0, BS_FLUX2, BS_FLUX3, BS_EMF, BS_FACC, BS_ZONE, BS_BX1, BS_X2R, BS_X2P, BS_X2M, BS_BX3, BS_PFB,
+       BS_BND, BS_N };
 
 __device__ __forceinline__ void batch_decode(const int* __restrict__ pre, int ng, int b, int& gi, int& lb)
 {
@@ -2087,14 +2083,6 @@ __global__ __launch_bounds__(kBlock) void kb_emf(const GridRef* __restrict__ G, 
   if (lb == 0 && threadIdx.x == 0) gmem(g.di)[DI_FIX] = 0;
   emf_body(g.d, g.emf_ni, g.emf_nj, g.emf_nk, gmem(g.arr[HARM_ARR_F1]), gmem(g.arr[HARM_ARR_F2]), gmem(g.arr[HARM_ARR_F3]),
            gmem(g.geom[HARM_LOC_FACE1]), gmem(g.geom[HARM_LOC_FACE2]), gmem(g.gcorn3), gmem(g.emf), lb);
-}
-
-__global__ __launch_bounds__(kBlock) void kb_ct_all(const GridRef* __restrict__ G, const int* __restrict__ pre,
-                                                    int ng)
-{
-  BATCH_DECODE(true)
-  ct_all_body(g.d, g.emf_ni, g.emf_nj, g.emf_nk, gmem(g.emf), gmem(g.arr[HARM_ARR_F1]), gmem(g.arr[HARM_ARR_F2]),
-              gmem(g.arr[HARM_ARR_F3]), lb);
 }
 
 // update of every grid (n blocks), then one block a grid for its boundary flux sums
@@ -2286,7 +2274,6 @@ harm_status batch_build(harm_batch* b)
     cnt[BS_FLUX2] = e1 ? h->ft[2].nblk : 0;
     cnt[BS_FLUX3] = e2 ? h->ft[3].nblk : 0;
     cnt[BS_EMF] = nblocks((long)h->emf_ni * h->emf_nj * h->emf_nk);
-    cnt[BS_CT] = nblocks((long)(d.n1 + e0) * (d.n2 + e1) * (d.n3 + e2));
     cnt[BS_FACC] = e0 ? kFaccBlocks : 0;
     cnt[BS_ZONE] = nblocks((long)d.n1 * d.n2 * d.n3);
     cnt[BS_BX1] = e0 ? nblocks(2L * d.ng1 * d.n2 * d.n3) : 0;
@@ -2295,7 +2282,6 @@ harm_status batch_build(harm_batch* b)
     cnt[BS_X2M] = e1 ? nblocks(2L * d.ns1 * d.n3 * d.ng2) : 0;
     if (e1 && d.n2 <= d.ng2) b->x2_merged = false;
     cnt[BS_BX3] = e2 ? nblocks(d.nplane * 2L * d.ng3) : 0;
-    cnt[BS_ONE] = 1;
     cnt[BS_PFB] = nblocks(std::max(bound_pflag_items(d, 0), bound_pflag_items(d, 1)));
     if (bounds_merge(d)) cnt[BS_BND] = d.n3 == 1 ? finish_blocks(d) : bound_plan(d, true).total();
     else b->bnd_merged = false;
@@ -2341,14 +2327,9 @@ harm_status enq_batch_substep(harm_batch* b, int to, int nto, const double CUf[4
   launch_flux_batch(b->recon, &b->ntot[BS_FLUX1], pf3, s, G, ng, pbb[to], 1);
   const int ne = b->ntot[BS_EMF], nz = b->ntot[BS_ZONE];
   hipLaunchKernelGGL(kb_emf, dim3((unsigned)(ne + b->ntot[BS_FACC])), blk, 0, s, G, P(BS_EMF), P(BS_FACC), ne, ng);
-  // update (the reduced-traffic modes: the RK2/RK3 tables keep ucum at zero
-  // until the last substep)
-  bool zero_ucum = true;
-  for (int st = 0; st + 1 < nto; st++)
-    zero_ucum = zero_ucum && Cunew[st][0] == 0.0 && Cunew[st][1] == 0.0 && Cunew[st][2] == 0.0;
-  const int mode = !zero_ucum ? kUpdAll : to == 0 ? kUpdFirst : finalstep ? kUpdLast : kUpdMiddle;
-  if (mode == kUpdAll && b->ntot[BS_CT])
-    hipLaunchKernelGGL(kb_ct_all, dim3((unsigned)b->ntot[BS_CT]), blk, 0, s, G, P(BS_CT), ng);
+  // update (the reduced-traffic modes: rk_tables keeps ucum at zero until the
+  // last substep)
+  const int mode = to == 0 ? kUpdFirst : finalstep ? kUpdLast : kUpdMiddle;
   const dim3 gz((unsigned)nz);
 #define BUPD(DM, MODE)                                                                                            \
   hipLaunchKernelGGL((kb_update<DM, MODE>), dim3((unsigned)(nz + ng)), blk, 0, s, G, P(BS_ZONE), ng, nz, pii[to], \
@@ -2358,8 +2339,7 @@ harm_status enq_batch_substep(harm_batch* b, int to, int nto, const double CUf[4
   switch (mode) {                                        \
     case kUpdFirst: BUPD(DM, kUpdFirst); break;          \
     case kUpdMiddle: BUPD(DM, kUpdMiddle); break;        \
-    case kUpdLast: BUPD(DM, kUpdLast); break;            \
-    default: BUPD(DM, kUpdAll); break;                   \
+    default: BUPD(DM, kUpdLast); break;                  \
   }
   if (b->dm == 7) { BUPD_MODES(7); }
   else if (b->dm == 3) { BUPD_MODES(3); }
