@@ -84,12 +84,16 @@ def algorithmic_bytes(g, kernel):
     if kernel == "emf_ct":
         # six field fluxes read, three EMFs written (the update applies the CT)
         return zones * (6 * 8 + 3 * 8)
+    # grids whose boundary pass is one launch (the library's bounds_merge): the
+    # second pass of a substep and failure averaging end at once unless a zone failed
+    merged = n1 >= 8 and n2 > 1 and n2 > g.cfg.ng
     if kernel == "bound":
-        # every ghost zone written once from a zone read once (8 doubles each)
+        # every ghost zone written once from a zone read once (8 doubles each);
+        # in 3-D two launches a substep of which the second has nothing to do
         ghosts = (n1 + 2 * 4 * e0) * (n2 + 2 * 4 * e1) * (n3 + 2 * 4 * e2) - zones
-        return ghosts * 128
+        return ghosts * 128 // (2 if merged and e2 else 1)
     if kernel == "fixup":
-        return zones * 4  # the failure flags; failed zones are few
+        return 0 if merged else zones * 4  # the failure flags; failed zones are few
     if kernel == "recon":
         # WENO5BND per substep, four timed launches: the dP pass (read the
         # primitives 64, write dP of three directions 24) and one line pass
@@ -620,12 +624,12 @@ def main():
                 "frac": tf / FP64_PEAK_TFLOPS, "flops_per_launch": md["flops"],
                 "source": "rocprofv3 --pmc SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS}_F64, " + os.path.relpath(COUNTERS, ROOT)}
     # whole step against HBM.  Algorithmic bytes per zone-update of the plain
-    # step, independent of how it is cut into kernels: per substep, recon +
-    # flux per direction read p 64 and write F 64 (384), CT 144, update 512,
-    # inversion 196 = 1236 B, three substeps.  Beside it the compulsory
+    # step: per substep, recon + flux per direction read p 64 and write F 64
+    # (384), EMFs from the field fluxes 72, update with the CT inside 448,
+    # inversion 196 = 1100 B, three substeps.  Beside it the compulsory
     # traffic of this build's kernel groups (the WENO5BND face values and dP
     # make the split reconstruction move more than the fused unit would).
-    alg_zu = 3 * (3 * 128 + 144 + 512 + 196)
+    alg_zu = 3 * (3 * 128 + 72 + 448 + 196)
     zps = zones * args.steps / el
     step_bytes = sum((algorithmic_bytes(g, k) or 0) * prof[k][1] / prof_steps for k in prof if prof[k][1])
     step_roof = {"bytes_per_zone_update_alg": alg_zu, "achieved": zps * alg_zu / 1e9, "peak": HBM_PEAK_GBS,
