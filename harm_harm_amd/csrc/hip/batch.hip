@@ -63,10 +63,12 @@ __device__ __forceinline__ bool invert_one(const double* __restrict__ U, const d
 // for a zone's 17.5.  With more than one round the solves stop at kFirst
 // iterations; the unfinished zones go into a list in LDS and are solved from
 // the start, in full waves, whenever a block's worth has come together and
-// after the last round.  2^24 zones take 4.9 ms (27.5 ms one zone a lane to the
-// end; 7.0 GB compulsory, so 1.4 TB/s), 4096 zones 0.16 ms (0.39), one zone's
-// 200 iterations; kFirst 12, 14 and 18: 5.9, 5.1 and 4.9 ms.  Four waves per
-// SIMD although 136 B a lane spill: 5.3 ms at three, 6.0 at two.
+// after the last round.  2^24 zones take 5.5 ms (27.5 ms one zone a lane to the
+// end; 7.0 GB compulsory, so 1.3 TB/s).  4096 zones take 0.09 ms, the slowest
+// zone's chain of 30 to 50 iterations (its cycles are counted, not run); with the
+// 200 that it has to its cap a round trip through p -> U -> p took 0.38, now 0.16.
+// Compared with one another on one box: kFirst 12, 14, 16 and 18 5.9, 5.1, 4.9 and
+// 4.9 ms; four waves per SIMD although 136 B a lane spill 4.9, three 5.3, two 6.0.
 constexpr int kFirst = 16;
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_invert_batch(const double* __restrict__ U, const double* __restrict__ geom,
                                                          double* __restrict__ p, int32_t* __restrict__ pflag,

@@ -1289,9 +1289,10 @@ __device__ __forceinline__ void bounds_flags(const Dims& d, int bc, int32_t* __r
 // (blocks yet to start have drawn nothing).  A phase reads what other blocks
 // wrote, hence the fences.  The last block to leave clears the queue for the next
 // launch.
-// RK2 steps of a torus with a tenth of its zones failed take 1.8 ms at 256x256 and
-// 3.8 at 512x512 (most of it their solves); with averaging every zone's run and
-// the second pass in the block that ends last they took 5 and 18 more.
+// Bound by the chains of the phases, about 12 us each, and the waits between them.
+// At 256x256 with 190 failed zones the launch takes 57 us, at 512x512 with 50 000
+// 186; walking every zone's flag and the whole second pass in the block that ends
+// last took 539 and 9157 us, the eight separate launches 60 and 85 and their gaps.
 //
 // Blocks of the launch: those of the boundary pass, on grids of many zones enough
 // to average a quarter of them at once (a block without work ends at once), up to
@@ -3105,8 +3106,8 @@ harm_status write_rows(FILE* f, const double* rows, long nz, int ncol)
 
 // The rows are built on the device a chunk at a time (37.7 MB, kept with the
 // handle) and copied into the caller's.  At 96x64x32 four steps with energy
-// sums, the currents and the 113 MB of rows take 7.5 ms; with an allocation a
-// call, planes copied back and rows and coordinates formed on the host, 49.2.
+// sums, the currents and the 113 MB of rows take 7.3 ms; with an allocation a
+// call, planes copied back and rows and coordinates formed on the host, 33.6.
 constexpr long kRowChunk = 65536;
 extern "C" harm_status harm_dump_columns(harm_handle* h, int32_t which, double* rows)
 {

@@ -41,8 +41,10 @@
 // Quotients are the largest part of it, so the weights of a zone share one
 // reciprocal per normalisation (hd::recip, hd::quot), 7 + 3 + 3 instructions for
 // three quotients instead of 33, and the SMONO and ratio tests settle clear
-// cases without a quotient.  At 256x128x64 the x1, x2 and x3 passes take 265, 301
-// and 337 us so, 311, 405 and 450 with the compiler's divisions.
+// cases without a quotient: on one state of the 256x128x64 torus the x1, x2 and x3
+// passes took 265, 301 and 337 us so, 311, 405 and 450 with the compiler's
+// divisions.  Alone on the chip they take 222, 227 and 175 us on the axisymmetric
+// start and 298, 362 and 394 some twenty steps on, when most windows need weights.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <float.h>
