@@ -49,7 +49,7 @@ def test_large_grid_with_failures_equals_kernel_sequence_and_is_no_slower():
 
 
 def test_batch_whose_launch_exceeds_the_chip():
-    """48 members of 160 x 160 zones, all but every fourth with failures: 1200
+    """24 members of 160 x 160 zones, all but every fourth with failures: 600
     blocks where the chip holds about 512, so members' blocks start while others
     wait.  Equal to single grids over three steps."""
     cfg = H.default_config(160, 160, 1, recon="para", flux="hll", timeorder=2)
@@ -57,7 +57,7 @@ def test_batch_whose_launch_exceeds_the_chip():
     for seed in range(4):
         og, p, dt = kicked(cfg, seed)
         states.append((og.init_torus(), 0.3 * dt) if seed == 3 else (p, dt))
-    B, singles = Batch([cfg] * 48), [Grid(cfg) for _ in states]
+    B, singles = Batch([cfg] * 24), [Grid(cfg) for _ in states]
     for i, g in enumerate(B.grids + singles):
         p, dt = states[i % 4]
         g.set("p", p)
