@@ -1308,7 +1308,7 @@ __device__ __forceinline__ void bounds_body(const Dims& d, const Params& P, doub
                                             unsigned long long* di, int finalstep, bool flags, bool cond, int blk,
                                             double* ds_end)
 {
-  const bool fix = (FIX2D || cond) && di[DI_FIX] != 0;
+  const bool fix = (FIX2D || cond) && __builtin_amdgcn_readfirstlane((int)di[DI_FIX]) != 0;
   const BoundPlan b = bound_plan(d, flags);
   // (the flags' last block has the least to do; in block 0, ahead of the count, the
   // scalars made the launch 13.9 us at 64x64, 13.7 so)
@@ -1344,12 +1344,12 @@ __device__ __forceinline__ void bounds_body(const Dims& d, const Params& P, doub
       __syncthreads();
       __threadfence();
     }
-    if (v < average) bound(v);
-    else if (v >= again) bound(v - again);
-    else {
-      const int e = (v < apply ? v - average : v - apply) * kBlock + threadIdx.x;
-      if (e < nf && v < apply) post_fixup_body(d, P, p, pflag, pfix, gcent, finalstep, list[e]);
-      else if (e < nf) fixup_apply_body(d, p, pflag, pfix, finalstep, list[e]);
+    if (v < average || v >= again) {  // one copy of the pass for both (three in all were 170 KB of instructions)
+      bound(v < average ? v : v - again);
+    } else {
+      const int z = (v < apply ? v - average : v - apply) * kBlock + threadIdx.x;
+      if (z < nf && v < apply) post_fixup_body(d, P, p, pflag, pfix, gcent, finalstep, list[z]);
+      else if (z < nf) fixup_apply_body(d, p, pflag, pfix, finalstep, list[z]);
     }
     __threadfence();
     __syncthreads();
