@@ -202,22 +202,22 @@ __device__ __forceinline__ void newton_counts_to(int ns, int nf, unsigned long l
   __shared__ unsigned long long red[2];
   if (threadIdx.x == 0) { red[0] = 0; red[1] = 0; }
   __syncthreads();
-  int rank = 0;
   if (ns) atomicAdd(&red[0], (unsigned long long)ns);
-  if (nf) rank = (int)atomicAdd(&red[1], 1ull);
-  __syncthreads();
-  const int nfail = __builtin_amdgcn_readfirstlane((int)red[1]);  // the same in every thread
-  if (threadIdx.x == 0) {
-    if (red[0]) atomicAdd(&di[DI_NSTROKE], red[0]);
-    if (nfail) {
-      atomicAdd(&di[DI_NFAIL], (unsigned long long)nfail);
-      red[0] = atomicAdd(&di[DI_FIX], (unsigned long long)nfail);  // the block's first place in the list
+  if (nf) {
+    atomicAdd(&red[1], 1ull);
+    if (cap) {
+      const unsigned long long at = atomicAdd(&di[DI_FIX], 1ull);
+      if (at < (unsigned long long)cap) ((int32_t*)(di + DI_N))[at] = zone;
     }
   }
-  if (cap == 0 || nfail == 0) return;
   __syncthreads();
-  const unsigned long long at = red[0] + rank;
-  if (nf && at < (unsigned long long)cap) ((int32_t*)(di + DI_N))[at] = zone;
+  if (threadIdx.x == 0) {
+    if (red[0]) atomicAdd(&di[DI_NSTROKE], red[0]);
+    if (red[1]) {
+      atomicAdd(&di[DI_NFAIL], red[1]);
+      if (!cap) atomicAdd(&di[DI_FIX], red[1]);
+    }
+  }
 }
 
 }  // namespace hk
